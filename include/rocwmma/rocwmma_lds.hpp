@@ -186,6 +186,11 @@ namespace rocwmma
                 const uint32_t row = lane / chunks;
                 return row * ldBytes + (((lane % chunks) ^ swz(wave * rowsPerCopy + row)) << 4);
             }
+            // First K byte of the 16 bytes `lane` copies, within the stage (any copy issued by wave `wave`)
+            ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t laneK(uint32_t lane, uint32_t wave)
+            {
+                return ((lane % chunks) ^ swz(wave * rowsPerCopy + lane / chunks)) << 4;
+            }
             // Source byte offset of copy `copy` (wave uniform)
             ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t copySourceOffset(uint32_t copy, uint32_t ldBytes)
             {
@@ -274,6 +279,11 @@ namespace rocwmma
             ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t copySourceOffset(uint32_t copy, uint32_t ldBytes)
             {
                 return copy * rowsPerCopy * ldBytes;
+            }
+            // (a copy's lanes differ in K row, not inside one: the buffer bounds end K)
+            ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t laneK(uint32_t, uint32_t)
+            {
+                return 0u;
             }
             ROCWMMA_DEVICE static ROCWMMA_INLINE size_t stageStep(uint32_t ldBytes)
             {
@@ -387,6 +397,11 @@ namespace rocwmma
             {
                 return copy * rowsPerCopy * ldBytes;
             }
+            // (a copy's lanes differ in K row, not inside one: the buffer bounds end K)
+            ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t laneK(uint32_t, uint32_t)
+            {
+                return 0u;
+            }
             ROCWMMA_DEVICE static ROCWMMA_INLINE size_t stageStep(uint32_t ldBytes)
             {
                 return static_cast<size_t>(kRows) * ldBytes;
@@ -435,6 +450,76 @@ namespace rocwmma
 #pragma unroll
                 for(uint32_t kk = 0; kk < KPackBytes / 8u; ++kk)
                     read8(reinterpret_cast<uint32_t(*)[2]>(regs)[kk], ldsBase, kBase + 8u * kk, dim16, lane);
+            }
+        };
+
+        // ---------------------------------------------------------------------------------
+        // Dim-major stage of 32-bit elements: KRows LDS rows (one per K index) of Dim floats, cut into
+        // 128-byte segments; segment s of K row k lives at segment position s ^ swz(k).
+        //
+        // v_mfma_f32_32x32x2_f32 takes one float per lane, so nothing is transposed: lanes 0-31 read 32
+        // neighbouring floats of K row k, lanes 32-63 those of K row k + 4 (a lane holds four K rows in a row,
+        // as it does of a K-major tile).  Rows are a multiple of 256 bytes apart, so without a swizzle the
+        // two halves of a wave would meet in the same 32 banks; with K bit 2 flipping the segment they take
+        // one half of the banks each.
+        // ---------------------------------------------------------------------------------
+        template <uint32_t Dim, uint32_t KRows>
+        struct DimMajorTile32
+        {
+            static_assert(Dim == 64u || Dim == 128u || Dim == 256u, "tile rows of 64, 128 or 256 floats");
+            static constexpr uint32_t kRows       = KRows;
+            static constexpr uint32_t rowBytes    = Dim * 4u;
+            static constexpr uint32_t bytes       = kRows * rowBytes;
+            static constexpr uint32_t copies      = bytes / 1024u;
+            static constexpr uint32_t slotsPerRow = rowBytes / 16u;
+            static constexpr uint32_t rowsPerCopy = 64u / slotsPerRow; // 4, 2 or 1 K rows per whole-wave copy
+
+            ROCWMMA_HOST_DEVICE static constexpr uint32_t swz(uint32_t k)
+            {
+                return (k >> 2) & 1u;
+            }
+            // Source byte offset of `lane` inside a copy issued by wave `wave` of a pool whose size times
+            // rowsPerCopy is a multiple of 8 (so k % 8 is the same for all of a wave's copies).
+            ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t laneSourceOffset(uint32_t lane, uint32_t wave, uint32_t ldBytes)
+            {
+                const uint32_t kInCopy = lane / slotsPerRow;
+                const uint32_t pos     = lane % slotsPerRow;
+                const uint32_t k       = wave * rowsPerCopy + kInCopy; // only k % 8 matters
+                return kInCopy * ldBytes + (((pos >> 3) ^ swz(k)) << 7) + ((pos & 7u) << 4);
+            }
+            ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t copySourceOffset(uint32_t copy, uint32_t ldBytes)
+            {
+                return copy * rowsPerCopy * ldBytes;
+            }
+            // (a copy's lanes differ in K row, not inside one: the buffer bounds end K)
+            ROCWMMA_DEVICE static ROCWMMA_INLINE uint32_t laneK(uint32_t, uint32_t)
+            {
+                return 0u;
+            }
+            ROCWMMA_DEVICE static ROCWMMA_INLINE size_t stageStep(uint32_t ldBytes)
+            {
+                return static_cast<size_t>(kRows) * ldBytes;
+            }
+
+            // Operand of one 32-wide MFMA block: lane l ends up with dim = dim0 + l % 32 and
+            // k = 8 ks + (l / 32) * 4 + 0..3 in four registers, the order of KMajorTile::readBlock32.
+            // Two reads of two rows each; as for the other dim-major tiles they are inline assembly (outside
+            // the compiler's dependency tracking), so the caller waits and pins the registers before use.
+            template <uint32_t KPackBytes>
+            ROCWMMA_DEVICE static ROCWMMA_INLINE void
+                readBlock32(void* regs, const char* ldsTile, uint32_t dim0, uint32_t ks, uint32_t lane)
+            {
+                static_assert(KPackBytes == 16u, "four floats per lane");
+                typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+                const uint32_t     ldsBase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsPtr)ldsTile));
+                const uint32_t     k       = ks * 8u + (lane >> 5) * 4u;
+                const uint32_t     addr    = ldsBase + k * rowBytes + (((dim0 >> 5) ^ swz(k)) << 7) + ((lane & 31u) << 2);
+                constexpr uint32_t row     = rowBytes / 256u; // rows in units of 64 dwords
+                u32x2_t            lo, hi;
+                asm volatile("ds_read2st64_b32 %0, %1 offset0:0 offset1:%2" : "=v"(lo) : "v"(addr), "n"(row) : "memory");
+                asm volatile("ds_read2st64_b32 %0, %1 offset0:%2 offset1:%3" : "=v"(hi) : "v"(addr), "n"(2u * row), "n"(3u * row) : "memory");
+                reinterpret_cast<u32x2_t*>(regs)[0] = lo;
+                reinterpret_cast<u32x2_t*>(regs)[1] = hi;
             }
         };
 

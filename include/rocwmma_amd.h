@@ -109,11 +109,10 @@ int rocwmma_amd_device_info(int* compute_units, int* clock_mhz, int* is_gfx950);
  *             the reference's static_cast<int8_t> does (test/reference_impl.hpp:77-78).
  * c may be NULL when beta == 0.  c may equal d.
  * Shapes: m and n multiples of 16, k a multiple of 32 bytes' worth of elements per row is the
- * minimum every kernel accepts (k % 16 == 0 for 16-bit types, k % 32 == 0 for 8-bit types);
- * the blocked kernel additionally needs k in whole 64-byte stages and at least three of them, takes every
- * type in all four A/B layout pairs (m, n that do not fill whole tiles run on partly filled edge tiles)
- * and is chosen automatically, as are the weight-streaming kernels for up to 48 rows of A against a
- * col-major B.
+ * minimum every kernel accepts (k % 16 == 0 for 16-bit types, k % 32 == 0 for 8-bit types, k % 8 == 0 for float32);
+ * the blocked kernel takes every such shape and every type in all four A/B layout pairs (m, n and k that do
+ * not fill whole tiles and stages run on partly filled ones) and is chosen automatically, as are the
+ * weight-streaming kernels for up to 48 rows of A against a col-major B.
  * One of those (48 rows against few columns or little K, or a 16-bit A of 16 / 32 rows too large for the
  * LDS; wide 48-row problems run on the blocked kernel) runs as two launches on the
  * stream and adds its K slices into D with atomic adds: I32 results are exact, F32 results can differ
@@ -141,8 +140,9 @@ int rocwmma_amd_gemm(int         dtype_in,
                      void*       stream);
 
 /* Same as rocwmma_amd_gemm with the kernel family forced (`algo` is a rocwmma_amd_gemm_algo).
- * ROCWMMA_AMD_GEMM_BLOCKED returns ROCWMMA_AMD_UNSUPPORTED_SHAPE when k is not in whole stages, and
- * _BLOCKED_256 when the shape does not fill whole 256 x 256 tiles, like the reference's perf_hgemm host
+ * Asked for by name, the blocked kernel keeps to whole stages: ROCWMMA_AMD_GEMM_BLOCKED returns
+ * ROCWMMA_AMD_UNSUPPORTED_SHAPE when k is not in whole 64-byte stages, at least three of them (and
+ * ROCWMMA_AMD_UNSUPPORTED_TYPE for float32), and _BLOCKED_256 when the shape does not fill whole 256 x 256 tiles, like the reference's perf_hgemm host
  * (samples/perf_hgemm.cpp:735-765). */
 int rocwmma_amd_gemm_ex(int         algo,
                         int         dtype_in,
@@ -276,8 +276,7 @@ int rocwmma_amd_gemm_streamk_static(int         dtype_in,
  *                          inputs of the same type); the sum and the activation are computed in f32;
  *   bias       : n floats (device memory, 16-byte aligned), or NULL for none;
  *   activation : a rocwmma_amd_activation.
- * Row-major C/D with k in whole 64-byte stages (at least three) runs on the blocked kernel, everything
- * else one block per wave.
+ * Row-major C/D runs on the blocked kernel, a column-major one block per wave.
  */
 int rocwmma_amd_gemm_bias_act(int          dtype_in,
                               int          dtype_out,

@@ -208,6 +208,15 @@ int rocwmma_amd_gemm_ex(int         algo,
     }
     if(algo != ROCWMMA_AMD_GEMM_WAVE_TILE)
     {
+        // asked for by name, the blocked kernel takes whole stages of K only, and no float32
+        if(algo != ROCWMMA_AMD_GEMM_AUTO)
+        {
+            const uint64_t kBytes = static_cast<uint64_t>(k) * dtypeSize(dtype_in);
+            if(dtype_in == ROCWMMA_AMD_F32)
+                return ROCWMMA_AMD_UNSUPPORTED_TYPE;
+            if(kBytes % 64u != 0u || kBytes < 192u)
+                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+        }
         GemmArgs blocked = args;
         int      la = layout_a, lb = layout_b;
         transposeForColMajorC(blocked, la, lb);

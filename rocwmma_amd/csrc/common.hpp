@@ -117,6 +117,15 @@ namespace rocwmma_amd
     // forceLargeTile: the 256 x 256 tile or nothing (ROCWMMA_AMD_GEMM_BLOCKED_256)
     int launchGemmBlocked(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream,
                           bool forceLargeTile = false);
+    // one translation unit per element type
+    int launchGemmBlockedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
+    int launchGemmBlockedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
+    int launchGemmBlockedI8(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
+    int launchGemmBlockedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
+    int launchGemmBlockedF32(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
+    int launchGemmFusedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
+    int launchGemmFusedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
+    int launchGemmFusedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
     int launchGemmSkinny(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream);
     // Stream-K: the 256 x 256 tiling with the tile count balanced over persistent workgroups.  The
     // workspace holds one slot of raw accumulators per workgroup plus flags (streamKWorkspaceBytes).

@@ -54,10 +54,11 @@ namespace rocwmma_amd
                   uint32_t Stages_       = 4u, // LDS ring depth
                   uint32_t WavesPerSimd_ = 1u, // waves per SIMD: sizes the register budget, and no more become resident
                   uint32_t BlockEdge_    = 32u, // MFMA block edge: 32 (32x32xK) or 16 (16x16x2K)
-                  bool     Edges_        = false, // M and N need not fill whole macro tiles (multiples of 16 do)
+                  bool     Edges_        = false, // M, N and K need not fill whole macro tiles and stages (multiples of 16, 32 bytes do)
                   bool     Scaled_       = false, // fp8 operands with one E8M0 scale per 32 elements of K (MX)
                   bool     Fused_        = false, // epilogue adds a per-column bias and applies an activation
-                  uint32_t StageKB_      = 0u> // bytes of K per stage (0: 128 in the ring of two, else 64)
+                  uint32_t StageKB_      = 0u, // bytes of K per stage (0: 64 in the ring of four, else 128)
+                  bool     ExtraB_       = false> // the ring of B is one stage deeper than the ring of A
         struct BlockedConfig
         {
             using InT   = InT_;
@@ -68,7 +69,9 @@ namespace rocwmma_amd
             static constexpr bool     BKMajor = BKMajor_;
             // Partly filled tiles at the lower and right edges of C/D: operand reads past a matrix end
             // are cut off by the buffer bounds (rows and columns beyond the problem only ever meet
-            // results beyond it), C reads and D stores are masked lane by lane.
+            // results beyond it), C reads and D stores are masked lane by lane.  Along K the copies of a
+            // last, partly filled stage (and of stages beyond it) read nothing past the end of K and
+            // store zeros for both operands.
             static constexpr bool     Edges   = Edges_;
             // Block-scaled operands: the scaled instruction's K order decides which bytes a lane holds
             // (two runs of 16 from the two halves of the stage, see rocwmma/internal/fragment_map.hpp),
@@ -89,11 +92,13 @@ namespace rocwmma_amd
             static constexpr uint32_t MacroN  = WavesN * WaveN;
             // bytes of K per pipeline stage: 64 in the ring of four, 128 (whole lines of a K-contiguous
             // operand) in the ring of two
-            static constexpr uint32_t StageKB = StageKB_ != 0u ? StageKB_ : (Stages_ == 2u ? 128u : 64u);
+            static constexpr uint32_t StageKB = StageKB_ != 0u ? StageKB_ : (Stages_ == 4u ? 64u : 128u);
             static constexpr uint32_t MacroK  = StageKB / sizeof(InT); // K elements per stage
 
             // Fragments of one MFMA step.  BlockK = K of the widest single instruction.
-            static constexpr uint32_t KPack      = detail::maxKPack(detail::packClassOf<InT>());
+            // (float32: the instruction takes one float per lane; a lane holds 16 bytes of K and feeds four
+            // instructions from them, the same four K indices for both operands, so their order does not matter)
+            static constexpr uint32_t KPack      = sizeof(InT) == 4u ? 4u : detail::maxKPack(detail::packClassOf<InT>());
             static constexpr uint32_t BlockK     = KPack * (64u / Block); // 2 (32-wide) or 4 (16-wide) lane groups along K
             static constexpr uint32_t KPackBytes = KPack * sizeof(InT);
             static constexpr uint32_t KSteps     = MacroK / BlockK; // MFMA steps per stage (1 or 2)
@@ -105,8 +110,10 @@ namespace rocwmma_amd
 
             // (a dim-major tile holds one K index per LDS row: StageKB / sizeof(InT) rows)
             template <uint32_t Dim>
-            using DimTile = std::conditional_t<sizeof(InT) == 2u, lds::DimMajorTile<Dim, StageKB / 2u>,
-                                               lds::DimMajorTile8<(Dim == 128u || Dim == 256u) ? Dim : 128u, StageKB>>;
+            using DimTile = std::conditional_t<
+                sizeof(InT) == 4u, lds::DimMajorTile32<Dim, StageKB / 4u>,
+                std::conditional_t<sizeof(InT) == 2u, lds::DimMajorTile<Dim % 128u == 0u ? Dim : 128u, StageKB / 2u>,
+                                   lds::DimMajorTile8<(Dim == 128u || Dim == 256u) ? Dim : 128u, StageKB>>>;
             // (16-wide blocks with 32 bytes of K per lane, fp8 16x16x128: the K-major tile's pair reader)
             static constexpr bool PairReads = Block == 16u && KPackBytes == 32u && !Scaled;
             using TileA = std::conditional_t<AKMajor, lds::KMajorTile<MacroM, StageKB, PairReads>, DimTile<MacroM>>;
@@ -117,7 +124,9 @@ namespace rocwmma_amd
             static constexpr uint32_t StageBytes = BytesA + BytesB;
             static constexpr uint32_t Stages     = Stages_; // ring of K stages in LDS
             static constexpr uint32_t WavesPerSimd = WavesPerSimd_;
-            static constexpr uint32_t LdsBytes   = Stages * StageBytes;
+            static constexpr uint32_t StagesB = Stages_ + (ExtraB_ ? 1u : 0u);
+            static constexpr uint32_t RingB   = Stages * BytesA; // LDS: the A stages, then the B stages
+            static constexpr uint32_t LdsBytes   = Stages * BytesA + StagesB * BytesB;
             static constexpr uint32_t CopiesA    = BytesA / 1024u / Waves; // direct copies per wave per stage
             static constexpr uint32_t CopiesB    = BytesB / 1024u / Waves;
             static constexpr uint32_t Copies     = CopiesA + CopiesB;
@@ -132,9 +141,9 @@ namespace rocwmma_amd
             // block scales: their main loop loads scales into registers, and behind a branch that only some
             // waves take the compiler waits for every copy in flight before it uses them (five times slower).
             static constexpr uint32_t CopyWaves
-                = (Waves == 8u && WavesPerSimd_ == 2u && Stages_ == 2u && (AKMajor || BKMajor) && !Scaled_) ? 4u : Waves;
+                = (Waves == 8u && WavesPerSimd_ == 2u && (Stages_ == 2u || Stages_ == 3u) && (AKMajor || BKMajor) && !Scaled_) ? 4u : Waves;
             // LDS read instructions per MFMA step: b128 reads per block (K-major) or two transposing b64 reads
-            static constexpr uint32_t TrReads      = KPackBytes / 8u; // transposing 8-byte reads per operand
+            static constexpr uint32_t TrReads      = KPackBytes / 8u; // transposing 8-byte reads (float32: reads of two dwords) per operand
             static constexpr uint32_t ReadsA       = BlocksM * (AKMajor ? KPackBytes / 16u : TrReads);
             static constexpr uint32_t ReadsB       = BlocksN * (BKMajor ? KPackBytes / 16u : TrReads);
             static constexpr uint32_t ReadsPerStep = ReadsA + ReadsB;
@@ -143,7 +152,7 @@ namespace rocwmma_amd
             // GroupBlocks blocks (256- or 512-byte rows), two group buffers per wave
             static constexpr uint32_t GroupBlocks
                 = (WaveN == 128u && 2u * Block * 128u * sizeof(OutT) * Waves <= LdsBytes) ? 128u / Block : 64u / Block;
-            static constexpr bool StagedC = !Edges && sizeof(OutT) == 4u && WaveN % 64u == 0u
+            static constexpr bool StagedC = sizeof(OutT) == 4u && WaveN % 64u == 0u
                                             && BlocksM * (BlocksN / GroupBlocks) >= 2u
                                             && 2u * Block * GroupBlocks * Block * sizeof(OutT) * Waves <= LdsBytes;
 
@@ -156,21 +165,22 @@ namespace rocwmma_amd
             static_assert(Block == 32u || KPackBytes == 16u || ((PairReads || Scaled) && AKMajor && BKMajor && Stages_ == 2u),
                           "16-wide blocks: 16 bytes of K per lane (16-bit types, int8), or fp8 16x16x128 on K-contiguous "
                           "operands in the ring of two");
-            static_assert(sizeof(InT) == 2u || sizeof(InT) == 1u, "16-bit and 8-bit operands");
-            static_assert(sizeof(InT) == 2u || ((AKMajor || MacroM == 128u || MacroM == 256u) && (BKMajor || MacroN == 128u || MacroN == 256u)),
+            static_assert(sizeof(InT) <= 4u && (sizeof(InT) != 4u || Block == 32u), "8-bit, 16-bit and (in 32-wide blocks) float32 operands");
+            static_assert(sizeof(InT) != 1u || ((AKMajor || MacroM == 128u || MacroM == 256u) && (BKMajor || MacroN == 128u || MacroN == 256u)),
                           "dim-major tiles of 8-bit operands are 128 or 256 wide");
             static_assert(TileA::bytes == BytesA && TileB::bytes == BytesB, "stage geometry mismatch");
             static_assert(BytesA % (1024u * Waves) == 0u && BytesB % (1024u * Waves) == 0u,
                           "a stage must split into whole-wave copies evenly");
             static_assert((Stages - 1u) * Copies < 64u, "too many copies in flight for vmcnt");
-            static_assert(Stages != 2u || KSteps == 2u || KSteps == 4u || (KSteps == 1u && BlocksN % 2u == 0u),
+            static_assert(Stages == 4u || StageKB == 64u || KSteps == 2u || KSteps == 4u || (KSteps == 1u && BlocksN % 2u == 0u),
                           "the ring of two runs one (fragments streamed by columns), two or four MFMA steps per stage");
             static_assert(LdsBytes <= Constants::AMDGCN_LDS_MAX_SIZE_BYTES, "macro tile does not fit the LDS");
             // the dim-major tile's swizzle looks at K row bits 0..3: a wave's copies must all start
             // on the same K row modulo 16
-            // (the 8-bit tile's looks at K row bit 4 as well)
-            static_assert((AKMajor || (Waves * TileA::rowsPerCopy) % (sizeof(InT) == 2u ? 16u : 32u) == 0u)
-                              && (BKMajor || (Waves * TileB::rowsPerCopy) % (sizeof(InT) == 2u ? 16u : 32u) == 0u),
+            // (the 8-bit tile's looks at K row bit 4 as well, the float32 tile's at bit 2 only)
+            static constexpr uint32_t SwizzleRows = sizeof(InT) == 4u ? 8u : (sizeof(InT) == 2u ? 16u : 32u);
+            static_assert((AKMajor || (Waves * TileA::rowsPerCopy) % SwizzleRows == 0u)
+                              && (BKMajor || (Waves * TileB::rowsPerCopy) % SwizzleRows == 0u),
                           "wave pool too small for the dim-major tile");
             // the K-major tile's swizzle looks at row bits 0..3 likewise
             static_assert((!AKMajor || (Waves * TileA::rowsPerCopy) % 16u == 0u)
@@ -464,12 +474,23 @@ namespace rocwmma_amd
                 bLaneOff[j] = TileB::laneSourceOffset(lane, wave % CopyWaves + (Cfg::BKMajor ? 0u : j * CopyWaves), ldbB);
             }
 
+            // Edges: what is left of K (elements) at the stage the next copies read, and the first K element of
+            // this lane's 16 bytes of a K-contiguous operand.  A lane whose bytes lie past the end of K asks for
+            // an address beyond the buffer's bounds and gets zeros; rows of a dim-major operand past K are
+            // beyond its end as they are.  Two vector instructions per operand and stage.
+            uint32_t       aLeft = k - stage0 * Cfg::MacroK, bLeft = aLeft;
+            const uint32_t aLaneK = TileA::laneK(lane, wave % CopyWaves) / static_cast<uint32_t>(sizeof(InT));
+            const uint32_t bLaneK = TileB::laneK(lane, wave % CopyWaves) / static_cast<uint32_t>(sizeof(InT));
+            auto           insideK = [](bool kMajor, uint32_t offset, uint32_t laneK, uint32_t left) {
+                return (Cfg::Edges && kMajor && laneK >= left) ? (offset | 0x80000000u) : offset;
+            };
+
             // A stage is copied in two halves (the A operand, then the B operand) so that each
             // MFMA phase of an iteration carries half of the copy instructions.
             // advance == false leaves the source on the stage just copied (used to re-copy the last
-            // stage instead of running past the end of the operand)
+            // stage instead of running past the end of the operand; edge tiles read nothing there)
             auto issueA = [&](uint32_t slot, bool advance = true) {
-                char*                 ldsA = ldsRaw + slot * Cfg::StageBytes;
+                char*                 ldsA = ldsRaw + slot * Cfg::BytesA;
                 const lds::BufferRsrc src  = Cfg::Edges ? lds::makeSource(aSrc, aEnd) : lds::makeSource(aSrc);
                 if constexpr(CopyWaves < Cfg::Waves)
                 {
@@ -480,7 +501,8 @@ namespace rocwmma_amd
                         {
                             // (copy i * CopyWaves + wave = copy i / CopyShares of wave + (i % CopyShares) * CopyWaves)
                             const uint32_t copy = i * CopyWaves + wave;
-                            lds::asyncCopy16(ldsA + copy * 1024u, src, aLaneOff[i % CopyShares], TileA::copySourceOffset(copy, ldaB));
+                            lds::asyncCopy16(ldsA + copy * 1024u, src, insideK(Cfg::AKMajor, aLaneOff[i % CopyShares], aLaneK, aLeft),
+                                             TileA::copySourceOffset(copy, ldaB));
                         }
                     }
                 }
@@ -490,13 +512,20 @@ namespace rocwmma_amd
                     for(uint32_t i = 0; i < Cfg::CopiesA; ++i)
                     {
                         const uint32_t copy = i * Cfg::Waves + wave;
-                        lds::asyncCopy16(ldsA + copy * 1024u, src, aLaneOff[0], TileA::copySourceOffset(copy, ldaB));
+                        lds::asyncCopy16(ldsA + copy * 1024u, src, insideK(Cfg::AKMajor, aLaneOff[0], aLaneK, aLeft),
+                                         TileA::copySourceOffset(copy, ldaB));
                     }
                 }
-                aSrc += advance ? aStep : size_t{0};
+                if constexpr(Cfg::Edges)
+                {
+                    aSrc += aStep;
+                    aLeft = aLeft > Cfg::MacroK ? aLeft - Cfg::MacroK : 0u;
+                }
+                else
+                    aSrc += advance ? aStep : size_t{0};
             };
             auto issueB = [&](uint32_t slot, bool advance = true) {
-                char*                 ldsB = ldsRaw + slot * Cfg::StageBytes + Cfg::BytesA;
+                char*                 ldsB = ldsRaw + Cfg::RingB + slot * Cfg::BytesB;
                 const lds::BufferRsrc src  = Cfg::Edges ? lds::makeSource(bSrc, bEnd) : lds::makeSource(bSrc);
                 if constexpr(CopyWaves < Cfg::Waves)
                 {
@@ -507,7 +536,8 @@ namespace rocwmma_amd
                         {
                             // (copy i * CopyWaves + wave = copy i / CopyShares of wave + (i % CopyShares) * CopyWaves)
                             const uint32_t copy = i * CopyWaves + wave;
-                            lds::asyncCopy16(ldsB + copy * 1024u, src, bLaneOff[i % CopyShares], TileB::copySourceOffset(copy, ldbB));
+                            lds::asyncCopy16(ldsB + copy * 1024u, src, insideK(Cfg::BKMajor, bLaneOff[i % CopyShares], bLaneK, bLeft),
+                                             TileB::copySourceOffset(copy, ldbB));
                         }
                     }
                 }
@@ -517,10 +547,17 @@ namespace rocwmma_amd
                     for(uint32_t i = 0; i < Cfg::CopiesB; ++i)
                     {
                         const uint32_t copy = i * Cfg::Waves + wave;
-                        lds::asyncCopy16(ldsB + copy * 1024u, src, bLaneOff[0], TileB::copySourceOffset(copy, ldbB));
+                        lds::asyncCopy16(ldsB + copy * 1024u, src, insideK(Cfg::BKMajor, bLaneOff[0], bLaneK, bLeft),
+                                         TileB::copySourceOffset(copy, ldbB));
                     }
                 }
-                bSrc += advance ? bStep : size_t{0};
+                if constexpr(Cfg::Edges)
+                {
+                    bSrc += bStep;
+                    bLeft = bLeft > Cfg::MacroK ? bLeft - Cfg::MacroK : 0u;
+                }
+                else
+                    bSrc += advance ? bStep : size_t{0};
             };
             auto issueStage = [&](uint32_t slot, bool advance = true) {
                 issueA(slot, advance);
@@ -533,9 +570,9 @@ namespace rocwmma_amd
                 typename Cfg::FragB b[Cfg::BlocksN];
             };
 
-            auto readFrags = [&](Frags& f, uint32_t slot, uint32_t ks) {
-                const char* ldsA = ldsRaw + slot * Cfg::StageBytes;
-                const char* ldsB = ldsA + Cfg::BytesA;
+            auto readFragsOf = [&](Frags& f, uint32_t slot, uint32_t slotB, uint32_t ks) {
+                const char* ldsA = ldsRaw + slot * Cfg::BytesA;
+                const char* ldsB = ldsRaw + Cfg::RingB + slotB * Cfg::BytesB;
                 if constexpr(Cfg::Scaled && Cfg::Block == 16u) // (has a reader of its own in its loop)
                     return;
                 else if constexpr(Cfg::Scaled)
@@ -575,6 +612,8 @@ namespace rocwmma_amd
                 }
                 }
             };
+
+            auto readFrags = [&](Frags& f, uint32_t slot, uint32_t ks) { readFragsOf(f, slot, slot, ks); };
 
             // Fragments of a dim-major operand come from inline-assembly transposing reads: after the wait
             // that covers those reads, their registers are tied to that point of the program.
@@ -649,10 +688,18 @@ namespace rocwmma_amd
                     loadScales(sA, sB, 0u);
                     __builtin_amdgcn_sched_barrier(0); // (and stay in front of them)
                 }
-                issueStage(0u, 1u < stages);
-                issueStage(1u, 2u < stages);
-                lds::waitCopiesAndReads<(CopyWaves == Cfg::Waves ? Cfg::Copies : 0u)>(); // stage 0 has landed
+                constexpr uint32_t SB = Cfg::StagesB;
+#pragma unroll
+                for(uint32_t st = 0; st < SB; ++st)
+                {
+                    if(st < S)
+                        issueA(st, st + 1u < stages);
+                    issueB(st, st + 1u < stages);
+                }
+                constexpr uint32_t InFlight = (SB - 2u) * Cfg::CopiesB * CopyShares;
+                lds::waitCopiesAndReads<(Cfg::CopiesA + (SB - 1u) * Cfg::CopiesB) * CopyShares>(); // stage 0 has landed
                 lds::barrier();
+                uint32_t slotB = 0u; // of the stage that is multiplied
                 // B column buffers: `Ahead` columns are read in advance.  With three (four buffers, whose indices
                 // repeat every stage of four or eight columns) the barrier moves in front of the last three
                 // columns, so that what follows it (the copies, the next stage's A fragments and first B columns)
@@ -665,7 +712,7 @@ namespace rocwmma_amd
                 typename Cfg::FragA fa[2][Cfg::BlocksM];
                 typename Cfg::FragB fb[NB];
                 auto readA = [&](typename Cfg::FragA(&dst)[Cfg::BlocksM], uint32_t slot) {
-                    const char* ldsA = ldsRaw + slot * Cfg::StageBytes;
+                    const char* ldsA = ldsRaw + slot * Cfg::BytesA;
 #pragma unroll
                     for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                     {
@@ -680,7 +727,7 @@ namespace rocwmma_amd
                     }
                 };
                 auto readB = [&](typename Cfg::FragB& dst, uint32_t slot, uint32_t bj) {
-                    const char*    ldsB = ldsRaw + slot * Cfg::StageBytes + Cfg::BytesA;
+                    const char*    ldsB = ldsRaw + Cfg::RingB + slot * Cfg::BytesB;
                     const uint32_t c0   = waveN * Cfg::WaveN + bj * Cfg::Block;
                     if constexpr(Cfg::Scaled)
                     {
@@ -726,15 +773,17 @@ namespace rocwmma_amd
                         constexpr uint32_t slot = decltype(slotC)::value;
                         staticFor<Cfg::BlocksN - Ahead>([&](auto bjC) {
                             constexpr uint32_t bj = decltype(bjC)::value;
-                            readB(fb[(bj + Ahead) % NB], slot, bj + Ahead);
+                            readB(fb[(bj + Ahead) % NB], slotB, bj + Ahead);
                             column(cur, fb[bj % NB], bjC, slotC);
                             scheduleInterleaved<Cfg::BlocksM, RB, 0u>();
                             __builtin_amdgcn_sched_barrier(0);
                         });
-                        lds::waitCopiesAndReads<0u>(); // stage ii + 1 has landed, stage ii is in registers
+                        lds::waitCopiesAndReads<InFlight>(); // stage ii + 1 has landed, stage ii is in registers
                         lds::barrier();
                         __builtin_amdgcn_sched_barrier(0);
-                        issueStage(slot, ii + 3u < stages);
+                        issueA(slot, ii + 3u < stages);
+                        issueB(slotB, ii + SB + 1u < stages);
+                        slotB = slotB + 1u == SB ? 0u : slotB + 1u;
                         if constexpr(Cfg::Scaled && slot == 0u)
                         {
                             // scales of the next pair of stages (the last pair again past the end of K)
@@ -744,7 +793,7 @@ namespace rocwmma_amd
                         staticFor<Ahead>([&](auto tC) {
                             constexpr uint32_t t  = decltype(tC)::value;
                             constexpr uint32_t bj = Cfg::BlocksN - Ahead + t;
-                            readB(fb[(bj + Ahead) % NB], slot ^ 1u, t);
+                            readB(fb[(bj + Ahead) % NB], slotB, t);
                             column(cur, fb[bj % NB], std::integral_constant<uint32_t, bj>{}, slotC);
                             if constexpr(Ahead > 1u)
                                 __builtin_amdgcn_sched_barrier(0);
@@ -771,7 +820,7 @@ namespace rocwmma_amd
                 lds::waitCopiesAndReads<0u>(); // the surplus copies still target this workgroup's LDS
                 lds::barrier();
             }
-            else if constexpr(S == 2u)
+            else if constexpr(S == 2u || S == 3u || (S == 5u && Cfg::StageKB == 128u))
             {
                 // Ring of two stages of 128 bytes of K (two or four MFMA steps each).  A phase multiplies
                 // one step while it reads the fragments of the next; the barrier in front of a stage's
@@ -811,9 +860,18 @@ namespace rocwmma_amd
                     loadScales32(sA, sB, 0u);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                issueStage(0u, 1u < stages);
-                issueStage(1u, 2u < stages);
-                lds::waitCopiesAndReads<(CopyWaves == Cfg::Waves ? Cfg::Copies : 0u)>(); // stage 0 has landed
+                constexpr uint32_t SB = Cfg::StagesB;
+#pragma unroll
+                for(uint32_t st = 0; st < SB; ++st)
+                {
+                    if(st < S)
+                        issueA(st, st + 1u < stages);
+                    issueB(st, st + 1u < stages);
+                }
+                // (copies of later stages that may be in flight when a stage must have landed; the waves that issue
+                // none do not wait)
+                constexpr uint32_t InFlight = ((S - 2u) * Cfg::CopiesA + (SB - 2u) * Cfg::CopiesB) * CopyShares;
+                lds::waitCopiesAndReads<((S - 1u) * Cfg::CopiesA + (SB - 1u) * Cfg::CopiesB) * CopyShares>(); // stage 0 has landed
                 lds::barrier();
                 constexpr uint32_t N = Cfg::KSteps; // MFMA steps per stage: 2 or 4 (even: the fragment sets alternate)
                 Frags              f[2];
@@ -844,8 +902,10 @@ namespace rocwmma_amd
                     }
                 };
                 readFrags(f[0], 0u, 0u);
+                uint32_t slot = 0u, slotB = 0u; // of stage i
                 for(uint32_t i = 0; i < stages; ++i)
                 {
+                    const uint32_t nextSlot = slot + 1u == S ? 0u : slot + 1u, nextSlotB = slotB + 1u == SB ? 0u : slotB + 1u;
 #pragma unroll
                     for(uint32_t ks = 0; ks + 1u < N; ++ks)
                     {
@@ -855,22 +915,25 @@ namespace rocwmma_amd
                             pinFrags(f[ks & 1u]);
                             __builtin_amdgcn_sched_barrier(0);
                         }
-                        readFrags(f[(ks + 1u) & 1u], i % 2u, ks + 1u);
+                        readFragsOf(f[(ks + 1u) & 1u], slot, slotB, ks + 1u);
                         multiplyStep(f[ks & 1u], i, ks);
                         scheduleInterleaved<Cfg::MfmasPerStep / 2u, Cfg::ReadsPerStep, 0u>();
                         __builtin_amdgcn_sched_barrier(0);
                     }
-                    lds::waitCopiesAndReads<0u>(); // stage i+1 has landed, stage i is in registers
+                    lds::waitCopiesAndReads<InFlight>(); // stage i+1 has landed, stage i is in registers
                     pinFrags(f[(N - 1u) & 1u]);
                     lds::barrier();
                     __builtin_amdgcn_sched_barrier(0);
-                    issueStage(i % 2u, i + 3u < stages);
+                    issueA(slot, i + S + 1u < stages);
+                    issueB(slotB, i + SB + 1u < stages);
                     if constexpr(Cfg::Scaled)
                     {
                         if(i % 2u == 0u)
                             loadScales32(sAnext, sBnext, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
                     }
-                    readFrags(f[0], (i + 1u) % 2u, 0u);
+                    readFragsOf(f[0], nextSlot, nextSlotB, 0u);
+                    slot  = nextSlot;
+                    slotB = nextSlotB;
                     multiplyStep(f[(N - 1u) & 1u], i, N - 1u);
                     if constexpr(Cfg::Scaled)
                     {
@@ -1068,8 +1131,8 @@ namespace rocwmma_amd
                 // stage, then its MFMAs): 5 % faster than leaving the reads in front of the MFMAs.  With
                 // only A dim-major (4 blocks) the compiler's placement is 1 % better and is kept.
                 auto phaseByColumns = [&](Frags const& cur, Frags& nxt, uint32_t slot) {
-                    const char* ldsA = ldsRaw + slot * Cfg::StageBytes;
-                    const char* ldsB = ldsA + Cfg::BytesA;
+                    const char* ldsA = ldsRaw + slot * Cfg::BytesA;
+                    const char* ldsB = ldsRaw + Cfg::RingB + slot * Cfg::BytesB;
                     if constexpr(Cfg::Block == 16u)
                     {
                         static_assert(Cfg::BlocksM <= Cfg::BlocksN, "the A blocks are read along with the first B columns");
@@ -1199,9 +1262,12 @@ namespace rocwmma_amd
             // (even rows: of the first block, odd rows: of the second) and moves 16 bytes; an
             // instruction then covers 64 contiguous bytes per matrix row.  The exchange is its own
             // inverse, so C is read the same way.
-            constexpr bool PairIO = !Cfg::Edges && Cfg::Block == 16u && sizeof(OutT) == 2u && Cfg::BlocksN % 2u == 0u;
+            constexpr bool PairIO = Cfg::Block == 16u && sizeof(OutT) == 2u && Cfg::BlocksN % 2u == 0u;
             const uint32_t pairCol = (accGroup & 1u) * 16u + 4u * (accGroup & 2u);
-            auto           swapPair = [](auto& fx, auto& fy) {
+            auto           blockOffset = [&](uint32_t bi, uint32_t bj, uint32_t ld) {
+                return static_cast<size_t>(wRow + bi * Cfg::Block) * ld + wCol + bj * Cfg::Block;
+            };
+            auto swapPair = [](auto& fx, auto& fy) {
                 uint32_t x[2], y[2];
                 __builtin_memcpy(x, fx.x, 8);
                 __builtin_memcpy(y, fy.x, 8);
@@ -1215,23 +1281,27 @@ namespace rocwmma_amd
                 __builtin_memcpy(fx.x, x, 8);
                 __builtin_memcpy(fy.x, y, 8);
             };
-            auto storePair = [&](OutT* dst, auto& fx, auto& fy, uint32_t ld) {
+            // (edge tiles: a lane's eight columns of one row are inside the problem or outside it as a whole)
+            auto insidePair = [&](uint32_t bi, uint32_t bj) {
+                return !Cfg::Edges || (wRow + bi * Cfg::Block + accRow < m && wCol + bj * Cfg::Block + pairCol < n);
+            };
+            auto storePair = [&](uint32_t bi, uint32_t bj, auto& fx, auto& fy) {
                 swapPair(fx, fy);
                 typedef uint32_t Words __attribute__((ext_vector_type(4)));
                 Words            v;
                 __builtin_memcpy(&v, fx.x, 8);
                 __builtin_memcpy(reinterpret_cast<char*>(&v) + 8, fy.x, 8);
-                *reinterpret_cast<Words*>(dst + static_cast<size_t>(accRow) * ld + pairCol) = v;
+                if(insidePair(bi, bj))
+                    *reinterpret_cast<Words*>(d + blockOffset(bi, bj, ldd) + static_cast<size_t>(accRow) * ldd + pairCol) = v;
             };
-            auto loadPair = [&](auto& fx, auto& fy, const OutT* src, uint32_t ld) {
+            auto loadPair = [&](uint32_t bi, uint32_t bj, auto& fx, auto& fy) {
                 typedef uint32_t Words __attribute__((ext_vector_type(4)));
-                const Words      v = *reinterpret_cast<const Words*>(src + static_cast<size_t>(accRow) * ld + pairCol);
+                Words            v = {};
+                if(insidePair(bi, bj))
+                    v = *reinterpret_cast<const Words*>(c + blockOffset(bi, bj, ldc) + static_cast<size_t>(accRow) * ldc + pairCol);
                 __builtin_memcpy(fx.x, &v, 8);
                 __builtin_memcpy(fy.x, reinterpret_cast<const char*>(&v) + 8, 8);
                 swapPair(fx, fy);
-            };
-            auto           blockOffset = [&](uint32_t bi, uint32_t bj, uint32_t ld) {
-                return static_cast<size_t>(wRow + bi * Cfg::Block) * ld + wCol + bj * Cfg::Block;
             };
             // Fused configurations: the bias values of a lane's columns of one block are fetched (four
             // consecutive floats per run, cache hits after the first row of blocks) just before the
@@ -1320,10 +1390,20 @@ namespace rocwmma_amd
 #pragma unroll
                         for(uint32_t i = 0; i < CopiesC; ++i)
                         {
-                            const uint32_t r = RowsPerCopy * i + cpRow;
-                            lds::asyncCopy16Streaming(myLds + (gi % 2u) * GroupBytes + i * 1024u,
-                                                      cWave + (bi * Cfg::Block + r) * ldcB + bj0 * Cfg::Block * sizeof(OutT)
-                                                          + ((chunk ^ (r & 15u)) << 4));
+                            const uint32_t r   = RowsPerCopy * i + cpRow;
+                            const uint32_t col = bj0 * Cfg::Block * static_cast<uint32_t>(sizeof(OutT)) + ((chunk ^ (r & 15u)) << 4);
+                            const char*    src;
+                            if constexpr(!Cfg::Edges)
+                                src = cWave + (bi * Cfg::Block + r) * ldcB + col;
+                            else
+                            {
+                                // (rows and columns past the problem's fetch some element of C, used by nobody)
+                                const uint32_t row  = wRow + bi * Cfg::Block + r;
+                                const uint32_t colB = wCol * static_cast<uint32_t>(sizeof(OutT)) + col;
+                                src = reinterpret_cast<const char*>(c) + static_cast<size_t>(row < m ? row : m - 1u) * ldcB
+                                      + (colB < n * static_cast<uint32_t>(sizeof(OutT)) ? colB : 0u);
+                            }
+                            lds::asyncCopy16Streaming(myLds + (gi % 2u) * GroupBytes + i * 1024u, src);
                         }
                     };
                     const uint32_t rdRow  = accRow;
@@ -1335,8 +1415,13 @@ namespace rocwmma_amd
                     {
                         const uint32_t bi = gi / GroupsPerRow, bj0 = (gi % GroupsPerRow) * GB;
                         // vector-memory operations younger than this group's copies: the next
-                        // group's copies and the stores of the two previous groups
-                        if(gi == 0u)
+                        // group's copies and the stores of the two previous groups (which edge tiles
+                        // may not issue: there only the copies count)
+                        if(Cfg::Edges && gi + 1u < NG)
+                            lds::waitCopiesAndReads<CopiesC>();
+                        else if(Cfg::Edges)
+                            lds::waitCopiesAndReads<0u>();
+                        else if(gi == 0u)
                             lds::waitCopiesAndReads<CopiesC>();
                         else if(gi == 1u)
                             lds::waitCopiesAndReads<(NG > 2u ? CopiesC : 0u) + StoresD>();
@@ -1386,7 +1471,7 @@ namespace rocwmma_amd
                     {
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; bj += 2u)
-                            loadPair(fc[bi % 2u][bj], fc[bi % 2u][bj + 1u], c + blockOffset(bi, bj, ldc), ldc);
+                            loadPair(bi, bj, fc[bi % 2u][bj], fc[bi % 2u][bj + 1u]);
                     }
                     else
                     {
@@ -1414,7 +1499,7 @@ namespace rocwmma_amd
                     {
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; bj += 2u)
-                            storePair(d + blockOffset(bi, bj, ldd), fc[bi % 2u][bj], fc[bi % 2u][bj + 1u], ldd);
+                            storePair(bi, bj, fc[bi % 2u][bj], fc[bi % 2u][bj + 1u]);
                     }
                     else
                     {
@@ -1468,7 +1553,7 @@ namespace rocwmma_amd
                         {
 #pragma unroll
                             for(uint32_t bj = 0; bj < Cfg::BlocksN; bj += 2u)
-                                storePair(d + blockOffset(bi, bj, ldd), fd[bj], fd[bj + 1u], ldd);
+                                storePair(bi, bj, fd[bj], fd[bj + 1u]);
                         }
                         else
                         {

@@ -1,0 +1,17 @@
+// The blocked GEMM's tile ladder for f16 operands.
+#include "gemm_blocked_ladder.hpp"
+
+using namespace rocwmma;
+
+namespace rocwmma_amd
+{
+    int launchGemmBlockedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile)
+    {
+        if(dtypeOut == ROCWMMA_AMD_F32)
+            return pickLayout<float16_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+        if(dtypeOut == ROCWMMA_AMD_F16)
+            return pickLayout<float16_t, float16_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+        return ROCWMMA_AMD_UNSUPPORTED_TYPE;
+    }
+
+} // namespace rocwmma_amd

@@ -1,0 +1,18 @@
+// The blocked GEMM's tile ladder for fp8 operands.
+#include "gemm_blocked_ladder.hpp"
+
+using namespace rocwmma;
+
+namespace rocwmma_amd
+{
+    int launchGemmBlockedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream,
+                             bool forceLargeTile)
+    {
+        if(dtypeIn == ROCWMMA_AMD_E4M3 && dtypeOut == ROCWMMA_AMD_F32)
+            return pickLayout<float8_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+        if(dtypeIn == ROCWMMA_AMD_E5M2 && dtypeOut == ROCWMMA_AMD_F32)
+            return pickLayout<bfloat8_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+        return ROCWMMA_AMD_UNSUPPORTED_TYPE;
+    }
+
+} // namespace rocwmma_amd

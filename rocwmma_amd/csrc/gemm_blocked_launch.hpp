@@ -1,6 +1,6 @@
 // Blocked GEMM for gfx950: the kernels around gemmTile (one macro tile per workgroup; two tilings in one
 // launch for a last round that would be at most half full) and their launch helpers.  Included by the
-// translation units that instantiate tile configurations (gemm_blocked.hip, gemm_fused.hip).
+// translation units that instantiate tile configurations.
 #ifndef ROCWMMA_AMD_CSRC_GEMM_BLOCKED_LAUNCH_HPP
 #define ROCWMMA_AMD_CSRC_GEMM_BLOCKED_LAUNCH_HPP
 
@@ -10,6 +10,17 @@ namespace rocwmma_amd
 {
     namespace
     {
+        // Pipeline stages of a whole K range.  Edge configurations take any K: the last stage may be partly filled, and
+        // a K shorter than the ring's prologue gets stages of zeros.
+        template <typename Cfg>
+        ROCWMMA_HOST_DEVICE ROCWMMA_INLINE uint32_t stagesOf(uint32_t k)
+        {
+            if constexpr(!Cfg::Edges)
+                return k / Cfg::MacroK;
+            const uint32_t stages = k / Cfg::MacroK + (k % Cfg::MacroK != 0u ? 1u : 0u);
+            return stages < Cfg::Stages - 1u ? Cfg::Stages - 1u : stages;
+        }
+
         template <typename Cfg>
         __global__ void __launch_bounds__(Cfg::Threads) __attribute__((amdgpu_waves_per_eu(Cfg::WavesPerSimd, Cfg::WavesPerSimd)))
         gemmBlockedKernel(uint32_t                   m,
@@ -29,7 +40,7 @@ namespace rocwmma_amd
         {
             uint32_t tm, tn;
             tileOfWorkgroup(blockIdx.x, ceilDiv(m, Cfg::MacroM), ceilDiv(n, Cfg::MacroN), tm, tn);
-            gemmTile<Cfg>(tm, tn, 0u, k / Cfg::MacroK, m, n, k, a, b, c, d, lda, ldb, ldc, ldd, alpha, beta, StreamKPart{}, ex);
+            gemmTile<Cfg>(tm, tn, 0u, stagesOf<Cfg>(k), m, n, k, a, b, c, d, lda, ldb, ldc, ldd, alpha, beta, StreamKPart{}, ex);
         }
 
         // Two tilings in one launch: the first `fullTiles` workgroups run Full tiles, the others the two
@@ -116,8 +127,8 @@ namespace rocwmma_amd
         template <typename Cfg>
         int launchCfg(GemmArgs const& g, hipStream_t stream, TileExtras const& ex = TileExtras{})
         {
-            if((!Cfg::Edges && (g.m % Cfg::MacroM != 0u || g.n % Cfg::MacroN != 0u)) || g.k % Cfg::MacroK != 0u
-               || g.k < (Cfg::Stages - 1u) * Cfg::MacroK)
+            if(!Cfg::Edges
+               && (g.m % Cfg::MacroM != 0u || g.n % Cfg::MacroN != 0u || g.k % Cfg::MacroK != 0u || g.k < (Cfg::Stages - 1u) * Cfg::MacroK))
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
             // a stage's copies address their source inside a 2 GiB window from the stage origin
             {
@@ -156,26 +167,6 @@ namespace rocwmma_amd
                                static_cast<typename Cfg::CompT>(g.beta),
                                ex);
             return launchStatus();
-        }
-
-        // The 4-wave configurations come with either LDS pipeline.  With at most one workgroup per
-        // compute unit a launch is one round of latency-bound workgroups, and the ring of four 64-byte
-        // stages (copies three stages ahead) hides more of it: 128 x 14336 x 4096 int8 25.8 against 29.7 us,
-        // 2048^3 f16 24 against 27 us.  With more workgroups than compute units the units stream operands
-        // all the time, the L2 request rate limits them, and the ring of two 128-byte stages (whole-line
-        // requests) wins: 512 x 14336 x 4096 int8 51 -> 44 us, f16 with a row-major B 101 -> 85 us,
-        // 192 x 14336 x 4096 f16 (64 x 64 tiles) 74 -> 56 us.  Results are identical bit for bit.
-        template <typename Ring4, typename Ring2>
-        int launchByRounds(GemmArgs const& g, hipStream_t stream, TileExtras const& ex = TileExtras{})
-        {
-            static_assert(Ring4::MacroM == Ring2::MacroM && Ring4::MacroN == Ring2::MacroN, "same tiling");
-            if(ceilDiv(g.m, Ring4::MacroM) * ceilDiv(g.n, Ring4::MacroN) > computeUnits())
-            {
-                const int rc = launchCfg<Ring2>(g, stream, ex);
-                if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE) // (K not in whole 128-byte stages)
-                    return rc;
-            }
-            return launchCfg<Ring4>(g, stream, ex);
         }
     } // namespace
 } // namespace rocwmma_amd
