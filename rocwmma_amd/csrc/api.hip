@@ -12,12 +12,12 @@ namespace rocwmma_amd
     int launchGemv(uint32_t m, uint32_t k, uint32_t ncols, const void* a, uint32_t lda, const void* x, uint32_t ldx,
                    float* y, uint32_t ldy, float alpha, float beta, hipStream_t stream);
     int launchDlrmFwd(const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
-    int launchDlrmFwdF32(const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
+    int launchDlrmFwdSample(int dtype, const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
+    int launchDlrmBwdSample(int dtype, const void* input, const void* upstream, void* grad, void* mlpGrad, uint32_t m, uint32_t k,
+                            uint32_t batch, hipStream_t stream);
     int launchDlrmFwdGeneral(int dtype, const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
     int launchDlrmBwdGeneral(int dtype, const void* input, const void* upstream, void* grad, void* mlpGrad, uint32_t m, uint32_t k,
                              uint32_t batch, hipStream_t stream);
-    int launchDlrmBwdF32(const void* input, const void* upstream, void* grad, void* mlpGrad, uint32_t m, uint32_t k, uint32_t batch,
-                         hipStream_t stream);
     int launchDlrmBwd(const void* input, const void* upstream, void* grad, void* mlpGrad, uint32_t m, uint32_t k,
                       uint32_t batch, hipStream_t stream);
 
@@ -579,8 +579,8 @@ int rocwmma_amd_gemv(uint32_t    m,
     return launchGemv(m, k, ncols, a, lda, x, ldx, y, ldy, alpha, beta, asStream(stream));
 }
 
-// The one-wave-per-sample kernels take these shapes; the tiled kernels of dlrm_general.hip take the others.
-static bool dlrmSampleFitsAWave(uint32_t m, uint32_t k)
+// Whether a width is one of those every kernel takes, whatever the element type and row count (up to 128).
+static bool dlrmCommonWidth(uint32_t m, uint32_t k)
 {
     return m <= 128u && (k == 32u || k == 64u || k == 128u || k == 256u);
 }
@@ -591,7 +591,7 @@ static int checkDlrm(int dtype, uint32_t m, uint32_t k, uint32_t batch)
         return ROCWMMA_AMD_INVALID_ARGUMENT;
     // the tiled kernels read rows in 16-byte pieces and address a sample's features with 32-bit byte offsets
     const uint32_t size = dtype == ROCWMMA_AMD_F16 ? 2u : 4u;
-    if(!dlrmSampleFitsAWave(m, k) && (m > 32768u || k % (16u / size) != 0u || static_cast<uint64_t>(m) * k * size >= (1ull << 31)))
+    if(!dlrmCommonWidth(m, k) && (m > 32768u || k % (16u / size) != 0u || static_cast<uint64_t>(m) * k * size >= (1ull << 31)))
         return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
     return ROCWMMA_AMD_OK;
 }
@@ -607,12 +607,13 @@ int rocwmma_amd_dlrm_fwd(const void* input, void* output, uint32_t m, uint32_t k
         return ROCWMMA_AMD_BAD_ALIGNMENT;
     if(!isGfx950Current())
         return ROCWMMA_AMD_NO_DEVICE;
-    if(dlrmSampleFitsAWave(m, k))
-    {
-        rc = launchDlrmFwd(input, output, m, k, batch, asStream(stream));
-        if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE) // (a sample larger than the LDS: tiles)
-            return rc;
-    }
+    // 17 to 32 rows of the usual widths; samples that fit the LDS; tiles
+    rc = launchDlrmFwd(input, output, m, k, batch, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+        return rc;
+    rc = launchDlrmFwdSample(ROCWMMA_AMD_F16, input, output, m, k, batch, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+        return rc;
     return launchDlrmFwdGeneral(ROCWMMA_AMD_F16, input, output, m, k, batch, asStream(stream));
 }
 
@@ -634,12 +635,12 @@ int rocwmma_amd_dlrm_bwd(const void* input,
         return ROCWMMA_AMD_BAD_ALIGNMENT;
     if(!isGfx950Current())
         return ROCWMMA_AMD_NO_DEVICE;
-    if(dlrmSampleFitsAWave(m, k))
-    {
-        rc = launchDlrmBwd(input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
-        if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
-            return rc;
-    }
+    rc = launchDlrmBwd(input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+        return rc;
+    rc = launchDlrmBwdSample(ROCWMMA_AMD_F16, input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+        return rc;
     return launchDlrmBwdGeneral(ROCWMMA_AMD_F16, input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
 }
 
@@ -658,8 +659,9 @@ int rocwmma_amd_dlrm_fwd_ex(int dtype, const void* input, void* output, uint32_t
         return ROCWMMA_AMD_BAD_ALIGNMENT;
     if(!isGfx950Current())
         return ROCWMMA_AMD_NO_DEVICE;
-    if(dlrmSampleFitsAWave(m, k))
-        return launchDlrmFwdF32(input, output, m, k, batch, asStream(stream));
+    rc = launchDlrmFwdSample(ROCWMMA_AMD_F32, input, output, m, k, batch, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+        return rc;
     return launchDlrmFwdGeneral(ROCWMMA_AMD_F32, input, output, m, k, batch, asStream(stream));
 }
 
@@ -686,8 +688,9 @@ int rocwmma_amd_dlrm_bwd_ex(int         dtype,
         return ROCWMMA_AMD_BAD_ALIGNMENT;
     if(!isGfx950Current())
         return ROCWMMA_AMD_NO_DEVICE;
-    if(dlrmSampleFitsAWave(m, k))
-        return launchDlrmBwdF32(input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
+    rc = launchDlrmBwdSample(ROCWMMA_AMD_F32, input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+        return rc;
     return launchDlrmBwdGeneral(ROCWMMA_AMD_F32, input, upstream_grad, grad, bottom_mlp_grad, m, k, batch, asStream(stream));
 }
 

@@ -1,5 +1,5 @@
-// DLRM dot interaction for the shapes the one-wave-per-sample kernels (dlrm.hip, dlrm_f32.hip) do not take:
-// more than 128 feature rows, or a feature width other than 32 / 64 / 128 / 256.  The reference's tests run
+// DLRM dot interaction for the shapes the kernels that hold samples in LDS (dlrm.hip, dlrm_sample.hip) do not take:
+// samples larger than the LDS or of more than 192 feature rows.  The reference's tests run
 // (m, k) = (1024, 1024) among others (test/dlrm/test/dlrm_test_params.hpp:51-68); semantics = dlrm_fwd_CPU /
 // dlrm_bwd_CPU (test/reference_impl.hpp:83-179).
 //
