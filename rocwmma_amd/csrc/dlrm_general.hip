@@ -403,8 +403,8 @@ namespace rocwmma_amd
                 for(uint32_t i = 0; i < 4u; ++i)
                     pieceAt[i] += below ? 128u : rowStep + 1024u * i;
                 rowStep += below ? 0u : 8192u;
-                // The waits below count these loads, so they are issued here: `upstream` is no __restrict pointer, or the
-                // compiler may move them past this statement and past barriers.
+                // Issued here, a stage ahead of their use: `upstream` is no __restrict pointer, or the compiler may move the
+                // loads past this statement and past barriers.
                 asm volatile("" ::: "memory");
             };
             auto storeS = [&](u32x4_t(&rs)[4], uint32_t c0) {
@@ -567,7 +567,7 @@ namespace rocwmma_amd
 #pragma unroll
             for(uint32_t st = 0; st < Cfg::RingF; ++st)
                 copyF(st);
-            __builtin_amdgcn_sched_barrier(0); // (the waits count on this order)
+            __builtin_amdgcn_sched_barrier(0);
             loadS(rs, 0u);
             loadS(rs1, 64u);
             __builtin_amdgcn_sched_barrier(0);
@@ -575,7 +575,7 @@ namespace rocwmma_amd
             loadS(rs, 128u);
             __builtin_amdgcn_sched_barrier(0);
             storeS(rs1, 64u);
-            lds::waitCopiesAndReads<4u>(); // all but S(2) has landed
+            lds::waitCopiesAndReads<2u * Cfg::CopiesF>(); // F(0) has landed
             lds::barrier();
 
             const std::integral_constant<uint32_t, 0u> first{};
@@ -594,9 +594,10 @@ namespace rocwmma_amd
                     multiply(f[ks & 1u]);
                     __builtin_amdgcn_sched_barrier(0);
                 });
-                // F(i + 1) has landed (F(i + 2) and the pieces of S(i + 2) may be on their way), this wave's part of S(i + 1) is
-                // in LDS, stage i is in registers
-                lds::waitCopiesAndReads<Cfg::CopiesF + 4u>();
+                // F(i + 1) has landed (F(i + 2) may be on its way), this wave's part of S(i + 1) is in LDS, stage i is in
+                // registers.  The loads of S(i + 2) are not counted: into registers they may arrive in front of copies
+                // into LDS that are older, so with them in the count a copy of F(i + 1) could be left out of it.
+                lds::waitCopiesAndReads<Cfg::CopiesF>();
                 pinFrags(f[(N - 1u) & 1u]);
                 lds::barrier();
                 __builtin_amdgcn_sched_barrier(0);
