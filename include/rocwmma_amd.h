@@ -320,7 +320,9 @@ int rocwmma_amd_gemm_bias_act(int          dtype_in,
  * (256 x 256 tiles of v_mfma_scale_f32_16x16x128_f8f6f4 blocks when m and n are multiples of 256 and the
  * tiles occupy at least half of the compute units, else 128 x 128 or 128 x 64 tiles of 32x32x64 blocks with
  * partly filled edge tiles): the call then
- * enqueues a small kernel that re-orders the scales into the workspace, and the GEMM (two launches).  Everything else
+ * enqueues a small kernel that re-orders the scales into the workspace, and the GEMM (two launches); where that costs
+ * more than it gives (128 x 128 and 128 x 64 tiles in one round or few, scales and their leading dimensions 4-byte
+ * aligned), the GEMM alone, on the scales as they are.  What the workspace holds afterwards is undefined.  Everything else
  * runs one block per wave straight from global memory, except up to 32 rows of a row-major A against a
  * col-major B with k a multiple of 1024 (few tokens against a wide weight matrix), which run on the
  * weight-streaming kernel with or without a workspace (m * k <= 128 KiB; scale_a 4-byte aligned with

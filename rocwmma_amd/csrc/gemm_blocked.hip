@@ -26,19 +26,20 @@ namespace rocwmma_amd
 
     namespace
     {
-        template <typename InT>
+        // Raw: the scales in the caller's order (MxPacked)
+        template <typename InT, bool Raw>
         int launchMxMid(GemmArgs const& g, TileExtras const& ex, hipStream_t stream)
         {
             // 128 x 128 tiles of 32x32x64 blocks with block scales, the last row and column of tiles partly
             // filled: any m, n in multiples of 16
-            using Mid = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 2, 2, 2, 32, true, true>;
+            using Mid = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 2, 2, 2, 32, true, true, false, 0, false, Raw>;
             // at most one 128 x 128 tile per two compute units (few token rows against a wide weight matrix):
             // 128 x 64 tiles put twice as many workgroups to work
-            using Narrow = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 2, 3, 32, true, true>;
+            using Narrow = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 2, 3, 32, true, true, false, 0, false, Raw>;
             // One round of 128 x 64 tiles with at least 4 KiB of K per row: the tile on the ring of four 128-byte
             // stages (whole-line requests, three stages in flight), as for the unscaled types (NarrowLinesEdge
             // above): 128 x 14336 x 4096 31 -> 21 us on scales packed beforehand.
-            using NarrowLines = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 4, 1, 32, true, true, false, 128>;
+            using NarrowLines = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 4, 1, 32, true, true, false, 128, false, Raw>;
             if(gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u))
             {
                 const int rc = launchCfg<NarrowLines>(g, stream, ex);
@@ -69,12 +70,35 @@ namespace rocwmma_amd
         if(g.layoutC != ROCWMMA_AMD_ROW_MAJOR || g.m % 16u != 0u || g.n % 16u != 0u || g.k % 128u != 0u)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         TileExtras ex{};
-        ex.mx = MxPacked{packedA, packedB, (g.k / 128u + 1u) / 2u};
+        ex.mx = MxPacked{packedA, packedB, (g.k / 128u + 1u) / 2u, 0u, 0u};
         const bool large = gemmMxBlockedUsesLargeTile(g);
         if(dtypeIn == ROCWMMA_AMD_E4M3)
-            return large ? launchMx<float8_t>(g, ex, stream) : launchMxMid<float8_t>(g, ex, stream);
+            return large ? launchMx<float8_t>(g, ex, stream) : launchMxMid<float8_t, false>(g, ex, stream);
         if(dtypeIn == ROCWMMA_AMD_E5M2)
-            return large ? launchMx<bfloat8_t>(g, ex, stream) : launchMxMid<bfloat8_t>(g, ex, stream);
+            return large ? launchMx<bfloat8_t>(g, ex, stream) : launchMxMid<bfloat8_t, false>(g, ex, stream);
+        return ROCWMMA_AMD_UNSUPPORTED_TYPE;
+    }
+
+    int launchGemmMxBlockedRaw(int dtypeIn, GemmArgs const& g, MxScales const& s, hipStream_t stream)
+    {
+        const bool dwords = ((reinterpret_cast<uintptr_t>(s.a) | reinterpret_cast<uintptr_t>(s.b)) & 3u) == 0u && (s.lda | s.ldb) % 4u == 0u;
+        if(g.layoutC != ROCWMMA_AMD_ROW_MAJOR || g.m % 16u != 0u || g.n % 16u != 0u || g.k % 128u != 0u || g.k < 256u || !dwords
+           || gemmMxBlockedUsesLargeTile(g))
+            return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+        // What the re-ordering launch costs (4 to 6 us) against what the scattered scale loads cost in the main loop: on the
+        // ring of four always less (48 x 14336 x 4096 27.6 -> 21.8 us, 128 rows 29.3 -> 26.5), on the ring of two about
+        // 0.13 us per stage with a tile per compute unit (384 x 1056 x 1536 16.1 -> 12.6, but 128 x 1024 x 8192 52 -> 57) and
+        // 0.4 per stage and round with two (2000 x 3056 x 1408 25.1 -> 24.0, 512 x 14336 x 4096 57 -> 75).
+        const uint32_t units = computeUnits(), stages = g.k / 128u, tiles = ceilDiv(g.m, 128u) * ceilDiv(g.n, 128u);
+        if(!gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u)
+           && (tiles <= units ? stages > 30u : static_cast<uint64_t>(stages) * ceilDiv(tiles, 2u * units) > 12u))
+            return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+        TileExtras ex{};
+        ex.mx = MxPacked{s.a, s.b, (g.k / 128u + 1u) / 2u, s.lda, s.ldb};
+        if(dtypeIn == ROCWMMA_AMD_E4M3)
+            return launchMxMid<float8_t, true>(g, ex, stream);
+        if(dtypeIn == ROCWMMA_AMD_E5M2)
+            return launchMxMid<bfloat8_t, true>(g, ex, stream);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 

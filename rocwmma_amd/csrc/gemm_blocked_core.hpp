@@ -58,7 +58,8 @@ namespace rocwmma_amd
                   bool     Scaled_       = false, // fp8 operands with one E8M0 scale per 32 elements of K (MX)
                   bool     Fused_        = false, // epilogue adds a per-column bias and applies an activation
                   uint32_t StageKB_      = 0u, // bytes of K per stage (0: 64 in the ring of four, else 128)
-                  bool     ExtraB_       = false> // the ring of B is one stage deeper than the ring of A
+                  bool     ExtraB_       = false, // the ring of B is one stage deeper than the ring of A
+                  bool     RawScales_    = false> // Scaled, 32-wide blocks: the scales as the caller has them (see MxPacked)
         struct BlockedConfig
         {
             using InT   = InT_;
@@ -77,6 +78,7 @@ namespace rocwmma_amd
             // (two runs of 16 from the two halves of the stage, see rocwmma/internal/fragment_map.hpp),
             // so the fragments are read like two steps of a 16-bytes-per-lane operand.
             static constexpr bool     Scaled  = Scaled_;
+            static constexpr bool     RawScales = RawScales_;
             // D = act(alpha * A * B + beta * C + bias[column]): see FusedEpilogue
             static constexpr bool     Fused   = Fused_;
             static constexpr uint32_t WavesM  = WavesM_;
@@ -162,6 +164,7 @@ namespace rocwmma_amd
                                   && (Stages_ == 2u || (Stages_ == 4u && StageKB == 128u && Block == 32u))),
                           "block scales: fp8 on K-contiguous operands in the ring of two (16x16x128 on whole tiles, or 32x32x64), "
                           "or 32x32x64 in the ring of four 128-byte stages");
+            static_assert(!RawScales || (Scaled && Block == 32u && Edges), "scales in the caller's order: 32x32x64 on edge tiles");
             static_assert(Block == 32u || KPackBytes == 16u || ((PairReads || Scaled) && AKMajor && BKMajor && Stages_ == 2u),
                           "16-wide blocks: 16 bytes of K per lane (16-bit types, int8), or fp8 16x16x128 on K-contiguous "
                           "operands in the ring of two");
@@ -257,6 +260,9 @@ namespace rocwmma_amd
             const void* a;
             const void* b;
             uint32_t    pairs; // pairs of stages along K (the last one padded when the stage count is odd)
+            // RawScales: a and b are the caller's scales, one row of k / 32 bytes per row of A / column of B, these many
+            // bytes apart (4-byte aligned).  A lane then loads the eight bytes of its row for a pair of stages as they lie.
+            uint32_t    lda, ldb;
         };
 
         // What a Fused configuration's epilogue does beyond alpha * acc + beta * C.
@@ -271,6 +277,81 @@ namespace rocwmma_amd
         {
             MxPacked      mx;
             FusedEpilogue fused;
+        };
+
+        // Scales of a wave's 32-wide blocks along one dimension, a pair of stages (256 bytes of K, four instruction steps) at a
+        // time.  Packed: one dword per block and lane, byte = step.  Raw: the eight bytes of the lane's row, of which the
+        // lanes 0..31 take the even and the lanes 32..63 the odd ones; rows past the problem's take its last row's (they
+        // only meet zeros), and a last pair that is half a pair starts four bytes early.
+        template <typename Cfg, uint32_t Blocks>
+        struct PairScales
+        {
+            static constexpr bool Raw = Cfg::RawScales;
+            static_assert(Blocks == 1u || Blocks % 2u == 0u, "a wave's blocks: one, or whole groups of two");
+            uint32_t       now[Raw ? 2u * Blocks : Blocks] = {}, next[Raw ? 2u * Blocks : Blocks] = {};
+            const char*    from[Raw ? Blocks : 1u];
+            uint32_t       pairs, last, half; // last: Raw, byte the last whole pair of a row starts at
+            ROCWMMA_DEVICE ROCWMMA_INLINE PairScales(const void* scales, uint32_t ld, uint32_t pairs_, uint32_t row0, uint32_t rows, uint32_t k, uint32_t lane)
+                : pairs(pairs_)
+                , last(k / 32u - 8u)
+                , half(lane >> 5)
+            {
+                if constexpr(Raw)
+                {
+#pragma unroll
+                    for(uint32_t b = 0; b < Blocks; ++b)
+                    {
+                        const uint32_t row = row0 + b * 32u + (lane & 31u);
+                        from[b]            = static_cast<const char*>(scales) + static_cast<size_t>(row < rows ? row : rows - 1u) * ld;
+                    }
+                }
+                else // (dword of block b, pair p, lane l: (((b / 2) * pairs + p) * 64 + l) * 2 + b % 2)
+                    from[0] = static_cast<const char*>(scales) + ((static_cast<size_t>(row0 / 64u) * pairs * 64u + lane) * 2u + (row0 / 32u) % 2u) * 4u;
+            }
+            ROCWMMA_DEVICE ROCWMMA_INLINE void load(uint32_t(&to)[Raw ? 2u * Blocks : Blocks], uint32_t pair) const
+            {
+#pragma unroll
+                for(uint32_t b = 0; b < Blocks; ++b)
+                {
+                    if constexpr(Raw)
+                    {
+                        typedef uint32_t Words __attribute__((ext_vector_type(2), aligned(4)));
+                        const Words      v = *reinterpret_cast<const Words*>(from[b] + (8u * pair < last ? 8u * pair : last));
+                        to[2u * b]         = v[0];
+                        to[2u * b + 1u]    = v[1];
+                    }
+                    else
+                        to[b] = reinterpret_cast<const uint32_t*>(from[0])[(static_cast<size_t>(b / 2u) * pairs + pair) * 128u + b % 2u];
+                }
+            }
+            // The loaded pair `pair` takes over.
+            ROCWMMA_DEVICE ROCWMMA_INLINE void take(uint32_t(&loaded)[Raw ? 2u * Blocks : Blocks], uint32_t pair)
+            {
+                if constexpr(Raw)
+                {
+                    const bool halfPair = 8u * pair > last; // (wave uniform)
+#pragma unroll
+                    for(uint32_t b = 0; b < Blocks; ++b)
+                    {
+                        now[2u * b]      = (halfPair ? loaded[2u * b + 1u] : loaded[2u * b]) >> (8u * half);
+                        now[2u * b + 1u] = loaded[2u * b + 1u] >> (8u * half);
+                    }
+                }
+                else
+                {
+#pragma unroll
+                    for(uint32_t b = 0; b < Blocks; ++b)
+                        now[b] = loaded[b];
+                }
+            }
+            // scale of block b at instruction step `step` (0..3) of the pair, in the lowest byte
+            ROCWMMA_DEVICE ROCWMMA_INLINE uint32_t at(uint32_t b, uint32_t step) const
+            {
+                if constexpr(Raw)
+                    return (step < 2u ? now[2u * b] : now[2u * b + 1u]) >> (16u * (step % 2u));
+                else
+                    return now[b] >> (8u * step);
+            }
         };
 
         // ---- stream-K support ------------------------------------------------------------------
@@ -832,32 +913,14 @@ namespace rocwmma_amd
                 // instruction steps), one dword per block of 32 rows, byte = step; the step's byte is shifted
                 // down at run time.  The next pair's are loaded behind the barrier of a pair's first stage.
                 static_assert(!Cfg::Scaled || Cfg::KSteps == 2u, "packed scales: two instruction steps per stage");
-                uint32_t        sA[Cfg::BlocksM] = {}, sB[Cfg::BlocksN] = {}, sAnext[Cfg::BlocksM] = {}, sBnext[Cfg::BlocksN] = {};
-                const uint32_t* mxA = nullptr; // dword of (this wave's first block, pair of stages 0, this lane)
-                const uint32_t* mxB = nullptr;
-                // (dword of block b of an operand, pair p, lane l: (((b / 2) * pairs + p) * 64 + l) * 2 + b % 2)
-                auto scalePtr = [&](const void* base, uint32_t firstBlock) {
-                    return static_cast<const uint32_t*>(base) + (static_cast<size_t>(firstBlock / 2u) * mx.pairs * 64u + lane) * 2u + firstBlock % 2u;
-                };
-                auto loadScales32 = [&](uint32_t(&a_)[Cfg::BlocksM], uint32_t(&b_)[Cfg::BlocksN], uint32_t pair) {
-                    // (a wave's blocks start at an even block or are a single one: block i sits i % 2 dwords and
-                    // i / 2 groups on)
-#pragma unroll
-                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
-                        a_[bi] = mxA[(static_cast<size_t>(bi / 2u) * mx.pairs + pair) * 128u + bi % 2u];
-#pragma unroll
-                    for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                        b_[bj] = mxB[(static_cast<size_t>(bj / 2u) * mx.pairs + pair) * 128u + bj % 2u];
-                };
+                PairScales<Cfg, Cfg::Scaled ? Cfg::BlocksM : 1u> sA(mx.a, mx.lda, mx.pairs, row0 + waveM * Cfg::WaveM, m, k, lane);
+                PairScales<Cfg, Cfg::Scaled ? Cfg::BlocksN : 1u> sB(mx.b, mx.ldb, mx.pairs, col0 + waveN * Cfg::WaveN, n, k, lane);
                 if constexpr(Cfg::Scaled)
                 {
-                    static_assert(Cfg::BlocksM == 1u || Cfg::BlocksM % 2u == 0u, "a wave's row blocks: one, or whole groups of two");
-                    static_assert(Cfg::BlocksN == 1u || Cfg::BlocksN % 2u == 0u, "a wave's column blocks: one, or whole groups of two");
-                    mxA = scalePtr(mx.a, (row0 + waveM * Cfg::WaveM) / 32u);
-                    mxB = scalePtr(mx.b, (col0 + waveN * Cfg::WaveN) / 32u);
                     // (in front of the first copies and kept there: the wait for stage 0 then covers these loads,
                     // and the loop is entered with none of them in flight)
-                    loadScales32(sA, sB, 0u);
+                    sA.load(sA.next, 0u);
+                    sB.load(sB.next, 0u);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 constexpr uint32_t SB = Cfg::StagesB;
@@ -867,6 +930,12 @@ namespace rocwmma_amd
                     if(st < S)
                         issueA(st, st + 1u < stages);
                     issueB(st, st + 1u < stages);
+                }
+                if constexpr(Cfg::Scaled)
+                {
+                    __builtin_amdgcn_sched_barrier(0);
+                    sA.take(sA.next, 0u);
+                    sB.take(sB.next, 0u);
                 }
                 // (copies of later stages that may be in flight when a stage must have landed; the waves that issue
                 // none do not wait)
@@ -881,7 +950,7 @@ namespace rocwmma_amd
 #if ROCWMMA_ARCH_GFX950 // (the instruction table exists in the device pass only)
                         using Op  = detail::MfmaScaled<detail::TypeInfo<InT>::cls, detail::TypeInfo<InT>::cls, 32u>;
                         using Acc = typename Op::Acc;
-                        const uint32_t shift = 8u * ((i % 2u) * N + ks); // the step's byte within the pair of stages
+                        const uint32_t step = (i % 2u) * N + ks; // within the pair of stages
 #pragma unroll
                         for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
 #pragma unroll
@@ -889,7 +958,7 @@ namespace rocwmma_amd
                             {
                                 Acc& v = *reinterpret_cast<Acc*>(acc[bi][bj].x);
                                 // (the accumulator is kept transposed: the instruction's first multiplicand is B)
-                                v = Op::template exec<0, 0>(fr.b[bj].x, fr.a[bi].x, v, sB[bj] >> shift, sA[bi] >> shift);
+                                v = Op::template exec<0, 0>(fr.b[bj].x, fr.a[bi].x, v, sB.at(bj, step), sA.at(bi, step));
                             }
 #else
                         (void)fr, (void)i, (void)ks;
@@ -929,7 +998,10 @@ namespace rocwmma_amd
                     if constexpr(Cfg::Scaled)
                     {
                         if(i % 2u == 0u)
-                            loadScales32(sAnext, sBnext, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
+                        {
+                            sA.load(sA.next, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
+                            sB.load(sB.next, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
+                        }
                     }
                     readFragsOf(f[0], nextSlot, nextSlotB, 0u);
                     slot  = nextSlot;
@@ -939,12 +1011,8 @@ namespace rocwmma_amd
                     {
                         if(i % 2u == 1u)
                         {
-#pragma unroll
-                            for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
-                                sA[bi] = sAnext[bi];
-#pragma unroll
-                            for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                                sB[bj] = sBnext[bj];
+                            sA.take(sA.next, i / 2u + 1u);
+                            sB.take(sB.next, i / 2u + 1u);
                         }
                     }
                     scheduleInterleaved<Cfg::MfmasPerStep / 2u, Cfg::ReadsPerStep, 0u>();
@@ -964,29 +1032,13 @@ namespace rocwmma_amd
                 // over.  Every trip issues its stages (past the end of K the last stage again, into a slot nobody
                 // reads), so the body and its counts are uniform.
                 static_assert(S == 4u && Cfg::StageKB == 128u && Cfg::Block == 32u && Part == TilePart::Whole, "scaled ring of four: 128-byte stages of 32-wide blocks");
-                uint32_t        sA[Cfg::BlocksM] = {}, sB[Cfg::BlocksN] = {}, sAnext[Cfg::BlocksM] = {}, sBnext[Cfg::BlocksN] = {};
-                // (dword of block b of an operand, pair p, lane l: (((b / 2) * pairs + p) * 64 + l) * 2 + b % 2)
-                const uint32_t* mxA = static_cast<const uint32_t*>(mx.a)
-                                      + (static_cast<size_t>((row0 + waveM * Cfg::WaveM) / 64u) * mx.pairs * 64u + lane) * 2u
-                                      + ((row0 + waveM * Cfg::WaveM) / 32u) % 2u;
-                const uint32_t* mxB = static_cast<const uint32_t*>(mx.b)
-                                      + (static_cast<size_t>((col0 + waveN * Cfg::WaveN) / 64u) * mx.pairs * 64u + lane) * 2u
-                                      + ((col0 + waveN * Cfg::WaveN) / 32u) % 2u;
-                static_assert(Cfg::BlocksM == 1u || Cfg::BlocksM % 2u == 0u, "a wave's row blocks: one, or whole groups of two");
-                static_assert(Cfg::BlocksN == 1u || Cfg::BlocksN % 2u == 0u, "a wave's column blocks: one, or whole groups of two");
-                auto loadScales32 = [&](uint32_t(&a_)[Cfg::BlocksM], uint32_t(&b_)[Cfg::BlocksN], uint32_t pair) {
-#pragma unroll
-                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
-                        a_[bi] = mxA[(static_cast<size_t>(bi / 2u) * mx.pairs + pair) * 128u + bi % 2u];
-#pragma unroll
-                    for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                        b_[bj] = mxB[(static_cast<size_t>(bj / 2u) * mx.pairs + pair) * 128u + bj % 2u];
-                };
+                PairScales<Cfg, Cfg::BlocksM> sA(mx.a, mx.lda, mx.pairs, row0 + waveM * Cfg::WaveM, m, k, lane);
+                PairScales<Cfg, Cfg::BlocksN> sB(mx.b, mx.ldb, mx.pairs, col0 + waveN * Cfg::WaveN, n, k, lane);
                 auto multiplyScaled = [&](Frags const& fr, auto stepC) {
 #if ROCWMMA_ARCH_GFX950 // (the instruction table exists in the device pass only)
                     using Op  = detail::MfmaScaled<detail::TypeInfo<InT>::cls, detail::TypeInfo<InT>::cls, 32u>;
                     using Acc = typename Op::Acc;
-                    constexpr uint32_t shift = 8u * decltype(stepC)::value; // the step's byte within the pair of stages
+                    constexpr uint32_t step = decltype(stepC)::value; // within the pair of stages
 #pragma unroll
                     for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
 #pragma unroll
@@ -994,18 +1046,22 @@ namespace rocwmma_amd
                         {
                             Acc& v = *reinterpret_cast<Acc*>(acc[bi][bj].x);
                             // (the accumulator is kept transposed: the instruction's first multiplicand is B)
-                            v = Op::template exec<0, 0>(fr.b[bj].x, fr.a[bi].x, v, sB[bj] >> shift, sA[bi] >> shift);
+                            v = Op::template exec<0, 0>(fr.b[bj].x, fr.a[bi].x, v, sB.at(bj, step), sA.at(bi, step));
                         }
 #else
                     (void)fr, (void)stepC;
 #endif
                 };
                 // (in front of the first copies and kept there: the wait for stage 0 covers them)
-                loadScales32(sA, sB, 0u);
+                sA.load(sA.next, 0u);
+                sB.load(sB.next, 0u);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for(uint32_t st = 0; st < S - 1u; ++st)
                     issueStage(st, st + 1u < stages);
+                __builtin_amdgcn_sched_barrier(0);
+                sA.take(sA.next, 0u);
+                sB.take(sB.next, 0u);
                 lds::waitCopiesAndReads<(S - 2u) * Cfg::Copies>();
                 lds::barrier();
                 Frags f0, f1;
@@ -1037,17 +1093,14 @@ namespace rocwmma_amd
                 };
                 for(uint32_t i = 0; i < stages; i += 2u)
                 {
-                    loadScales32(sAnext, sBnext, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
+                    sA.load(sA.next, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
+                    sB.load(sB.next, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
                     __builtin_amdgcn_sched_barrier(0);
                     stage(i, std::integral_constant<uint32_t, 0u>{});
                     if(i + 1u < stages)
                         stage(i + 1u, std::integral_constant<uint32_t, 1u>{});
-#pragma unroll
-                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
-                        sA[bi] = sAnext[bi];
-#pragma unroll
-                    for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                        sB[bj] = sBnext[bj];
+                    sA.take(sA.next, i / 2u + 1u);
+                    sB.take(sB.next, i / 2u + 1u);
                 }
                 lds::waitCopiesAndReads<0u>(); // the surplus copies still target this workgroup's LDS
                 lds::barrier();
