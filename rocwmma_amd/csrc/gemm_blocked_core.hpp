@@ -158,6 +158,11 @@ namespace rocwmma_amd
                                             && BlocksM * (BlocksN / GroupBlocks) >= 2u
                                             && 2u * Block * GroupBlocks * Block * sizeof(OutT) * Waves <= LdsBytes;
 
+            // C of the small tiles (at most 32 registers of it) is loaded in front of the main loop: behind it, the loads' latency
+            // is a large part of a short problem (per call in a captured graph: 256^3 f16 4.0 -> 3.55 us, 512 x 1024 x 1024 e4m3
+            // 5.4 -> 4.8, 640 x 1200 x 1360 bf16 10.0 -> 9.5).
+            static constexpr bool PrefetchC = !StagedC && !Scaled && WaveM * WaveN * sizeof(OutT) <= 64u * 128u;
+
             static_assert(Block == 32u || Block == 16u, "MFMA blocks are 32 or 16 wide");
             static_assert(!Scaled
                               || (KPackBytes == 32u && AKMajor && BKMajor && (Block == 32u || !Edges_)
@@ -728,6 +733,30 @@ namespace rocwmma_amd
                     for(uint32_t j = 0; j < Cfg::BlocksN; ++j)
                         mma_sync(acc[i][j], f.a[i], f.b[j], acc[i][j]);
             };
+
+            typename Cfg::FragC early[Cfg::PrefetchC ? Cfg::BlocksM : 1u][Cfg::PrefetchC ? Cfg::BlocksN : 1u];
+            if constexpr(Cfg::PrefetchC)
+            {
+                if(beta != static_cast<CompT>(0))
+                {
+                    typedef uint32_t Words __attribute__((ext_vector_type(sizeof(OutT))));
+                    const uint32_t   r0 = row0 + waveM * Cfg::WaveM + (lane & (Cfg::Block - 1u)), c0 = col0 + waveN * Cfg::WaveN + 4u * (lane / Cfg::Block);
+#pragma unroll
+                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                            for(uint32_t r = 0; r < Cfg::FragC::num_elements / 4u; ++r)
+                            {
+                                const uint32_t row = r0 + bi * Cfg::Block, col = c0 + bj * Cfg::Block + 8u * r;
+                                Words          v   = {};
+                                if(!Cfg::Edges || (row < m && col < n))
+                                    v = *reinterpret_cast<const Words*>(c + static_cast<size_t>(row) * ldc + col);
+                                __builtin_memcpy(early[bi][bj].x + 4u * r, &v, sizeof(v));
+                            }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
 
             constexpr uint32_t S      = Cfg::Stages;
             // `stages` stages of K from stage0 on: >= S - 1 of them (checked by the host)
@@ -1514,6 +1543,26 @@ namespace rocwmma_amd
                         for(uint32_t bj = 0; bj < GB; ++bj)
                             storeBlock(bi, bj0 + bj, acc[bi][bj0 + bj]);
                         __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+                else if constexpr(Cfg::PrefetchC)
+                {
+#pragma unroll
+                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
+                    {
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+                        {
+                            auto&             io = early[bi][bj];
+                            const BiasOfBlock bv = biasOf(bj);
+#pragma unroll
+                            for(uint32_t e = 0; e < io.num_elements; ++e)
+                                io.x[e] = static_cast<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
+                            if constexpr(!PairIO)
+                                storeBlock(bi, bj, io);
+                            else if(bj % 2u == 1u)
+                                storePair(bi, bj - 1u, early[bi][bj - 1u], io);
+                        }
                     }
                 }
                 else
