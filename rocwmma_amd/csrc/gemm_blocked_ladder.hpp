@@ -20,10 +20,9 @@ namespace rocwmma_amd
         {
             float start, alone, shared, perTile;
         };
-        inline float rungTime(RungCost const& c, uint32_t tiles, float kKB, float outBytes)
+        inline float rungTime(RungCost const& c, uint32_t tiles, uint32_t units, float kKB, float outBytes)
         {
-            const uint32_t units = computeUnits();
-            const float    load  = static_cast<float>((tiles + units - 1u) / units);
+            const float load = static_cast<float>((tiles + units - 1u) / units);
             return c.start + (tiles <= units ? c.alone * kKB : load * (c.perTile * outBytes + c.shared * kKB));
         }
         template <typename Cfg>
@@ -92,7 +91,8 @@ namespace rocwmma_amd
             constexpr RungCost LinesCost = AK && BK ? RungCost{5.5f, 1.77f, 2.56f, 0.52f} : RungCost{5.1f, 2.75f, 4.05f, 0.48f};
             constexpr RungCost TinyCost  = RungCost{5.1f, Byte ? 1.45f : 1.95f, Byte ? 1.6f : 1.75f, 0.14f};
 
-            const float kKB = static_cast<float>(g.k) * (sizeof(InT) * 1e-3f), outBytes = sizeof(OutT);
+            const uint32_t units = computeUnits(); // (once: it asks the runtime for the current device)
+            const float    kKB = static_cast<float>(g.k) * (sizeof(InT) * 1e-3f), outBytes = sizeof(OutT);
             enum Rung
             {
                 kBig,
@@ -103,16 +103,16 @@ namespace rocwmma_amd
                 kTiny
             };
             Rung  best = kBig;
-            float time = rungTime(BigCost, tilesOf<Big>(g), kKB, outBytes);
+            float time = rungTime(BigCost, tilesOf<Big>(g), units, kKB, outBytes);
             if(aligned)
             {
                 // a last round that would be at most half full runs as half tiles (launchSplitTail)
-                const uint32_t units = computeUnits(), tiles = tilesOf<Big>(g), rest = tiles % units;
+                const uint32_t tiles = tilesOf<Big>(g), rest = tiles % units;
                 if(tiles > units && rest != 0u && 2u * rest <= units)
                     time -= 0.4f * (BigCost.perTile * outBytes + BigCost.shared * kKB);
             }
             auto consider = [&](Rung r, RungCost const& c, uint32_t tiles) {
-                const float t = rungTime(c, tiles, kKB, outBytes);
+                const float t = rungTime(c, tiles, units, kKB, outBytes);
                 if(t < time)
                 {
                     time = t;
