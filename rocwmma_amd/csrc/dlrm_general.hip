@@ -8,7 +8,8 @@
 //
 //   * forward: tile (I, J), J <= I, of Z = F F^T; both operands are rows of F with K contiguous.  The strict lower
 //     triangle leaves through a 32 x 32 LDS block per wave as row pieces, which are contiguous in the packed
-//     output.  No m x m scratch in global memory.
+//     output.  No m x m scratch in global memory.  (float32, and float16 where 128 feature rows span 2 GiB; other float16
+//     samples: dlrm_general_fwd.hip.)
 //   * backward: tile (I, N) of grad = S F, S = the symmetric matrix with zero diagonal whose strict lower triangle
 //     is the packed upstream gradient, never materialised: where the contraction index lies below the tile's rows
 //     the packed triangle holds S row by row, where it lies above them it holds the transpose, and only the
@@ -26,6 +27,8 @@ using namespace rocwmma;
 
 namespace rocwmma_amd
 {
+    int launchDlrmFwdTilesF16(const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream);
+
     namespace
     {
         typedef uint32_t u32x4_t __attribute__((ext_vector_type(4), may_alias));
@@ -894,8 +897,13 @@ namespace rocwmma_amd
         if(grid == 0u)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         if(dtype == ROCWMMA_AMD_F16)
+        {
+            const int rc = launchDlrmFwdTilesF16(input, output, m, k, batch, stream);
+            if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE) // (feature rows of more than 16 MiB)
+                return rc;
             hipLaunchKernelGGL(dlrmFwdStagedKernel<float16_t>, dim3(grid), dim3(256), 0, stream, static_cast<const float16_t*>(input),
                                static_cast<float16_t*>(output), m, k, batch, tiles);
+        }
         else
             hipLaunchKernelGGL(dlrmFwdStagedKernel<float>, dim3(grid), dim3(256), 0, stream, static_cast<const float*>(input),
                                static_cast<float*>(output), m, k, batch, tiles);

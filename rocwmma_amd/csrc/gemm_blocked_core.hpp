@@ -485,7 +485,11 @@ namespace rocwmma_amd
         // stage.
         // One macro tile (or, with Part != Whole, a part of its K range): tile (tm, tn) of the tile grid,
         // `stages` pipeline stages of K starting at stage `stage0`.
-        template <typename Cfg, TilePart Part = TilePart::Whole>
+        // With an Emit other than Epilogue the results go to emit(acc, wave row, wave column) instead, once the LDS is free.
+        struct Epilogue
+        {
+        };
+        template <typename Cfg, TilePart Part = TilePart::Whole, typename Emit = Epilogue>
         ROCWMMA_DEVICE ROCWMMA_INLINE void gemmTile(uint32_t                   tm,
                                                     uint32_t                   tn,
                                                     uint32_t                   stage0,
@@ -504,7 +508,8 @@ namespace rocwmma_amd
                                                     typename Cfg::CompT        alpha,
                                                     typename Cfg::CompT        beta,
                                                     StreamKPart const&         sk,
-                                                    TileExtras const&          ex = TileExtras{})
+                                                    TileExtras const&          ex = TileExtras{},
+                                                    Emit const&                emit = Emit{})
         {
             const MxPacked& mx = ex.mx;
             using InT   = typename Cfg::InT;
@@ -1288,6 +1293,15 @@ namespace rocwmma_amd
                     return;
             }
 
+            if constexpr(!std::is_same<Emit, Epilogue>::value)
+            {
+                emit(acc, row0 + waveM * Cfg::WaveM, col0 + waveN * Cfg::WaveN);
+                return;
+            }
+            else
+            {
+                (void)emit;
+            }
             // Epilogue: D = alpha * acc + beta * C, one row of blocks (BlocksN blocks) at a time,
             // 16-byte accesses per lane.  Every block of a group has registers of its own, so
             // the stores of a group issue back to back (a store whose data registers are about

@@ -1,4 +1,4 @@
-"""DLRM samples that do not fit the LDS, float16 backward in tiles of 128 or 256 rows and columns: feature counts and widths at
+"""DLRM samples that do not fit the LDS, float16 forward in tiles of 128 x 128, backward in tiles of 128 or 256 rows and columns: feature counts and widths at
 the edges of its tiles, stages and 64-row strips, the last rows of the packed triangle at the end of the tensor, and both
 tile sizes, against the CPU oracle; a sample of NaNs between the others must not reach them.
 Tolerance as in tests/test_gpu_dlrm.py: 10 eps of float16."""
@@ -19,7 +19,7 @@ SHAPES = [(3, 1, 81920), (3, 2, 65544), (3, 3, 40960), (2, 7, 20480), (2, 64, 20
 
 
 @pytest.mark.parametrize("batch,m,k", SHAPES)
-def test_backward_tiles(batch, m, k):
+def test_tiles(batch, m, k):
     import torch
 
     width = k + m * (m - 1) // 2
@@ -32,11 +32,15 @@ def test_backward_tiles(batch, m, k):
         pu[poisoned] = 0x7E00
     grad, mlp = (to_device(np.full(n, 0x7E00, dtype=np.uint16)) for n in (batch * m * k, batch * k))
     rw.dlrm_bwd(to_device(pf.ravel()), to_device(pu.ravel()), grad, mlp, m, k, batch, rw.F16)
+    out = to_device(np.full(batch * width, 0x7E00, dtype=np.uint16))
+    rw.dlrm_fwd(to_device(pf.ravel()), out, m, k, batch, rw.F16)
     torch.cuda.synchronize()
     # the oracle is slow at the full batches: the first, the last and the poisoned sample's neighbours
     keep = sorted({0, 1, batch - 1, max(poisoned - 1, 0), min(poisoned + 1, batch - 1)} & set(range(batch)) - {poisoned})
     wgrad, wmlp = orc.dlrm_bwd(np.ascontiguousarray(feat[keep]), np.ascontiguousarray(up[keep]), m, k, len(keep), orc.F16)
-    got = grad.cpu().numpy().view(np.uint16).reshape(batch, m * k)[keep]
-    err, inf, nan = orc.compare_equal(orc.F16, np.ascontiguousarray(got).ravel(), orc.F16, np.ascontiguousarray(wgrad).ravel())
-    assert not inf and not nan and err <= 10 * 2.0 ** -10, (err, inf, nan)
+    want = orc.dlrm_fwd(np.ascontiguousarray(feat[keep]), m, k, len(keep), orc.F16)
+    for dev, ref in ((grad, wgrad), (out, want)):
+        got = np.ascontiguousarray(dev.cpu().numpy().view(np.uint16).reshape(batch, -1)[keep]).ravel()
+        err, inf, nan = orc.compare_equal(orc.F16, got, orc.F16, np.ascontiguousarray(ref).ravel())
+        assert not inf and not nan and err <= 10 * 2.0 ** -10, (err, inf, nan)
     assert np.array_equal(mlp.cpu().numpy().view(np.uint16).reshape(batch, k)[keep].ravel(), np.ascontiguousarray(wmlp).ravel())
