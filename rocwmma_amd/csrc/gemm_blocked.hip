@@ -37,8 +37,8 @@ namespace rocwmma_amd
             // 128 x 64 tiles put twice as many workgroups to work
             using Narrow = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 2, 3, 32, true, true, false, 0, false, Raw>;
             // One round of 128 x 64 tiles with at least 4 KiB of K per row: the tile on the ring of four 128-byte
-            // stages (whole-line requests, three stages in flight), as for the unscaled types (NarrowLinesEdge
-            // above): 128 x 14336 x 4096 31 -> 21 us on scales packed beforehand.
+            // stages (whole-line requests, three stages in flight), as for the unscaled types (the ladder's
+            // NarrowLines): 128 x 14336 x 4096 31 -> 21 us on scales packed beforehand.
             using NarrowLines = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 4, 1, 32, true, true, false, 128, false, Raw>;
             if(gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u))
             {

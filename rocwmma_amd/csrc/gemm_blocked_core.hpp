@@ -1008,7 +1008,12 @@ namespace rocwmma_amd
                 uint32_t slot = 0u, slotB = 0u; // of stage i
                 for(uint32_t i = 0; i < stages; ++i)
                 {
-                    const uint32_t nextSlot = slot + 1u == S ? 0u : slot + 1u, nextSlotB = slotB + 1u == SB ? 0u : slotB + 1u;
+                    if constexpr(S == 2u)
+                        slot = i % 2u;
+                    if constexpr(SB == S)
+                        slotB = slot;
+                    const uint32_t nextSlot  = S == 2u ? (i + 1u) % 2u : (slot + 1u == S ? 0u : slot + 1u);
+                    const uint32_t nextSlotB = SB == S ? nextSlot : (slotB + 1u == SB ? 0u : slotB + 1u);
 #pragma unroll
                     for(uint32_t ks = 0; ks + 1u < N; ++ks)
                     {

@@ -38,7 +38,8 @@ namespace rocwmma_amd
         // a flop costs (a compute unit takes at most 64 bytes a clock from its L2, so 128 x 128 tiles are bound by their
         // copies, 256 x 256 tiles are not) and how many stages are in flight while a tile waits for memory:
         //   Big    256 x 256, 8 waves, A ring of two stages, B ring of three (all 160 KiB of LDS).  The third B stage keeps
-        //          copies in flight at the barrier: 512 x 14336 x 4096 f16 99 -> 90 us, int8 4096 x 14336 x 4096 1.5 %.
+        //          copies in flight at the barrier: 512 x 14336 x 4096 f16 99 -> 90 us, int8 4096 x 14336 x 4096 1.5 %.  Whole tiles with
+        //          a dim-major operand keep two (8192^3 bf16 0.5-0.7 % faster in both such pairs with one).
         //   Wide   256 x 128, 8 waves, ring of three (144 KiB): 512 x 14336 x 4096 f16 77 -> 63 us against 128 x 128 tiles on
         //          the ring of two, int8 43 -> 34; on a ring of two of its own it was 82.
         //   Mid    128 x 128, 4 waves, two workgroups per unit with 80 KiB each (A ring of two, B ring of three):
@@ -60,9 +61,9 @@ namespace rocwmma_amd
             // blocks of 16 (or half as many of 32 where the 16-wide instruction does not fit the ring)
             static constexpr uint32_t E2 = Edge16 ? 16u : 32u, D2 = Edge16 ? 1u : 2u;
             static constexpr uint32_t E3 = Fp8 ? 32u : 16u, D3 = Fp8 ? 2u : 1u;
-            using Aligned = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / D2, 8 / D2, 2, 2, E2, false, false, Fused, 0, true>;
+            using Aligned = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / D2, 8 / D2, 2, 2, E2, false, false, Fused, 0, AK && BK>;
             // same rows and pipeline with half the columns, for the tiles of a last round that would be at most half full
-            using AlignedHalf = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / D2, 4 / D2, 2, 2, E2, false, false, Fused, 0, true>;
+            using AlignedHalf = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / D2, 4 / D2, 2, 2, E2, false, false, Fused, 0, AK && BK>;
             using Big    = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / D2, 8 / D2, 2, 2, E2, true, false, Fused, 0, true>;
             using Wide   = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / D3, 4 / D3, 3, 2, E3, true, false, Fused>;
             using Mid    = BlockedConfig<InT, OutT, CompT, AK, BK, 2, 2, 4 / D2, 4 / D2, 2, 2, E2, true, false, Fused, 0, true>;
