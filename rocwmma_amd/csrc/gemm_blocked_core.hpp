@@ -161,7 +161,10 @@ namespace rocwmma_amd
             // C of the small tiles (at most 32 registers of it) is loaded in front of the main loop: behind it, the loads' latency
             // is a large part of a short problem (per call in a captured graph: 256^3 f16 4.0 -> 3.55 us, 512 x 1024 x 1024 e4m3
             // 5.4 -> 4.8, 640 x 1200 x 1360 bf16 10.0 -> 9.5).
-            static constexpr bool PrefetchC = !StagedC && !Scaled && WaveM * WaveN * sizeof(OutT) <= 64u * 128u;
+            // (int8 results count as registers, not as bytes: the early elements are held one to a register, so the 64 x 128 wave
+            // tiles of the 256 x 256 rung spilled more than a hundred registers: 3072^3 int8 -> int8 38 -> 50 us.)
+            static constexpr bool PrefetchC
+                = !StagedC && !Scaled && WaveM * WaveN * sizeof(OutT) <= 64u * 128u && WaveM * WaveN <= 64u * 64u;
 
             static_assert(Block == 32u || Block == 16u, "MFMA blocks are 32 or 16 wide");
             static_assert(!Scaled
