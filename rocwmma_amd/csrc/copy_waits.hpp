@@ -1,0 +1,23 @@
+// How many vector-memory operations a wave may have in flight while it waits for direct copies into LDS.  Plain C++, so
+// that the counts can be checked on the host.
+//
+// Copies into LDS complete in the order they were issued among themselves, and only among themselves: loads into
+// registers and stores may retire in front of older copies (loads have been seen to, with a cold cache).  A wait that
+// counted one of those as in flight would pass with a copy outstanding as soon as it had retired, so only younger copies
+// count.  Anything else that is still in flight makes the wait longer, never too short.
+#ifndef ROCWMMA_AMD_CSRC_COPY_WAITS_HPP
+#define ROCWMMA_AMD_CSRC_COPY_WAITS_HPP
+
+#include <cstdint>
+
+namespace rocwmma_amd
+{
+    // C staged through two LDS buffers: `groups` groups of `copies` copies each, group g + 2 issued when group g has been
+    // read and its results have been stored.  In flight when group `group` must have landed: the next group's copies.
+    constexpr uint32_t stagedCInFlight(uint32_t group, uint32_t groups, uint32_t copies)
+    {
+        return group + 1u < groups ? copies : 0u;
+    }
+} // namespace rocwmma_amd
+
+#endif // ROCWMMA_AMD_CSRC_COPY_WAITS_HPP

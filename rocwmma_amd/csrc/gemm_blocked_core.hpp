@@ -32,6 +32,7 @@
 #define ROCWMMA_AMD_CSRC_GEMM_BLOCKED_CORE_HPP
 
 #include "common.hpp"
+#include "copy_waits.hpp"
 #include <rocwmma/rocwmma_lds.hpp>
 
 using namespace rocwmma;
@@ -1478,7 +1479,6 @@ namespace rocwmma_amd
                     constexpr uint32_t RowChunks   = RowBytes / 16u;
                     constexpr uint32_t RowsPerCopy = 1024u / RowBytes;
                     constexpr uint32_t CopiesC     = GroupBytes / 1024u;
-                    constexpr uint32_t StoresD     = GB * Runs; // 16-byte stores per group
                     constexpr uint32_t GroupsPerRow = Cfg::BlocksN / GB;
                     constexpr uint32_t NG          = Cfg::BlocksM * GroupsPerRow;
                     static_assert((RowBytes == 256u || RowBytes == 512u) && 2u * GroupBytes * Cfg::Waves <= Cfg::LdsBytes
@@ -1494,16 +1494,15 @@ namespace rocwmma_amd
 #pragma unroll
                         for(uint32_t i = 0; i < CopiesC; ++i)
                         {
-                            const uint32_t r   = RowsPerCopy * i + cpRow;
-                            const uint32_t col = bj0 * Cfg::Block * static_cast<uint32_t>(sizeof(OutT)) + ((chunk ^ (r & 15u)) << 4);
+                            const uint32_t r = RowsPerCopy * i + cpRow;
                             const char*    src;
                             if constexpr(!Cfg::Edges)
-                                src = cWave + (bi * Cfg::Block + r) * ldcB + col;
+                                src = cWave + (bi * Cfg::Block + r) * ldcB + bj0 * Cfg::Block * sizeof(OutT) + ((chunk ^ (r & 15u)) << 4);
                             else
                             {
                                 // (rows and columns past the problem's fetch some element of C, used by nobody)
                                 const uint32_t row  = wRow + bi * Cfg::Block + r;
-                                const uint32_t colB = wCol * static_cast<uint32_t>(sizeof(OutT)) + col;
+                                const uint32_t colB = (wCol + bj0 * Cfg::Block) * static_cast<uint32_t>(sizeof(OutT)) + ((chunk ^ (r & 15u)) << 4);
                                 src = reinterpret_cast<const char*>(c) + static_cast<size_t>(row < m ? row : m - 1u) * ldcB
                                       + (colB < n * static_cast<uint32_t>(sizeof(OutT)) ? colB : 0u);
                             }
@@ -1518,21 +1517,11 @@ namespace rocwmma_amd
                     for(uint32_t gi = 0; gi < NG; ++gi)
                     {
                         const uint32_t bi = gi / GroupsPerRow, bj0 = (gi % GroupsPerRow) * GB;
-                        // vector-memory operations younger than this group's copies: the next
-                        // group's copies and the stores of the two previous groups (which edge tiles
-                        // may not issue: there only the copies count)
-                        if(Cfg::Edges && gi + 1u < NG)
+                        // (the stores of D do not count, see copy_waits.hpp)
+                        if(stagedCInFlight(gi, NG, CopiesC) != 0u)
                             lds::waitCopiesAndReads<CopiesC>();
-                        else if(Cfg::Edges)
-                            lds::waitCopiesAndReads<0u>();
-                        else if(gi == 0u)
-                            lds::waitCopiesAndReads<CopiesC>();
-                        else if(gi == 1u)
-                            lds::waitCopiesAndReads<(NG > 2u ? CopiesC : 0u) + StoresD>();
-                        else if(gi + 1u < NG)
-                            lds::waitCopiesAndReads<CopiesC + 2u * StoresD>();
                         else
-                            lds::waitCopiesAndReads<2u * StoresD>();
+                            lds::waitCopiesAndReads<0u>();
                         asm volatile("" ::: "memory");
                         typename Cfg::FragC io[GB];
 #pragma unroll
@@ -1545,12 +1534,6 @@ namespace rocwmma_amd
                                 detail::copyBytes<16u>(io[bj].x + 4u * r,
                                                        myLds + (gi % 2u) * GroupBytes + rdBase + ((g ^ (rdRow & 15u)) << 4));
                             }
-                        if(gi + 2u < NG)
-                        {
-                            lds::waitReads(); // the buffer is overwritten next
-                            asm volatile("" ::: "memory");
-                            copyGroup(gi + 2u);
-                        }
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
                         {
@@ -1565,6 +1548,13 @@ namespace rocwmma_amd
                         for(uint32_t bj = 0; bj < GB; ++bj)
                             storeBlock(bi, bj0 + bj, acc[bi][bj0 + bj]);
                         __builtin_amdgcn_sched_barrier(0);
+                        // behind the stores: the next wait then leaves these copies in flight and not the stores
+                        if(gi + 2u < NG)
+                        {
+                            lds::waitReads(); // the buffer is overwritten next
+                            asm volatile("" ::: "memory");
+                            copyGroup(gi + 2u);
+                        }
                     }
                 }
                 else if constexpr(Cfg::PrefetchC)
