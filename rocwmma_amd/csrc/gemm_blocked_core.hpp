@@ -128,7 +128,12 @@ namespace rocwmma_amd
             static constexpr uint32_t Stages     = Stages_; // ring of K stages in LDS
             static constexpr uint32_t WavesPerSimd = WavesPerSimd_;
             static constexpr uint32_t StagesB = Stages_ + (ExtraB_ ? 1u : 0u);
-            static constexpr uint32_t RingB   = Stages * BytesA; // LDS: the A stages, then the B stages
+            // LDS: stage by stage, A in front of B (one address serves both operands: with the rings of A and B apart the kernels
+            // on the ring of two needed more registers, the stream-K kernel of int8 spilled a third more and took 115.8 -> 131.9 us
+            // at 2560 x 2560 x 8192); with an extra B stage the ring of A, then the ring of B
+            static constexpr uint32_t StrideA = ExtraB_ ? BytesA : StageBytes;
+            static constexpr uint32_t StrideB = ExtraB_ ? BytesB : StageBytes;
+            static constexpr uint32_t FirstB  = ExtraB_ ? Stages * BytesA : BytesA;
             static constexpr uint32_t LdsBytes   = Stages * BytesA + StagesB * BytesB;
             static constexpr uint32_t CopiesA    = BytesA / 1024u / Waves; // direct copies per wave per stage
             static constexpr uint32_t CopiesB    = BytesB / 1024u / Waves;
@@ -585,7 +590,7 @@ namespace rocwmma_amd
             // advance == false leaves the source on the stage just copied (used to re-copy the last
             // stage instead of running past the end of the operand; edge tiles read nothing there)
             auto issueA = [&](uint32_t slot, bool advance = true) {
-                char*                 ldsA = ldsRaw + slot * Cfg::BytesA;
+                char*                 ldsA = ldsRaw + slot * Cfg::StrideA;
                 const lds::BufferRsrc src  = Cfg::Edges ? lds::makeSource(aSrc, aEnd) : lds::makeSource(aSrc);
                 if constexpr(CopyWaves < Cfg::Waves)
                 {
@@ -620,7 +625,7 @@ namespace rocwmma_amd
                     aSrc += advance ? aStep : size_t{0};
             };
             auto issueB = [&](uint32_t slot, bool advance = true) {
-                char*                 ldsB = ldsRaw + Cfg::RingB + slot * Cfg::BytesB;
+                char*                 ldsB = ldsRaw + Cfg::FirstB + slot * Cfg::StrideB;
                 const lds::BufferRsrc src  = Cfg::Edges ? lds::makeSource(bSrc, bEnd) : lds::makeSource(bSrc);
                 if constexpr(CopyWaves < Cfg::Waves)
                 {
@@ -666,8 +671,8 @@ namespace rocwmma_amd
             };
 
             auto readFragsOf = [&](Frags& f, uint32_t slot, uint32_t slotB, uint32_t ks) {
-                const char* ldsA = ldsRaw + slot * Cfg::BytesA;
-                const char* ldsB = ldsRaw + Cfg::RingB + slotB * Cfg::BytesB;
+                const char* ldsA = ldsRaw + slot * Cfg::StrideA;
+                const char* ldsB = ldsRaw + Cfg::FirstB + slotB * Cfg::StrideB;
                 if constexpr(Cfg::Scaled && Cfg::Block == 16u) // (has a reader of its own in its loop)
                     return;
                 else if constexpr(Cfg::Scaled)
@@ -831,7 +836,7 @@ namespace rocwmma_amd
                 typename Cfg::FragA fa[2][Cfg::BlocksM];
                 typename Cfg::FragB fb[NB];
                 auto readA = [&](typename Cfg::FragA(&dst)[Cfg::BlocksM], uint32_t slot) {
-                    const char* ldsA = ldsRaw + slot * Cfg::BytesA;
+                    const char* ldsA = ldsRaw + slot * Cfg::StrideA;
 #pragma unroll
                     for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                     {
@@ -846,7 +851,7 @@ namespace rocwmma_amd
                     }
                 };
                 auto readB = [&](typename Cfg::FragB& dst, uint32_t slot, uint32_t bj) {
-                    const char*    ldsB = ldsRaw + Cfg::RingB + slot * Cfg::BytesB;
+                    const char*    ldsB = ldsRaw + Cfg::FirstB + slot * Cfg::StrideB;
                     const uint32_t c0   = waveN * Cfg::WaveN + bj * Cfg::Block;
                     if constexpr(Cfg::Scaled)
                     {
@@ -1009,15 +1014,15 @@ namespace rocwmma_amd
                     }
                 };
                 readFrags(f[0], 0u, 0u);
-                uint32_t slot = 0u, slotB = 0u; // of stage i
+                // Slots of stage i.  Rings of two: its parity, taken where it is needed.  (Held in a variable over the body, the
+                // LDS addresses made from it stayed live with it: the stream-K kernels spilled 245 to 360 registers instead of 160
+                // to 256, 2560 x 2560 x 8192 int8 115.8 -> 131.9 us.)
+                constexpr bool ParityA = S == 2u, ParityB = SB == 2u;
+                uint32_t       ringA = 0u, ringB = 0u;
+                auto           slotA = [&](uint32_t i) { return ParityA ? i % 2u : ringA; };
+                auto           slotB = [&](uint32_t i) { return ParityB ? i % 2u : (SB == S ? slotA(i) : ringB); };
                 for(uint32_t i = 0; i < stages; ++i)
                 {
-                    if constexpr(S == 2u)
-                        slot = i % 2u;
-                    if constexpr(SB == S)
-                        slotB = slot;
-                    const uint32_t nextSlot  = S == 2u ? (i + 1u) % 2u : (slot + 1u == S ? 0u : slot + 1u);
-                    const uint32_t nextSlotB = SB == S ? nextSlot : (slotB + 1u == SB ? 0u : slotB + 1u);
 #pragma unroll
                     for(uint32_t ks = 0; ks + 1u < N; ++ks)
                     {
@@ -1027,7 +1032,7 @@ namespace rocwmma_amd
                             pinFrags(f[ks & 1u]);
                             __builtin_amdgcn_sched_barrier(0);
                         }
-                        readFragsOf(f[(ks + 1u) & 1u], slot, slotB, ks + 1u);
+                        readFragsOf(f[(ks + 1u) & 1u], slotA(i), slotB(i), ks + 1u);
                         multiplyStep(f[ks & 1u], i, ks);
                         scheduleInterleaved<Cfg::MfmasPerStep / 2u, Cfg::ReadsPerStep, 0u>();
                         __builtin_amdgcn_sched_barrier(0);
@@ -1036,8 +1041,8 @@ namespace rocwmma_amd
                     pinFrags(f[(N - 1u) & 1u]);
                     lds::barrier();
                     __builtin_amdgcn_sched_barrier(0);
-                    issueA(slot, i + S + 1u < stages);
-                    issueB(slotB, i + SB + 1u < stages);
+                    issueA(slotA(i), i + S + 1u < stages);
+                    issueB(slotB(i), i + SB + 1u < stages);
                     if constexpr(Cfg::Scaled)
                     {
                         if(i % 2u == 0u)
@@ -1046,9 +1051,11 @@ namespace rocwmma_amd
                             sB.load(sB.next, i / 2u + 1u < mx.pairs ? i / 2u + 1u : mx.pairs - 1u);
                         }
                     }
-                    readFragsOf(f[0], nextSlot, nextSlotB, 0u);
-                    slot  = nextSlot;
-                    slotB = nextSlotB;
+                    if constexpr(!ParityA)
+                        ringA = ringA + 1u == S ? 0u : ringA + 1u;
+                    if constexpr(SB != S)
+                        ringB = ringB + 1u == SB ? 0u : ringB + 1u;
+                    readFragsOf(f[0], slotA(i + 1u), slotB(i + 1u), 0u);
                     multiplyStep(f[(N - 1u) & 1u], i, N - 1u);
                     if constexpr(Cfg::Scaled)
                     {
@@ -1227,8 +1234,8 @@ namespace rocwmma_amd
                 // stage, then its MFMAs): 5 % faster than leaving the reads in front of the MFMAs.  With
                 // only A dim-major (4 blocks) the compiler's placement is 1 % better and is kept.
                 auto phaseByColumns = [&](Frags const& cur, Frags& nxt, uint32_t slot) {
-                    const char* ldsA = ldsRaw + slot * Cfg::BytesA;
-                    const char* ldsB = ldsRaw + Cfg::RingB + slot * Cfg::BytesB;
+                    const char* ldsA = ldsRaw + slot * Cfg::StrideA;
+                    const char* ldsB = ldsRaw + Cfg::FirstB + slot * Cfg::StrideB;
                     if constexpr(Cfg::Block == 16u)
                     {
                         static_assert(Cfg::BlocksM <= Cfg::BlocksN, "the A blocks are read along with the first B columns");

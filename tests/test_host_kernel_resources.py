@@ -10,7 +10,7 @@ import rocwmma_amd.api as api
 
 MAGIC = b"__CLANG_OFFLOAD_BUNDLE__"
 READELF = "/opt/rocm/llvm/bin/llvm-readelf"
-STREAMK_SPILLS = 360
+STREAMK_SPILLS = 256
 
 
 def device_objects(path):
