@@ -322,7 +322,8 @@ int rocwmma_amd_gemm_bias_act(int          dtype_in,
  * partly filled edge tiles): the call then
  * enqueues a small kernel that re-orders the scales into the workspace, and the GEMM (two launches); where that costs
  * more than it gives (128 x 128 and 128 x 64 tiles in one round or few, scales and their leading dimensions 4-byte
- * aligned), the GEMM alone, on the scales as they are.  What the workspace holds afterwards is undefined.  Everything else
+ * aligned), the GEMM alone, which reads the scales as they are.  Either way the re-ordered scales are in the workspace
+ * afterwards, as rocwmma_amd_gemm_mx_pack_scales leaves them.  Everything else
  * runs one block per wave straight from global memory, except up to 32 rows of a row-major A against a
  * col-major B with k a multiple of 1024 (few tokens against a wide weight matrix), which run on the
  * weight-streaming kernel with or without a workspace (m * k <= 128 KiB; scale_a 4-byte aligned with

@@ -433,13 +433,12 @@ int rocwmma_amd_gemm_mx(int         dtype_in,
         MxScales sc;
         if(mxBlockedProblem(layout_a, layout_b, args, scales, blocked, sc))
         {
-            rc = launchGemmMxBlockedRaw(dtype_in, blocked, sc, asStream(stream));
-            if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
-                return rc;
             char* packedA = static_cast<char*>(workspace);
             char* packedB = packedA + mxPackedScaleOffsetB(blocked.m, k);
-            rc            = launchMxPackScales(sc, blocked.m, blocked.n, k, packedA, packedB, !gemmMxBlockedUsesLargeTile(blocked),
-                                               asStream(stream));
+            rc            = launchGemmMxBlockedRaw(dtype_in, blocked, sc, packedA, packedB, asStream(stream));
+            if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
+                return rc;
+            rc = launchMxPackScales(sc, blocked.m, blocked.n, k, packedA, packedB, !gemmMxBlockedUsesLargeTile(blocked), asStream(stream));
             if(rc != ROCWMMA_AMD_OK)
                 return rc;
             rc = launchGemmMxBlocked(dtype_in, blocked, packedA, packedB, asStream(stream));

@@ -168,8 +168,9 @@ namespace rocwmma_amd
     // `elemBytes`-byte elements on partly filled 128 x 64 tiles over the ring of four 128-byte stages:
     // one round of workgroups with enough K to stream.  (The weight-streaming kernels leave those to it.)
     bool gemmBlockedTakesPartlyFilledLineTiles(uint32_t m, uint32_t n, uint32_t k, uint32_t elemBytes);
-    // the same on the scales as the caller has them (no re-ordering launch), for the shapes where that is faster
-    int  launchGemmMxBlockedRaw(int dtypeIn, GemmArgs const& args, MxScales const& scales, hipStream_t stream);
+    // the same on the scales as the caller has them (no re-ordering launch), for the shapes where that is faster; leaves the
+    // packed scales in packedA and packedB as launchMxPackScales does
+    int  launchGemmMxBlockedRaw(int dtypeIn, GemmArgs const& args, MxScales const& scales, void* packedA, void* packedB, hipStream_t stream);
     int  launchGemmMxBlocked(int dtypeIn, GemmArgs const& args, const void* packedA, const void* packedB, hipStream_t stream);
 
     // The blocked kernel with the fused epilogue (float types, row-major C/D; args.bias / args.activation)

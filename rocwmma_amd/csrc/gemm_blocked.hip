@@ -70,7 +70,7 @@ namespace rocwmma_amd
         if(g.layoutC != ROCWMMA_AMD_ROW_MAJOR || g.m % 16u != 0u || g.n % 16u != 0u || g.k % 128u != 0u)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         TileExtras ex{};
-        ex.mx = MxPacked{packedA, packedB, (g.k / 128u + 1u) / 2u, 0u, 0u};
+        ex.mx = MxPacked{packedA, packedB, (g.k / 128u + 1u) / 2u, 0u, 0u, nullptr, nullptr};
         const bool large = gemmMxBlockedUsesLargeTile(g);
         if(dtypeIn == ROCWMMA_AMD_E4M3)
             return large ? launchMx<float8_t>(g, ex, stream) : launchMxMid<float8_t, false>(g, ex, stream);
@@ -79,22 +79,25 @@ namespace rocwmma_amd
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 
-    int launchGemmMxBlockedRaw(int dtypeIn, GemmArgs const& g, MxScales const& s, hipStream_t stream)
+    int launchGemmMxBlockedRaw(int dtypeIn, GemmArgs const& g, MxScales const& s, void* packedA, void* packedB, hipStream_t stream)
     {
         const bool dwords = ((reinterpret_cast<uintptr_t>(s.a) | reinterpret_cast<uintptr_t>(s.b)) & 3u) == 0u && (s.lda | s.ldb) % 4u == 0u;
-        if(g.layoutC != ROCWMMA_AMD_ROW_MAJOR || g.m % 16u != 0u || g.n % 16u != 0u || g.k % 128u != 0u || g.k < 256u || !dwords
+        if(g.layoutC != ROCWMMA_AMD_ROW_MAJOR || g.m % 16u != 0u || g.n % 16u != 0u || g.k % 128u != 0u || g.k < 256u || g.k >= (1u << 30) || !dwords
            || gemmMxBlockedUsesLargeTile(g))
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-        // What the re-ordering launch costs (4 to 6 us) against what the scattered scale loads cost in the main loop: on the
-        // ring of four always less (48 x 14336 x 4096 27.6 -> 21.8 us, 128 rows 29.3 -> 26.5), on the ring of two about
-        // 0.13 us per stage with a tile per compute unit (384 x 1056 x 1536 16.1 -> 12.6, but 128 x 1024 x 8192 52 -> 57) and
-        // 0.4 per stage and round with two (2000 x 3056 x 1408 25.1 -> 24.0, 512 x 14336 x 4096 57 -> 75).
+        // What the re-ordering launch costs (1.5 to 3 us on operands from HBM) against what the scattered scale loads and the
+        // stores of the packed order cost in the main loop.  On the ring of four that grows with the rows a tile has and with K:
+        // 48 x 14336 x 4096 26.1 -> 23.1 us and x 8192 x 8192 40.0 -> 37.1, 128 rows 27.9 -> 26.5 but 42.0 -> 43.5, 256 x 4096 x
+        // 14336 68.6 -> 71.1.  On the ring of two: 384 x 7168 x 2048 24.4 -> 20.9, 1024 x 1200 x 1408 14.0 -> 12.1, but 128 x 1024 x
+        // 8192 52 -> 57; with more tiles than units 4096 x 1200 x 1408 24.4 -> 21.1, 512 x 14336 x 4096 57 -> 75.
         const uint32_t units = computeUnits(), stages = g.k / 128u, tiles = ceilDiv(g.m, 128u) * ceilDiv(g.n, 128u);
-        if(!gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u)
-           && (tiles <= units ? stages > 30u : static_cast<uint64_t>(stages) * ceilDiv(tiles, 2u * units) > 12u))
+        const bool     raw   = gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u) ? stages <= (g.m <= 96u ? 64u : 44u)
+                               : tiles <= units ? stages <= 30u
+                                                : static_cast<uint64_t>(stages) * ceilDiv(tiles, 2u * units) <= 12u;
+        if(!raw)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         TileExtras ex{};
-        ex.mx = MxPacked{s.a, s.b, (g.k / 128u + 1u) / 2u, s.lda, s.ldb};
+        ex.mx = MxPacked{s.a, s.b, (g.k / 128u + 1u) / 2u, s.lda, s.ldb, packedA, packedB};
         if(dtypeIn == ROCWMMA_AMD_E4M3)
             return launchMxMid<float8_t, true>(g, ex, stream);
         if(dtypeIn == ROCWMMA_AMD_E5M2)

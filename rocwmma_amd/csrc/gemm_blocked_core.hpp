@@ -277,7 +277,20 @@ namespace rocwmma_amd
             // RawScales: a and b are the caller's scales, one row of k / 32 bytes per row of A / column of B, these many
             // bytes apart (4-byte aligned).  A lane then loads the eight bytes of its row for a pair of stages as they lie.
             uint32_t    lda, ldb;
+            void*       packedA; // RawScales: where the packed order is left (PairScales)
+            void*       packedB;
         };
+
+        // The packed dword of a 32-wide block and lane out of the eight scales of the lane's row for a pair of stages (lo: K blocks
+        // 0..3, hi: 4..7): byte = instruction step, of which lanes 0..31 take the even K block and lanes 32..63 the odd one.
+        ROCWMMA_DEVICE ROCWMMA_INLINE uint32_t packPairScales(uint32_t lo, uint32_t hi, uint32_t lane)
+        {
+#if ROCWMMA_ARCH_GFX950
+            return __builtin_amdgcn_perm(hi, lo, lane < 32u ? 0x06040200u : 0x07050301u);
+#else
+            return lo ^ hi ^ lane;
+#endif
+        }
 
         // What a Fused configuration's epilogue does beyond alpha * acc + beta * C.
         struct FusedEpilogue
@@ -294,21 +307,27 @@ namespace rocwmma_amd
         };
 
         // Scales of a wave's 32-wide blocks along one dimension, a pair of stages (256 bytes of K, four instruction steps) at a
-        // time.  Packed: one dword per block and lane, byte = step.  Raw: the eight bytes of the lane's row, of which the
-        // lanes 0..31 take the even and the lanes 32..63 the odd ones; rows past the problem's take its last row's (they
-        // only meet zeros), and a last pair that is half a pair starts four bytes early.
+        // time: one dword per block and lane, byte = step.  Raw: made from the eight bytes of the lane's row (rows past the
+        // problem's get the scale 1; a last pair that is half a pair starts four bytes early), and left in the workspace in
+        // the packed order all the same, as the re-ordering launch leaves them: the workspace then serves calls on packed
+        // scales.  The dwords are what the lanes hold anyway, so that is a store per pair of stages: 128 x 14336 x 4096 e4m3
+        // 18.6 -> 19.2 us (read again and written behind the results: 21.0; with the re-ordering launch: 20.7).  Waves that have
+        // nothing to leave store past the end of an empty buffer, without a branch.
         template <typename Cfg, uint32_t Blocks>
         struct PairScales
         {
             static constexpr bool Raw = Cfg::RawScales;
-            static_assert(Blocks == 1u || Blocks % 2u == 0u, "a wave's blocks: one, or whole groups of two");
-            uint32_t       now[Raw ? 2u * Blocks : Blocks] = {}, next[Raw ? 2u * Blocks : Blocks] = {};
+            static_assert(Blocks == 1u || Blocks == 2u || (!Raw && Blocks % 2u == 0u), "a wave's blocks: one, or whole groups of two");
+            uint32_t       now[Blocks] = {}, next[Raw ? 2u * Blocks : Blocks] = {};
             const char*    from[Raw ? Blocks : 1u];
-            uint32_t       pairs, last, half; // last: Raw, byte the last whole pair of a row starts at
-            ROCWMMA_DEVICE ROCWMMA_INLINE PairScales(const void* scales, uint32_t ld, uint32_t pairs_, uint32_t row0, uint32_t rows, uint32_t k, uint32_t lane)
+            bool           inside[Raw ? Blocks : 1u]; // this lane's row of a block is one of the problem's
+            uint32_t       pairs, last, lane, keepAt; // last: Raw, byte the last whole pair of a row starts at
+            lds::BufferRsrc kept; // Raw: the packed scales of this wave's group of 64 rows
+            ROCWMMA_DEVICE ROCWMMA_INLINE
+                PairScales(const void* scales, uint32_t ld, uint32_t pairs_, uint32_t row0, uint32_t rows, uint32_t k, uint32_t lane_, void* packed, bool keeper)
                 : pairs(pairs_)
                 , last(k / 32u - 8u)
-                , half(lane >> 5)
+                , lane(lane_)
             {
                 if constexpr(Raw)
                 {
@@ -316,8 +335,12 @@ namespace rocwmma_amd
                     for(uint32_t b = 0; b < Blocks; ++b)
                     {
                         const uint32_t row = row0 + b * 32u + (lane & 31u);
-                        from[b]            = static_cast<const char*>(scales) + static_cast<size_t>(row < rows ? row : rows - 1u) * ld;
+                        inside[b]          = row < rows;
+                        from[b]            = static_cast<const char*>(scales) + static_cast<size_t>(inside[b] ? row : rows - 1u) * ld;
                     }
+                    char* group = static_cast<char*>(packed) + static_cast<size_t>(row0 / 64u) * pairs * 512u;
+                    kept        = lds::makeSource(group, keeper && row0 / 64u * 64u < rows ? group + static_cast<size_t>(pairs) * 512u : group);
+                    keepAt      = lane * 8u + (row0 / 32u) % 2u * 4u;
                 }
                 else // (dword of block b, pair p, lane l: (((b / 2) * pairs + p) * 64 + l) * 2 + b % 2)
                     from[0] = static_cast<const char*>(scales) + ((static_cast<size_t>(row0 / 64u) * pairs * 64u + lane) * 2u + (row0 / 32u) % 2u) * 4u;
@@ -341,30 +364,32 @@ namespace rocwmma_amd
             // The loaded pair `pair` takes over.
             ROCWMMA_DEVICE ROCWMMA_INLINE void take(uint32_t(&loaded)[Raw ? 2u * Blocks : Blocks], uint32_t pair)
             {
+                const bool halfPair = 8u * pair > last; // (wave uniform)
+#pragma unroll
+                for(uint32_t b = 0; b < Blocks; ++b)
+                {
+                    if constexpr(Raw)
+                    {
+                        const uint32_t lo = halfPair ? loaded[2u * b + 1u] : loaded[2u * b], hi = halfPair ? 0x7f7f7f7fu : loaded[2u * b + 1u];
+                        now[b]            = inside[b] ? packPairScales(lo, hi, lane) : 0x7f7f7f7fu;
+                    }
+                    else
+                        now[b] = loaded[b];
+                }
                 if constexpr(Raw)
                 {
-                    const bool halfPair = 8u * pair > last; // (wave uniform)
-#pragma unroll
-                    for(uint32_t b = 0; b < Blocks; ++b)
-                    {
-                        now[2u * b]      = (halfPair ? loaded[2u * b + 1u] : loaded[2u * b]) >> (8u * half);
-                        now[2u * b + 1u] = loaded[2u * b + 1u] >> (8u * half);
-                    }
-                }
-                else
-                {
-#pragma unroll
-                    for(uint32_t b = 0; b < Blocks; ++b)
-                        now[b] = loaded[b];
+                    // (a pair past the last lies past the end of the buffer as well)
+                    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+                    if constexpr(Blocks == 2u)
+                        __builtin_amdgcn_raw_buffer_store_b64(u32x2_t{now[0], now[1]}, kept, static_cast<int>(keepAt + pair * 512u), 0, 0);
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b32(now[0], kept, static_cast<int>(keepAt + pair * 512u), 0, 0);
                 }
             }
             // scale of block b at instruction step `step` (0..3) of the pair, in the lowest byte
             ROCWMMA_DEVICE ROCWMMA_INLINE uint32_t at(uint32_t b, uint32_t step) const
             {
-                if constexpr(Raw)
-                    return (step < 2u ? now[2u * b] : now[2u * b + 1u]) >> (16u * (step % 2u));
-                else
-                    return now[b] >> (8u * step);
+                return now[b] >> (8u * step);
             }
         };
 
@@ -956,8 +981,8 @@ namespace rocwmma_amd
                 // instruction steps), one dword per block of 32 rows, byte = step; the step's byte is shifted
                 // down at run time.  The next pair's are loaded behind the barrier of a pair's first stage.
                 static_assert(!Cfg::Scaled || Cfg::KSteps == 2u, "packed scales: two instruction steps per stage");
-                PairScales<Cfg, Cfg::Scaled ? Cfg::BlocksM : 1u> sA(mx.a, mx.lda, mx.pairs, row0 + waveM * Cfg::WaveM, m, k, lane);
-                PairScales<Cfg, Cfg::Scaled ? Cfg::BlocksN : 1u> sB(mx.b, mx.ldb, mx.pairs, col0 + waveN * Cfg::WaveN, n, k, lane);
+                PairScales<Cfg, Cfg::Scaled ? Cfg::BlocksM : 1u> sA(mx.a, mx.lda, mx.pairs, row0 + waveM * Cfg::WaveM, m, k, lane, mx.packedA, tn == 0u && waveN == 0u);
+                PairScales<Cfg, Cfg::Scaled ? Cfg::BlocksN : 1u> sB(mx.b, mx.ldb, mx.pairs, col0 + waveN * Cfg::WaveN, n, k, lane, mx.packedB, tm == 0u && waveM == 0u);
                 if constexpr(Cfg::Scaled)
                 {
                     // (in front of the first copies and kept there: the wait for stage 0 then covers these loads,
@@ -1082,8 +1107,8 @@ namespace rocwmma_amd
                 // over.  Every trip issues its stages (past the end of K the last stage again, into a slot nobody
                 // reads), so the body and its counts are uniform.
                 static_assert(S == 4u && Cfg::StageKB == 128u && Cfg::Block == 32u && Part == TilePart::Whole, "scaled ring of four: 128-byte stages of 32-wide blocks");
-                PairScales<Cfg, Cfg::BlocksM> sA(mx.a, mx.lda, mx.pairs, row0 + waveM * Cfg::WaveM, m, k, lane);
-                PairScales<Cfg, Cfg::BlocksN> sB(mx.b, mx.ldb, mx.pairs, col0 + waveN * Cfg::WaveN, n, k, lane);
+                PairScales<Cfg, Cfg::BlocksM> sA(mx.a, mx.lda, mx.pairs, row0 + waveM * Cfg::WaveM, m, k, lane, mx.packedA, tn == 0u && waveN == 0u);
+                PairScales<Cfg, Cfg::BlocksN> sB(mx.b, mx.ldb, mx.pairs, col0 + waveN * Cfg::WaveN, n, k, lane, mx.packedB, tm == 0u && waveM == 0u);
                 auto multiplyScaled = [&](Frags const& fr, auto stepC) {
 #if ROCWMMA_ARCH_GFX950 // (the instruction table exists in the device pass only)
                     using Op  = detail::MfmaScaled<detail::TypeInfo<InT>::cls, detail::TypeInfo<InT>::cls, 32u>;
