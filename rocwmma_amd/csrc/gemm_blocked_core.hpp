@@ -80,6 +80,8 @@ namespace rocwmma_amd
             // so the fragments are read like two steps of a 16-bytes-per-lane operand.
             static constexpr bool     Scaled  = Scaled_;
             static constexpr bool     RawScales = RawScales_;
+            // (block scales come with K in whole stages: 64 x 4096 x 4096 e4m3 27.1 us with the K bounds, 26.4 without)
+            static constexpr bool     EdgesK  = Edges_ && !Scaled_;
             // D = act(alpha * A * B + beta * C + bias[column]): see FusedEpilogue
             static constexpr bool     Fused   = Fused_;
             static constexpr uint32_t WavesM  = WavesM_;
@@ -599,7 +601,7 @@ namespace rocwmma_amd
                 bLaneOff[j] = TileB::laneSourceOffset(lane, wave % CopyWaves + (Cfg::BKMajor ? 0u : j * CopyWaves), ldbB);
             }
 
-            // Edges: what is left of K (elements) at the stage the next copies read, and the first K element of
+            // EdgesK: what is left of K (elements) at the stage the next copies read, and the first K element of
             // this lane's 16 bytes of a K-contiguous operand.  A lane whose bytes lie past the end of K asks for
             // an address beyond the buffer's bounds and gets zeros; rows of a dim-major operand past K are
             // beyond its end as they are.  Two vector instructions per operand and stage.
@@ -607,7 +609,7 @@ namespace rocwmma_amd
             const uint32_t aLaneK = TileA::laneK(lane, wave % CopyWaves) / static_cast<uint32_t>(sizeof(InT));
             const uint32_t bLaneK = TileB::laneK(lane, wave % CopyWaves) / static_cast<uint32_t>(sizeof(InT));
             auto           insideK = [](bool kMajor, uint32_t offset, uint32_t laneK, uint32_t left) {
-                return (Cfg::Edges && kMajor && laneK >= left) ? (offset | 0x80000000u) : offset;
+                return (Cfg::EdgesK && kMajor && laneK >= left) ? (offset | 0x80000000u) : offset;
             };
 
             // A stage is copied in two halves (the A operand, then the B operand) so that each
@@ -641,7 +643,7 @@ namespace rocwmma_amd
                                          TileA::copySourceOffset(copy, ldaB));
                     }
                 }
-                if constexpr(Cfg::Edges)
+                if constexpr(Cfg::EdgesK)
                 {
                     aSrc += aStep;
                     aLeft = aLeft > Cfg::MacroK ? aLeft - Cfg::MacroK : 0u;
@@ -676,7 +678,7 @@ namespace rocwmma_amd
                                          TileB::copySourceOffset(copy, ldbB));
                     }
                 }
-                if constexpr(Cfg::Edges)
+                if constexpr(Cfg::EdgesK)
                 {
                     bSrc += bStep;
                     bLeft = bLeft > Cfg::MacroK ? bLeft - Cfg::MacroK : 0u;
