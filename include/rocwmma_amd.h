@@ -141,8 +141,8 @@ int rocwmma_amd_gemm(int         dtype_in,
 
 /* Same as rocwmma_amd_gemm with the kernel family forced (`algo` is a rocwmma_amd_gemm_algo).
  * Asked for by name, the blocked kernel keeps to whole stages: ROCWMMA_AMD_GEMM_BLOCKED returns
- * ROCWMMA_AMD_UNSUPPORTED_SHAPE when k is not in whole 64-byte stages, at least three of them (and
- * ROCWMMA_AMD_UNSUPPORTED_TYPE for float32), and _BLOCKED_256 when the shape does not fill whole 256 x 256 tiles, like the reference's perf_hgemm host
+ * ROCWMMA_AMD_UNSUPPORTED_SHAPE when k is not in whole 64-byte stages, at least three of them (two for problems of
+ * more than one round of workgroups; ROCWMMA_AMD_UNSUPPORTED_TYPE for float32), and _BLOCKED_256 when the shape does not fill whole 256 x 256 tiles, like the reference's perf_hgemm host
  * (samples/perf_hgemm.cpp:735-765). */
 int rocwmma_amd_gemm_ex(int         algo,
                         int         dtype_in,

@@ -111,6 +111,22 @@ namespace rocwmma_amd
             layoutB      = lb;
             g.layoutC    = ROCWMMA_AMD_ROW_MAJOR;
         }
+
+        // K that the blocked kernel takes when a caller names it: whole stages of 64 bytes, three of them, or two for problems
+        // of more than one round of workgroups (in whole tiles, or 128 x 128 tiles partly filled) and for the 256 x 256 tile
+        // asked for by name.  (AUTO takes any K.)
+        bool blockedTakesByName(GemmArgs const& g, int layoutA, int layoutB, uint32_t elemBytes, bool largeTile, uint32_t units)
+        {
+            const uint64_t kBytes = static_cast<uint64_t>(g.k) * elemBytes;
+            if(kBytes % 64u != 0u || kBytes < 128u)
+                return false;
+            if(kBytes != 128u || largeTile)
+                return true;
+            const bool contiguous = layoutA == ROCWMMA_AMD_ROW_MAJOR && layoutB == ROCWMMA_AMD_COL_MAJOR; // (both along K)
+            auto       whole      = [&](uint32_t edge) { return g.m % edge == 0u && g.n % edge == 0u; };
+            auto       tiles      = [&](uint32_t edge) { return static_cast<uint64_t>(rocwmma::ceilDiv(g.m, edge)) * rocwmma::ceilDiv(g.n, edge); };
+            return (whole(256u) && 2u * tiles(256u) >= units) || tiles(128u) > units || (contiguous && whole(64u) && tiles(64u) > units);
+        }
     } // namespace
 } // namespace rocwmma_amd
 
@@ -208,18 +224,17 @@ int rocwmma_amd_gemm_ex(int         algo,
     }
     if(algo != ROCWMMA_AMD_GEMM_WAVE_TILE)
     {
-        // asked for by name, the blocked kernel takes whole stages of K only, and no float32
-        if(algo != ROCWMMA_AMD_GEMM_AUTO)
-        {
-            const uint64_t kBytes = static_cast<uint64_t>(k) * dtypeSize(dtype_in);
-            if(dtype_in == ROCWMMA_AMD_F32)
-                return ROCWMMA_AMD_UNSUPPORTED_TYPE;
-            if(kBytes % 64u != 0u || kBytes < 192u)
-                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-        }
         GemmArgs blocked = args;
         int      la = layout_a, lb = layout_b;
         transposeForColMajorC(blocked, la, lb);
+        // asked for by name, the blocked kernel takes whole stages of K only, and no float32
+        if(algo != ROCWMMA_AMD_GEMM_AUTO)
+        {
+            if(dtype_in == ROCWMMA_AMD_F32)
+                return ROCWMMA_AMD_UNSUPPORTED_TYPE;
+            if(!blockedTakesByName(blocked, la, lb, dtypeSize(dtype_in), algo == ROCWMMA_AMD_GEMM_BLOCKED_256, computeUnits()))
+                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+        }
         rc = launchGemmBlocked(dtype_in, dtype_out, la, lb, blocked, asStream(stream), algo == ROCWMMA_AMD_GEMM_BLOCKED_256);
         if(rc == ROCWMMA_AMD_OK || algo == ROCWMMA_AMD_GEMM_BLOCKED || algo == ROCWMMA_AMD_GEMM_BLOCKED_256)
             return rc;
