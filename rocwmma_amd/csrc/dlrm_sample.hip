@@ -23,6 +23,7 @@
 // 8192 119 -> 41 us (4.3 TB/s), 94 x 232 float16 batch 5738 394 -> 183 us.  (A first version unpacked G into an LDS
 // square with loads of its own, a serial chain of load latencies: 41 x 72 backward 65 instead of 26 us.)
 #include "common.hpp"
+#include "launch_limits.hpp"
 #include <rocwmma/rocwmma_lds.hpp>
 
 using namespace rocwmma;
@@ -459,9 +460,15 @@ namespace rocwmma_amd
             const uint32_t lds    = s.sampleBytes * (wavesOf(PerSample) / PerSample);
             if(int rc = optInLds(kernel, lds))
                 return rc;
-            hipLaunchKernelGGL(kernel, dim3(ceilDiv(s.batch, wavesOf(PerSample) / PerSample)), dim3(64u * wavesOf(PerSample)), lds, stream, static_cast<const T*>(input),
-                               static_cast<T*>(output), s);
-            return launchStatus();
+            constexpr uint32_t perGroup = wavesOf(PerSample) / PerSample, threads = 64u * wavesOf(PerSample);
+            return forEachLaunch(s.batch, threads, perGroup, [&](uint32_t first, uint32_t count) {
+                SampleShape part = s;
+                part.batch       = count;
+                hipLaunchKernelGGL(kernel, dim3(ceilDiv(count, perGroup)), dim3(threads), lds, stream,
+                                   static_cast<const T*>(input) + static_cast<size_t>(first) * s.m * s.k,
+                                   static_cast<T*>(output) + static_cast<size_t>(first) * s.width, part);
+                return launchStatus();
+            });
         }
         template <typename T, uint32_t PerSample, uint32_t Max>
         int launchBwd(const void* input, const void* upstream, void* grad, void* mlpGrad, SampleShape const& s, hipStream_t stream)
@@ -470,9 +477,16 @@ namespace rocwmma_amd
             const uint32_t lds    = s.sampleBytes * (wavesOf(PerSample) / PerSample);
             if(int rc = optInLds(kernel, lds))
                 return rc;
-            hipLaunchKernelGGL(kernel, dim3(ceilDiv(s.batch, wavesOf(PerSample) / PerSample)), dim3(64u * wavesOf(PerSample)), lds, stream, static_cast<const T*>(input),
-                               static_cast<const T*>(upstream), static_cast<T*>(grad), static_cast<T*>(mlpGrad), s);
-            return launchStatus();
+            constexpr uint32_t perGroup = wavesOf(PerSample) / PerSample, threads = 64u * wavesOf(PerSample);
+            return forEachLaunch(s.batch, threads, perGroup, [&](uint32_t first, uint32_t count) {
+                SampleShape  part     = s;
+                const size_t features = static_cast<size_t>(first) * s.m * s.k;
+                part.batch            = count;
+                hipLaunchKernelGGL(kernel, dim3(ceilDiv(count, perGroup)), dim3(threads), lds, stream, static_cast<const T*>(input) + features,
+                                   static_cast<const T*>(upstream) + static_cast<size_t>(first) * s.width, static_cast<T*>(grad) + features,
+                                   static_cast<T*>(mlpGrad) + static_cast<size_t>(first) * s.k, part);
+                return launchStatus();
+            });
         }
 
         template <typename T, uint32_t PerSample>
