@@ -624,7 +624,7 @@ int rocwmma_amd_dlrm_fwd(const void* input, void* output, uint32_t m, uint32_t k
         return ROCWMMA_AMD_BAD_ALIGNMENT;
     if(!isGfx950Current())
         return ROCWMMA_AMD_NO_DEVICE;
-    // 17 to 32 rows of the usual widths; samples that fit the LDS; tiles
+    // up to 32 rows of the usual widths; samples that fit the LDS; tiles
     rc = launchDlrmFwd(input, output, m, k, batch, asStream(stream));
     if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
         return rc;

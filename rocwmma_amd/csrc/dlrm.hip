@@ -16,10 +16,8 @@
 //     gradient (no global m x m scratch, no second launch), reads F^T operands with the
 //     transposing LDS load, and writes grad through LDS the same way.
 //
-// The general form of both is in dlrm_sample.hip, which is as fast or faster everywhere but where these are still
-// used: 17 to 32 rows, from five samples per compute unit on, widths of 32, 64 and 128 forward and 64 and 128 backward
-// (forward, 24 x 32 batch 16384 8.5 against 10.0 us, 17 x 128 14.5 against 15.8; forward + backward, 27 x 128 batch 1024 9.0
-// against 8.7, 2048 12.2 against 12.7, 8192 34.9 against 37.1, 262144 1077 against 1108; 27 x 64 batch 2048 8.6 against 9.1).
+// The general form of both is in dlrm_sample.hip, which is as fast or faster everywhere but where these are still used (takesFwd,
+// takesBwd).
 //
 // Both kernels are judged on bytes moved: forward reads m*k and writes k + m(m-1)/2 halves per
 // sample; backward reads m*k + k + m(m-1)/2 and writes m*k + k.
@@ -454,10 +452,23 @@ namespace rocwmma_amd
                                static_cast<float16_t*>(mlpGrad), m, batch);
             return launchStatus();
         }
-        // The batch from which these kernels are used (see the head of the file).
-        inline bool largeEnough(uint32_t m, uint32_t batch)
+        // Where these kernels are used, against those of dlrm_sample.hip.  Forward, in us, these / those: widths 32, 64 and 128,
+        // 17 to 32 rows, whatever the batch (27 x 128 batch 16 2.87 / 2.99, 512 2.99 / 3.21, 1024 3.7 / 4.1; 24 x 32 batch 16384
+        // 8.5 / 10.0) and up to 16 rows for batches of up to 16 samples per unit (8 x 64 batch 2048 2.7 / 3.7, 4096 3.4 / 4.0, but 8192
+        // 4.4 / 4.1); width 256 for up to two samples per unit (27 x 256 batch 512 3.35 / 3.59).  (Forward of width 256 stays there
+        // for larger batches, 6 to 13 % slower on its own at three to eight samples per unit: backward then finds a sample's
+        // features in its XCD's L2, forward and backward 27 x 256 batch 2048 21.7 with forward here, 19.0 with both there.)
+        inline bool takesFwd(uint32_t m, uint32_t k, uint32_t batch)
         {
-            return m > 16u && m <= kMaxM && batch >= 5u * computeUnits();
+            const uint64_t units = computeUnits();
+            return m <= kMaxM && (k == 256u ? batch <= 2u * units : m > 16u || batch <= 16u * units);
+        }
+        // Backward: 17 to 32 rows, widths 64 and 128 from five samples per unit on (27 x 128 batch 1024 5.2 / 4.7, 2048 7.2 / 7.5, 8192 forward
+        // and backward 34.9 / 37.1), width 32 from eight on (27 x 32 batch 2048 forward and backward 6.6 / 6.9).
+        inline bool takesBwd(uint32_t m, uint32_t k, uint32_t batch)
+        {
+            const uint64_t units = computeUnits();
+            return m > 16u && m <= kMaxM && batch >= (k == 32u ? 8u : 5u) * units;
         }
 
         // Samples per workgroup.  Backward: 8 once that still leaves >= 8 workgroups per compute unit (the longest
@@ -484,7 +495,7 @@ namespace rocwmma_amd
 
     int launchDlrmFwd(const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream)
     {
-        if(!largeEnough(m, batch))
+        if(!takesFwd(m, k, batch))
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         switch(k)
         {
@@ -494,6 +505,8 @@ namespace rocwmma_amd
             return launchFwd<64>(input, output, m, batch, stream);
         case 128:
             return launchFwd<128>(input, output, m, batch, stream);
+        case 256:
+            return launchFwd<256>(input, output, m, batch, stream);
         default:
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         }
@@ -502,10 +515,12 @@ namespace rocwmma_amd
     int launchDlrmBwd(const void* input, const void* upstream, void* grad, void* mlpGrad, uint32_t m, uint32_t k,
                       uint32_t batch, hipStream_t stream)
     {
-        if(!largeEnough(m, batch))
+        if(!takesBwd(m, k, batch))
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         switch(k)
         {
+        case 32:
+            return launchBwd<32>(input, upstream, grad, mlpGrad, m, batch, stream);
         case 64:
             return launchBwd<64>(input, upstream, grad, mlpGrad, m, batch, stream);
         case 128:

@@ -885,6 +885,26 @@ namespace rocwmma_amd
         }
     } // namespace
 
+    namespace
+    {
+        // float16 forward, where dlrmFwdStagedKernel is ahead of the tiles of dlrm_general_fwd.hip: batches of many rounds of tiles (two
+        // per unit) whose tiles are partly filled or half above the diagonal.  Its waves skip 64 x 64 blocks that hold no result
+        // and four of its workgroups share a unit.  Staged / tiles in us: (193, 64) batch 4096 118 / 128, (256, 64) 145 / 163,
+        // (320, 128) 32 rounds 1.16 times, (400, 128) 451 / 481; but 8 rounds of (256, 128) 0.97, (384, k) never above 1.02, (512, k) 0.80
+        // to 0.99.  One tile per sample (up to 128 rows that do not fit the LDS): (96, 512) batch 1024 26.3.
+        bool stagedFwdIsFaster(uint32_t m, uint32_t k, uint32_t tiles, uint32_t batch)
+        {
+            const uint64_t units = computeUnits(), rounds = static_cast<uint64_t>(tiles) * batch / (2u * units);
+            if(m <= 128u)
+                return batch > units;
+            if(m <= 256u)
+                return k <= 512u && rounds >= 12u;
+            if(m <= 352u)
+                return k <= 512u && rounds >= 6u;
+            return m > 384u && m <= 416u && k <= 256u && rounds >= 24u;
+        }
+    } // namespace
+
     // Shapes: 1 <= m <= 32768; k a multiple of 8 (f16) or 4 (f32), so that a row's 16-byte pieces are whole; a sample's
     // features below 2 GiB (32-bit byte offsets into a bounds-checked buffer).
     int launchDlrmFwdGeneral(int dtype, const void* input, void* output, uint32_t m, uint32_t k, uint32_t batch, hipStream_t stream)
@@ -898,7 +918,7 @@ namespace rocwmma_amd
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         if(dtype == ROCWMMA_AMD_F16)
         {
-            const int rc = launchDlrmFwdTilesF16(input, output, m, k, batch, stream);
+            const int rc = stagedFwdIsFaster(m, k, tiles, batch) ? ROCWMMA_AMD_UNSUPPORTED_SHAPE : launchDlrmFwdTilesF16(input, output, m, k, batch, stream);
             if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE) // (feature rows of more than 16 MiB)
                 return rc;
             hipLaunchKernelGGL(dlrmFwdStagedKernel<float16_t>, dim3(grid), dim3(256), 0, stream, static_cast<const float16_t*>(input),

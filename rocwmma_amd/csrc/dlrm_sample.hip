@@ -519,6 +519,15 @@ namespace rocwmma_amd
         const SampleShape s    = shapeOf(m, k, batch, size, false);
         if(m > kMaxRows || s.sampleBytes > kLdsBytes)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+        // The 128 x 128 tiles of a few large samples (three each from 129 rows on) run side by side where one workgroup per
+        // sample leaves units idle: float32 180 x 160 batch 64 22.4 -> 17.4 us, 192 x 136 20.9 -> 17.5, but not up to 160 rows (160 x 200
+        // 10.5 here) nor at narrow ones.  float16 samples of more than half the LDS have a unit to themselves: as tiles where those
+        // fill the device better, 192 x 256 batch 64 11.1 -> 8.4, and from two samples per unit on, 192 x 256 batch 1024 56.9 -> 44.5, 96 x 512
+        // 34.9 -> 26.3.
+        const uint32_t units = computeUnits();
+        const bool     fewTiles = m > 128u && 3u * static_cast<uint64_t>(batch) <= units;
+        if(size == 4u ? fewTiles && m > 160u && k >= 64u : s.sampleBytes > kLdsBytes / 2u && (fewTiles || batch > units))
+            return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         const uint32_t perSample = wavesPerSample(s, false);
         if(dtype == ROCWMMA_AMD_F16)
             return perSample == 1u   ? fwdByRows<float16_t, 1>(input, output, s, stream)
@@ -537,6 +546,10 @@ namespace rocwmma_amd
         const uint32_t    size = dtype == ROCWMMA_AMD_F16 ? 2u : 4u;
         const SampleShape s    = shapeOf(m, k, batch, size, true);
         if(m > kMaxRows || s.sampleBytes > kLdsBytes)
+            return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+        // float32, wide samples in a batch that leaves units idle: 128-column tiles of their own (64 x 512 batch 64 15.9 -> 13.1 us,
+        // 40 x 700 batch 16 12.3 -> 10.6)
+        if(size == 4u && k > 256u && static_cast<uint64_t>(ceilDiv(k, 128u)) * batch <= computeUnits())
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         const uint32_t perSample = wavesPerSample(s, true);
         if(dtype == ROCWMMA_AMD_F16)
