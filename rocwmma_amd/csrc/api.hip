@@ -235,7 +235,8 @@ int rocwmma_amd_gemm_ex(int         algo,
             if(!blockedTakesByName(blocked, la, lb, dtypeSize(dtype_in), algo == ROCWMMA_AMD_GEMM_BLOCKED_256, computeUnits()))
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         }
-        rc = launchGemmBlocked(dtype_in, dtype_out, la, lb, blocked, asStream(stream), algo == ROCWMMA_AMD_GEMM_BLOCKED_256);
+        rc = launchGemmBlocked(dtype_in, dtype_out, la, lb, blocked, asStream(stream),
+                               algo == ROCWMMA_AMD_GEMM_AUTO ? TileUse::Any : (algo == ROCWMMA_AMD_GEMM_BLOCKED_256 ? TileUse::Large : TileUse::Blocked));
         if(rc == ROCWMMA_AMD_OK || algo == ROCWMMA_AMD_GEMM_BLOCKED || algo == ROCWMMA_AMD_GEMM_BLOCKED_256)
             return rc;
         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)

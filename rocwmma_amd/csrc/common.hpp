@@ -114,14 +114,21 @@ namespace rocwmma_amd
     // Family launchers (one translation unit each).  Return a rocwmma_amd_status;
     // ROCWMMA_AMD_UNSUPPORTED_SHAPE / _TYPE mean "this family has no kernel for it".
     int launchGemmWaveTile(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream);
-    // forceLargeTile: the 256 x 256 tile or nothing (ROCWMMA_AMD_GEMM_BLOCKED_256)
+    // Which tiles a call may run on: any, one block per wave among them (ROCWMMA_AMD_UNSUPPORTED_SHAPE then asks for it), any of the
+    // blocked kernel's (ROCWMMA_AMD_GEMM_BLOCKED), or the 256 x 256 tile (ROCWMMA_AMD_GEMM_BLOCKED_256)
+    enum class TileUse
+    {
+        Any,
+        Blocked,
+        Large
+    };
     int launchGemmBlocked(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream,
-                          bool forceLargeTile = false);
+                          TileUse use);
     // one translation unit per element type
-    int launchGemmBlockedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
-    int launchGemmBlockedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
-    int launchGemmBlockedI8(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
-    int launchGemmBlockedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile);
+    int launchGemmBlockedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use);
+    int launchGemmBlockedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use);
+    int launchGemmBlockedI8(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use);
+    int launchGemmBlockedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use);
     int launchGemmBlockedF32(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
     int launchGemmFusedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
     int launchGemmFusedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);

@@ -106,23 +106,23 @@ namespace rocwmma_amd
     }
 
     int launchGemmBlocked(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream,
-                          bool forceLargeTile)
+                          TileUse use)
     {
         if(g.layoutC != ROCWMMA_AMD_ROW_MAJOR)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE; // caller transposes the problem first
         switch(dtypeIn)
         {
         case ROCWMMA_AMD_F16:
-            return launchGemmBlockedF16(dtypeOut, layoutA, layoutB, g, stream, forceLargeTile);
+            return launchGemmBlockedF16(dtypeOut, layoutA, layoutB, g, stream, use);
         case ROCWMMA_AMD_BF16:
-            return launchGemmBlockedBf16(dtypeOut, layoutA, layoutB, g, stream, forceLargeTile);
+            return launchGemmBlockedBf16(dtypeOut, layoutA, layoutB, g, stream, use);
         case ROCWMMA_AMD_I8:
-            return launchGemmBlockedI8(dtypeOut, layoutA, layoutB, g, stream, forceLargeTile);
+            return launchGemmBlockedI8(dtypeOut, layoutA, layoutB, g, stream, use);
         case ROCWMMA_AMD_E4M3:
         case ROCWMMA_AMD_E5M2:
-            return launchGemmBlockedFp8(dtypeIn, dtypeOut, layoutA, layoutB, g, stream, forceLargeTile);
+            return launchGemmBlockedFp8(dtypeIn, dtypeOut, layoutA, layoutB, g, stream, use);
         case ROCWMMA_AMD_F32:
-            return forceLargeTile ? ROCWMMA_AMD_UNSUPPORTED_TYPE : launchGemmBlockedF32(dtypeOut, layoutA, layoutB, g, stream);
+            return use == TileUse::Large ? ROCWMMA_AMD_UNSUPPORTED_TYPE : launchGemmBlockedF32(dtypeOut, layoutA, layoutB, g, stream);
         default:
             return ROCWMMA_AMD_UNSUPPORTED_TYPE;
         }

@@ -5,12 +5,12 @@ using namespace rocwmma;
 
 namespace rocwmma_amd
 {
-    int launchGemmBlockedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile)
+    int launchGemmBlockedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use)
     {
         if(dtypeOut == ROCWMMA_AMD_F32)
-            return pickLayout<bfloat16_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<bfloat16_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, use);
         if(dtypeOut == ROCWMMA_AMD_BF16)
-            return pickLayout<bfloat16_t, bfloat16_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<bfloat16_t, bfloat16_t, float32_t, false>(layoutA, layoutB, g, stream, use);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 

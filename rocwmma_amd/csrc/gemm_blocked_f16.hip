@@ -5,12 +5,12 @@ using namespace rocwmma;
 
 namespace rocwmma_amd
 {
-    int launchGemmBlockedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile)
+    int launchGemmBlockedF16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use)
     {
         if(dtypeOut == ROCWMMA_AMD_F32)
-            return pickLayout<float16_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<float16_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, use);
         if(dtypeOut == ROCWMMA_AMD_F16)
-            return pickLayout<float16_t, float16_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<float16_t, float16_t, float32_t, false>(layoutA, layoutB, g, stream, use);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 

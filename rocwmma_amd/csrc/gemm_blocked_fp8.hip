@@ -6,12 +6,12 @@ using namespace rocwmma;
 namespace rocwmma_amd
 {
     int launchGemmBlockedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream,
-                             bool forceLargeTile)
+                             TileUse use)
     {
         if(dtypeIn == ROCWMMA_AMD_E4M3 && dtypeOut == ROCWMMA_AMD_F32)
-            return pickLayout<float8_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<float8_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, use);
         if(dtypeIn == ROCWMMA_AMD_E5M2 && dtypeOut == ROCWMMA_AMD_F32)
-            return pickLayout<bfloat8_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<bfloat8_t, float32_t, float32_t, false>(layoutA, layoutB, g, stream, use);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 

@@ -5,12 +5,12 @@ using namespace rocwmma;
 
 namespace rocwmma_amd
 {
-    int launchGemmBlockedI8(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, bool forceLargeTile)
+    int launchGemmBlockedI8(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream, TileUse use)
     {
         if(dtypeOut == ROCWMMA_AMD_I32)
-            return pickLayout<int8_t, int32_t, int32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<int8_t, int32_t, int32_t, false>(layoutA, layoutB, g, stream, use);
         if(dtypeOut == ROCWMMA_AMD_I8)
-            return pickLayout<int8_t, int8_t, int32_t, false>(layoutA, layoutB, g, stream, forceLargeTile);
+            return pickLayout<int8_t, int8_t, int32_t, false>(layoutA, layoutB, g, stream, use);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 

@@ -8,9 +8,9 @@ namespace rocwmma_amd
     int launchGemmFusedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream)
     {
         if(dtypeOut == ROCWMMA_AMD_F32)
-            return pickLayout<bfloat16_t, float32_t, float32_t, true>(layoutA, layoutB, g, stream, false);
+            return pickLayout<bfloat16_t, float32_t, float32_t, true>(layoutA, layoutB, g, stream, TileUse::Any);
         if(dtypeOut == ROCWMMA_AMD_BF16)
-            return pickLayout<bfloat16_t, bfloat16_t, float32_t, true>(layoutA, layoutB, g, stream, false);
+            return pickLayout<bfloat16_t, bfloat16_t, float32_t, true>(layoutA, layoutB, g, stream, TileUse::Any);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 
