@@ -597,19 +597,13 @@ int rocwmma_amd_gemv(uint32_t    m,
     return launchGemv(m, k, ncols, a, lda, x, ldx, y, ldy, alpha, beta, asStream(stream));
 }
 
-// Whether a width is one of those every kernel takes, whatever the element type and row count (up to 128).
-static bool dlrmCommonWidth(uint32_t m, uint32_t k)
-{
-    return m <= 128u && (k == 32u || k == 64u || k == 128u || k == 256u);
-}
-
 static int checkDlrm(int dtype, uint32_t m, uint32_t k, uint32_t batch)
 {
     if(m == 0u || k == 0u || batch == 0u)
         return ROCWMMA_AMD_INVALID_ARGUMENT;
     // the tiled kernels read rows in 16-byte pieces and address a sample's features with 32-bit byte offsets
     const uint32_t size = dtype == ROCWMMA_AMD_F16 ? 2u : 4u;
-    if(!dlrmCommonWidth(m, k) && (m > 32768u || k % (16u / size) != 0u || static_cast<uint64_t>(m) * k * size >= (1ull << 31)))
+    if(m > 32768u || k % (16u / size) != 0u || static_cast<uint64_t>(m) * k * size >= (1ull << 31))
         return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
     return ROCWMMA_AMD_OK;
 }

@@ -24,8 +24,9 @@
 //   grid (m/128, n/128)                          1-D grid, tiles dealt to XCDs in L2-friendly patches
 //                                                (9 % faster than the plain order at 8192^3)
 //
-// The smaller configurations (128 x 128, 128 x 64, 64 x 64 tiles of 4 waves) come with a ring of four stages
-// of 64 bytes of K (copies three stages ahead), a ring of four stages of 128 bytes, or the ring of two.
+// The smaller configurations (256 x 128 tiles of 8 waves; 128 x 128, 128 x 64, 64 x 64 tiles of 4) come with rings of two, three
+// and four such stages, the ring of B perhaps a stage deeper than that of two of A, or with a ring of four stages of 64 bytes
+// (copies three stages ahead).
 //
 // Column-major C/D is handled by the caller as the transposed problem (D^T = B^T A^T).
 #ifndef ROCWMMA_AMD_CSRC_GEMM_BLOCKED_CORE_HPP
@@ -95,8 +96,8 @@ namespace rocwmma_amd
             static constexpr uint32_t WaveN   = BlocksN * Block;
             static constexpr uint32_t MacroM  = WavesM * WaveM;
             static constexpr uint32_t MacroN  = WavesN * WaveN;
-            // bytes of K per pipeline stage: 64 in the ring of four, 128 (whole lines of a K-contiguous
-            // operand) in the ring of two
+            // bytes of K per pipeline stage: 128 (whole lines of a K-contiguous operand), 64 in the ring of four that does not say
+            // otherwise
             static constexpr uint32_t StageKB = StageKB_ != 0u ? StageKB_ : (Stages_ == 4u ? 64u : 128u);
             static constexpr uint32_t MacroK  = StageKB / sizeof(InT); // K elements per stage
 
@@ -130,9 +131,8 @@ namespace rocwmma_amd
             static constexpr uint32_t Stages     = Stages_; // ring of K stages in LDS
             static constexpr uint32_t WavesPerSimd = WavesPerSimd_;
             static constexpr uint32_t StagesB = Stages_ + (ExtraB_ ? 1u : 0u);
-            // LDS: stage by stage, A in front of B (one address serves both operands: with the rings of A and B apart the kernels
-            // on the ring of two needed more registers, the stream-K kernel of int8 spilled a third more and took 115.8 -> 131.9 us
-            // at 2560 x 2560 x 8192); with an extra B stage the ring of A, then the ring of B
+            // LDS: stage by stage, A in front of B (one address serves both operands); with an extra B stage the ring of A, then the
+            // ring of B
             static constexpr uint32_t StrideA = ExtraB_ ? BytesA : StageBytes;
             static constexpr uint32_t StrideB = ExtraB_ ? BytesB : StageBytes;
             static constexpr uint32_t FirstB  = ExtraB_ ? Stages * BytesA : BytesA;
@@ -500,7 +500,8 @@ namespace rocwmma_amd
 
         // Main loop schedules (per wave), by ring:
         //
-        //   ring of two stages of 128 bytes of K (the 256 x 256 tile; N = 2 or 4 MFMA steps per stage):
+        //   ring of two stages of 128 bytes of K (the 256 x 256 tile; N = 2 or 4 MFMA steps per stage), of three or with B a stage
+        //   deeper (copies one stage further ahead, and left in flight at the wait):
         //     prologue : copies of stages 0 and 1 in flight; wait for stage 0; barrier; read F(0, step 0)
         //     stage i  : steps 0 .. N-2: read the next step's fragments while this step's MFMAs run
         //                wait: stage i+1 landed and own LDS reads returned;  barrier
@@ -971,9 +972,10 @@ namespace rocwmma_amd
                 lds::waitCopiesAndReads<0u>(); // the surplus copies still target this workgroup's LDS
                 lds::barrier();
             }
-            else if constexpr(S == 2u || S == 3u || (S == 5u && Cfg::StageKB == 128u))
+            else if constexpr(S == 2u || S == 3u)
             {
-                // Ring of two stages of 128 bytes of K (two or four MFMA steps each).  A phase multiplies
+                // Ring of two or three stages of 128 bytes of K (two or four MFMA steps each), the ring of B perhaps a stage
+                // deeper.  A phase multiplies
                 // one step while it reads the fragments of the next; the barrier in front of a stage's
                 // last phase is where stage i has been read completely and stage i+1 has landed, so
                 // the copies of stage i+2 go out right behind it, into stage i's slot, and have the
@@ -1247,52 +1249,22 @@ namespace rocwmma_amd
             }
             else
             {
-                // One MFMA step per stage (wide fp8): a phase multiplies stage s (fragments read
+                // One MFMA step per stage (fp8 in 64-byte stages): a phase multiplies stage s (fragments read
                 // during the previous phase) while it reads the fragments of stage s+1 and issues
                 // the copies of stage s+3; the wait + barrier closing the phase makes stage s+2
                 // visible.  Two phases per loop trip so the fragment sets swap without copies.
                 // Every phase issues a stage, so the loop body and its wait counts are uniform:
                 // past the end of K the last stage is copied again into a ring slot nobody reads.
-                static_assert(Cfg::KSteps == 1u, "one MFMA step per stage");
+                static_assert(S == 4u && Cfg::KSteps == 1u, "ring of four, one MFMA step per stage");
                 Frags f0, f1;
-                // Transposing LDS reads are inline assembly, which the scheduling hints cannot
-                // place: with a dim-major B (two such reads for each of its 8 blocks) the phase is laid
-                // out by hand, one column of blocks at a time (the reads of that column of the next
-                // stage, then its MFMAs): 5 % faster than leaving the reads in front of the MFMAs.  With
-                // only A dim-major (4 blocks) the compiler's placement is 1 % better and is kept.
-                auto phaseByColumns = [&](Frags const& cur, Frags& nxt, uint32_t slot) {
-                    const char* ldsA = ldsRaw + slot * Cfg::StrideA;
-                    const char* ldsB = ldsRaw + Cfg::FirstB + slot * Cfg::StrideB;
-                    if constexpr(Cfg::Block == 16u)
-                    {
-                        static_assert(Cfg::BlocksM <= Cfg::BlocksN, "the A blocks are read along with the first B columns");
-#pragma unroll
-                        for(uint32_t j = 0; j < Cfg::BlocksN; ++j)
-                        {
-                            TileB::template readBlock16<Cfg::KPackBytes>(nxt.b[j].x, ldsB, waveN * Cfg::WaveN + j * Cfg::Block, 0u, lane);
-                            if(j < Cfg::BlocksM)
-                                TileA::template readBlock16<Cfg::KPackBytes>(nxt.a[j].x, ldsA, waveM * Cfg::WaveM + j * Cfg::Block, 0u, lane);
-#pragma unroll
-                            for(uint32_t i = 0; i < Cfg::BlocksM; ++i)
-                                mma_sync(acc[i][j], cur.a[i], cur.b[j], acc[i][j]);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
-                };
-#define ROCWMMA_AMD_PHASE(STAGE, CUR, NXT, READ)                                                         \
+#define ROCWMMA_AMD_PHASE(STAGE, CUR, NXT)                                                               \
     do                                                                                                  \
     {                                                                                                   \
         issueStage(((STAGE) + S - 1u) % S, (STAGE) + S < stages);                                       \
-        if constexpr(Cfg::BKMajor || Cfg::Block != 16u)                                                 \
-        {                                                                                               \
-            if(READ)                                                                                    \
-                readFrags(NXT, ((STAGE) + 1u) % S, 0u);                                                 \
-            multiply(CUR);                                                                              \
-            scheduleInterleaved<Cfg::MfmasPerStep / 2u, Cfg::ReadsPerStep, 0u>();                       \
-            scheduleInterleaved<Cfg::MfmasPerStep - Cfg::MfmasPerStep / 2u, 0u, Cfg::Copies>();         \
-        }                                                                                               \
-        else                                                                                            \
-            phaseByColumns(CUR, NXT, ((STAGE) + 1u) % S);                                               \
+        readFrags(NXT, ((STAGE) + 1u) % S, 0u);                                                         \
+        multiply(CUR);                                                                                  \
+        scheduleInterleaved<Cfg::MfmasPerStep / 2u, Cfg::ReadsPerStep, 0u>();                           \
+        scheduleInterleaved<Cfg::MfmasPerStep - Cfg::MfmasPerStep / 2u, 0u, Cfg::Copies>();             \
         __builtin_amdgcn_sched_barrier(0);                                                              \
         lds::waitCopiesAndReads<(S - 3u) * Cfg::Copies>();                                              \
         pinFrags(NXT);                                                                                  \
@@ -1315,10 +1287,10 @@ namespace rocwmma_amd
                 uint32_t s = 0;
                 for(; s + 1u < stages; s += 2u)
                 {
-                    ROCWMMA_AMD_PHASE(s, f0, f1, true);
+                    ROCWMMA_AMD_PHASE(s, f0, f1);
                     // (past the last stage this reads a ring slot whose content nobody multiplies:
                     // an unconditional phase body keeps the instruction interleave intact)
-                    ROCWMMA_AMD_PHASE(s + 1u, f1, f0, true);
+                    ROCWMMA_AMD_PHASE(s + 1u, f1, f0);
                 }
                 if(s < stages)
                     multiply(f0);
