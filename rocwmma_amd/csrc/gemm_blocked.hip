@@ -26,6 +26,13 @@ namespace rocwmma_amd
 
     namespace
     {
+        // One round of 128 x 64 tiles, more than a quarter full, with at least 4 KiB of K per row.
+        bool mxTakesLineTiles(GemmArgs const& g)
+        {
+            const uint32_t tiles = ceilDiv(g.m, 128u) * ceilDiv(g.n, 64u);
+            return g.k % 128u == 0u && g.k >= 4096u && tiles <= computeUnits() && 4u * tiles > computeUnits();
+        }
+
         // Raw: the scales in the caller's order (MxPacked)
         template <typename InT, bool Raw>
         int launchMxMid(GemmArgs const& g, TileExtras const& ex, hipStream_t stream)
@@ -36,11 +43,10 @@ namespace rocwmma_amd
             // at most one 128 x 128 tile per two compute units (few token rows against a wide weight matrix):
             // 128 x 64 tiles put twice as many workgroups to work
             using Narrow = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 2, 3, 32, true, true, false, 0, false, Raw>;
-            // One round of 128 x 64 tiles with at least 4 KiB of K per row: the tile on the ring of four 128-byte
-            // stages (whole-line requests, three stages in flight), as for the unscaled types (the ladder's
-            // NarrowLines): 128 x 14336 x 4096 31 -> 21 us on scales packed beforehand.
+            // mxTakesLineTiles: the tile on the ring of four 128-byte stages (whole-line requests, three stages in flight), as the
+            // unscaled types' rung of that name: 128 x 14336 x 4096 31 -> 21 us on scales packed beforehand.
             using NarrowLines = BlockedConfig<InT, float32_t, float32_t, true, true, 2, 2, 2, 1, 4, 1, 32, true, true, false, 128, false, Raw>;
-            if(gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u))
+            if(mxTakesLineTiles(g))
             {
                 const int rc = launchCfg<NarrowLines>(g, stream, ex);
                 if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
@@ -51,14 +57,6 @@ namespace rocwmma_amd
             return launchCfg<Mid>(g, stream, ex);
         }
     } // namespace
-
-    bool gemmBlockedTakesPartlyFilledLineTiles(uint32_t m, uint32_t n, uint32_t k, uint32_t elemBytes)
-    {
-        const uint32_t tiles  = ceilDiv(m, 128u) * ceilDiv(n, 64u);
-        const size_t   kBytes = static_cast<size_t>(k) * elemBytes;
-        const size_t   minK   = (elemBytes == 2u && m <= 64u) ? 16384u : 4096u;
-        return kBytes % 128u == 0u && kBytes >= minK && tiles <= computeUnits() && 4u * tiles > computeUnits();
-    }
 
     bool gemmMxBlockedUsesLargeTile(GemmArgs const& g)
     {
@@ -91,7 +89,7 @@ namespace rocwmma_amd
         // 14336 68.6 -> 71.1.  On the ring of two: 384 x 7168 x 2048 24.4 -> 20.9, 1024 x 1200 x 1408 14.0 -> 12.1, but 128 x 1024 x
         // 8192 52 -> 57; with more tiles than units 4096 x 1200 x 1408 24.4 -> 21.1, 512 x 14336 x 4096 57 -> 75.
         const uint32_t units = computeUnits(), stages = g.k / 128u, tiles = ceilDiv(g.m, 128u) * ceilDiv(g.n, 128u);
-        const bool     raw   = gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, 1u) ? stages <= (g.m <= 96u ? 64u : 44u)
+        const bool     raw   = mxTakesLineTiles(g) ? stages <= (g.m <= 96u ? 64u : 44u)
                                : tiles <= units ? stages <= 30u
                                                 : static_cast<uint64_t>(stages) * ceilDiv(tiles, 2u * units) <= 12u;
         if(!raw)

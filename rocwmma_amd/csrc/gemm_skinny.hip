@@ -499,13 +499,20 @@ namespace rocwmma_amd
             // (n: the kernel that initialises D counts 4-element groups in 32 bits)
             if(g.m % 16u != 0u || g.m >= kSlicedMaxM || g.n % 16u != 0u || g.n > (1u << 24) || (g.k * E) % 1024u != 0u)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            // From 64 rows on the blocked kernel is as fast or faster, in one launch and without atomic adds
-            // (its 64 x 64 tiles at 64 rows: 21 against 21 us; its partly filled 128 x 128 tiles at 80, 96,
-            // 112 rows of int8 against 14336 x 4096: 25.5, 25.4, 26.4 us against 26.8, 29.0, 32.3 us here);
-            // 48 rows stayed (20.8 against 24.6 us) until the blocked kernel got partly filled 128 x 64 tiles on
-            // whole-line stages: where it runs those (one round of workgroups, 4 KiB of K and more) it takes 48
-            // rows as well, 17.7 / 16.9 us int8 / fp8 against 20.9 / 22.5 us here.
-            if(g.m >= 64u || gemmBlockedTakesPartlyFilledLineTiles(g.m, g.n, g.k, E))
+            // From 64 rows on the blocked kernel is as fast or faster, in one launch and without atomic adds.  Below, K is what decides,
+            // alike for 8- and 16-bit types: the blocked kernel has one workgroup walk all of K (about 2.4 us per KiB of it), here
+            // the second launch and the atomic adds of every slice (more with more columns) come on top of the weights.  48 rows,
+            // n columns, int8, blocked / here in us:
+            //     K bytes     n = 256      4096         7168         8192         14336        28672
+            //        4096   11.7 / 13.6  11.9 / 14.8  15.0 / 17.5  15.4 / 18.0  17.4 / 22.6  29.7 / 32.6
+            //        6144   16.2 / 14.0  19.5 / 16.7  20.9 / 19.8  21.1 / 20.9  23.1 / 32.1  39.0 / 55.6
+            //        8192   20.5 / 13.6  25.3 / 18.1  26.5 / 22.5  27.0 / 24.7  31.2 / 32.0  51.8 / 59.6
+            //       28672   64.2 / 14.2  81.1 / 32.2  85.6 / 57.4  87.7 / 60.7
+            // (float16 with 6144 bytes and n = 7168, 8192: 48 rows 20.8 / 21.1, 21.2 / 22.4; 32 rows, fewer adds, 20.4 / 18.2, 20.6 / 19.3.)
+            const uint64_t kBytes    = static_cast<uint64_t>(g.k) * E;
+            const uint64_t perUnit   = kBytes / (g.m > 32u ? 256u : 192u); // columns
+            const bool     fewerAdds = g.n <= computeUnits() * (perUnit < 32u ? perUnit : 32u);
+            if(g.m >= 64u || kBytes <= 4096u || !fewerAdds)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
             // K slices: whole 1 KiB copies per row and whole batches of fragment steps per slice, the
             // A slice within 128 KiB of LDS; as few slices as fill the compute units
