@@ -62,7 +62,7 @@ def check(dtype_in, dtype_out, got, want, tol):
 @pytest.mark.parametrize("dtype_in,dtype_out,tol", [
     (orc.F16, orc.F16, 1e-3),    # <f16, f16, f32>
     (orc.BF16, orc.BF16, 4e-3),  # <bf16, bf16, f32>: one bf16 ulp (2^-8) of a value v costs v/(2v+1) * 2^-8 <= 2e-3
-    (orc.F32, orc.F32, 1e-5),    # <f32, f32, f32> (wave-tile kernel only)
+    (orc.F32, orc.F32, 1e-5),    # <f32, f32, f32> (here one block per wave)
 ])
 @pytest.mark.parametrize("beta", [-0.5, 0.0])
 def test_narrow_output_and_f32_type_combinations(dtype_in, dtype_out, tol, la, lb, algo, beta):

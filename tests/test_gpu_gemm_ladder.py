@@ -1,5 +1,6 @@
-"""The blocked GEMM's tile ladder on sizes that fill neither tiles nor K stages: every rung, K shorter than the
-pipeline's prologue and ending inside a stage, all element types, plain and with the fused epilogue.
+"""The blocked GEMM on sizes that fill neither tiles nor K stages, one block to the largest tiles: K shorter than the
+pipeline's prologue and ending inside a stage, all element types, plain and with the fused epilogue.  (Which of the tiles and
+pipelines a size runs on is for the cost table to say; tests/test_gpu_gemm_rungs.py reaches every one of them by name.)
 
 Operands are padded (leading dimensions and further K rows) with NaN (int8: 99), so a copy that reads past the
 end of K or lets a padded byte into a sum shows in the result; D is framed by a guard.  The oracle sees the same bits
@@ -92,7 +93,7 @@ def test_partly_filled_tiles_and_stages(dtype_in, dtype_out, m, n, k, la, lb):
         compare(dtype_in, dtype_out, frame, dev, want, tol)
 
 
-@pytest.mark.parametrize("la,lb", [(RM, CM), (CM, RM)])
+@pytest.mark.parametrize("la,lb", PAIRS)
 @pytest.mark.parametrize("m,n,k", SHAPES)
 @pytest.mark.parametrize("dtype_in,dtype_out", [(orc.F16, orc.F16), (orc.BF16, orc.F32), (orc.E4M3, orc.F32)])
 def test_fused_epilogue_on_every_rung(dtype_in, dtype_out, m, n, k, la, lb):
