@@ -56,11 +56,12 @@ namespace rocwmma_amd
     //     start + alone * kKB + write * outBytes                   (one tile at a time: its copies' latency shows)
     // and with L tiles for the busiest unit
     //     start + L * (shared * kKB + writeShared * outBytes),
-    // kKB = thousands of bytes of K per row, outBytes = bytes per element of D.
+    // kKB = thousands of bytes of K per row, outBytes = bytes per element of D; `edges` times the terms of K where tiles or stages
+    // are partly filled (bounds on every copy, rows that begin off a line).
     struct RungCost
     {
         Rung  rung;
-        float start, alone, write, shared, writeShared;
+        float start, alone, write, shared, writeShared, edges;
     };
     // One block per wave, blocks of 16 (m or n no multiple of 32) or 32:
     //     start + steps * kKB + waves * (fetch * kKB + store * outBytes),     waves in thousands.
@@ -122,8 +123,21 @@ namespace rocwmma_amd
         }
     }
 
-    constexpr float rungTime(RungCost const& c, uint32_t pair, uint32_t m, uint32_t n, float kKB, float outBytes, uint32_t units)
+    // Whether the problem is whole tiles and stages, and long enough for the ring.
+    constexpr bool fillsTiles(Rung rung, uint32_t pair, uint32_t m, uint32_t n, uint64_t kBytes)
     {
+        const bool     half  = rung == Rung::Ring4 || rung == Rung::Narrow64 || rung == Rung::Tiny64;
+        const uint32_t stage = half ? 64u : 128u;
+        const uint32_t ahead = half || rung == Rung::MidLines || rung == Rung::NarrowLines || rung == Rung::Tiny ? 3u
+                               : rung == Rung::Wide || rung == Rung::Narrow                                      ? 2u
+                                                                                                                 : 1u;
+        return m % tileRows(rung, pair) == 0u && n % tileCols(rung, pair) == 0u && kBytes % stage == 0u && kBytes >= ahead * stage;
+    }
+
+    constexpr float rungTime(RungCost const& c, uint32_t pair, uint32_t m, uint32_t n, float kKB, float outBytes, uint32_t units, bool edges)
+    {
+        if(edges)
+            kKB *= c.edges;
         const uint32_t rows = tileRows(c.rung, pair), cols = tileCols(c.rung, pair);
         const uint64_t tiles = (static_cast<uint64_t>(m) + rows - 1u) / rows * ((static_cast<uint64_t>(n) + cols - 1u) / cols);
         if(tiles <= units)
@@ -143,7 +157,7 @@ namespace rocwmma_amd
         return c.start + c.steps * kKB + waves * (c.fetch * kKB + c.store * outBytes);
     }
 
-    // The rung with the least estimated time.
+    // The rung with the least estimated time.  waveTile: one block per wave may be chosen.
     constexpr Rung cheapestRung(OperandKind kind, uint32_t pair, uint32_t m, uint32_t n, uint64_t kBytes, uint32_t outBytes, uint32_t units,
                                 bool waveTile)
     {
@@ -153,10 +167,11 @@ namespace rocwmma_amd
         float            time = 0.0f;
         for(uint32_t i = 0; i < kMaxRungs && table.rungs[i].rung != Rung::None; ++i)
         {
-            const float t = rungTime(table.rungs[i], pair, m, n, kKB, out, units);
+            const Rung  rung = table.rungs[i].rung;
+            const float t    = rungTime(table.rungs[i], pair, m, n, kKB, out, units, !fillsTiles(rung, pair, m, n, kBytes));
             if(best == Rung::None || t < time)
             {
-                best = table.rungs[i].rung;
+                best = rung;
                 time = t;
             }
         }

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 PAIRS = [(RM, CM), (RM, RM), (CM, CM), (CM, RM)]
 TYPES = {(0, 4): [(orc.F16, orc.F32), (orc.BF16, orc.F32), (orc.F16, orc.F16), (orc.BF16, orc.BF16)], (1, 4): [(orc.I8, orc.I32), (orc.I8, orc.I8)],
-         (1, 1): [(orc.I8, orc.I8)], (2, 4): [(orc.E4M3, orc.F32), (orc.E5M2, orc.F32)]}
+         (0, 2): [(orc.F16, orc.F16), (orc.BF16, orc.BF16)], (1, 1): [(orc.I8, orc.I8)], (2, 4): [(orc.E4M3, orc.F32), (orc.E5M2, orc.F32)]}
 
 
 def torch_type(dtype):
