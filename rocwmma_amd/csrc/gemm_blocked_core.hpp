@@ -1575,7 +1575,7 @@ namespace rocwmma_amd
                             const BiasOfBlock bv = biasOf(bj);
 #pragma unroll
                             for(uint32_t e = 0; e < io.num_elements; ++e)
-                                io.x[e] = static_cast<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
+                                io.x[e] = narrowed<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
                             if constexpr(!PairIO)
                                 storeBlock(bi, bj, io);
                             else if(bj % 2u == 1u)
@@ -1613,7 +1613,7 @@ namespace rocwmma_amd
                         const BiasOfBlock bv = biasOf(bj);
 #pragma unroll
                         for(uint32_t e = 0; e < io.num_elements; ++e)
-                            io.x[e] = static_cast<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
+                            io.x[e] = narrowed<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
                     }
                     if constexpr(PairIO)
                     {
@@ -1667,7 +1667,7 @@ namespace rocwmma_amd
                             const BiasOfBlock bv = biasOf(bj);
 #pragma unroll
                             for(uint32_t e = 0; e < fd[bj].num_elements; ++e)
-                                fd[bj].x[e] = static_cast<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e]));
+                                fd[bj].x[e] = narrowed<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e]));
                         }
                         if constexpr(PairIO)
                         {

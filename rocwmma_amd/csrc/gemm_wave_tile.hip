@@ -98,13 +98,13 @@ namespace rocwmma_amd
                 load_matrix_sync(fc, c + cOff, ldc, layoutC);
 #pragma unroll
                 for(uint32_t i = 0; i < fc.num_elements; ++i)
-                    fc.x[i] = static_cast<OutT>(finish(i, alpha * acc.x[i] + beta * static_cast<CompT>(fc.x[i])));
+                    fc.x[i] = narrowed<OutT>(finish(i, alpha * acc.x[i] + beta * static_cast<CompT>(fc.x[i])));
             }
             else
             {
 #pragma unroll
                 for(uint32_t i = 0; i < fc.num_elements; ++i)
-                    fc.x[i] = static_cast<OutT>(finish(i, alpha * acc.x[i]));
+                    fc.x[i] = narrowed<OutT>(finish(i, alpha * acc.x[i]));
             }
             store_matrix_sync(d + dOff, fc, ldd, layoutC);
         }
