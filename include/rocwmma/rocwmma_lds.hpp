@@ -310,15 +310,14 @@ namespace rocwmma
                 const uint32_t seg   = (dim0 >> 4) + (group & 1u);
                 const uint32_t kBase = ks * 16u + (group >> 1) * 8u + (s >> 2);
                 const uint32_t inSeg = (s & 3u) << 3; // 4 elements = 8 bytes per source lane
-#pragma unroll
-                for(uint32_t kk = 0; kk < 2u; ++kk)
-                {
-                    const uint32_t k    = kBase + kk * 4u;
-                    const uint32_t addr = ldsBase + offset(k, seg) + inSeg;
-                    s16x4          v;
-                    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v) : "v"(addr) : "memory");
-                    reinterpret_cast<s16x4*>(regs)[kk] = v;
-                }
+                // (the second four K rows: kBase has bit 2 clear and swz does not look at it, so they are a constant away.  With an address
+                // of its own every read had a vector instruction in front: 1280 x 1280 x 2048 f16, both dim-major, 24.5 -> 21.8 us)
+                const uint32_t addr = ldsBase + offset(kBase, seg) + inSeg;
+                s16x4          v0, v1;
+                asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v0) : "v"(addr) : "memory");
+                asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v1) : "v"(addr), "n"(4u * rowBytes) : "memory");
+                reinterpret_cast<s16x4*>(regs)[0] = v0;
+                reinterpret_cast<s16x4*>(regs)[1] = v1;
             }
 
             // Operand of one 16-wide MFMA block with 8 K values per lane (v_mfma_*_16x16x32):
@@ -336,15 +335,13 @@ namespace rocwmma
                 const uint32_t seg     = dim0 >> 4;
                 const uint32_t kBase   = ks * 32u + group * 8u + (s >> 2);
                 const uint32_t inSeg   = (s & 3u) << 3;
-#pragma unroll
-                for(uint32_t kk = 0; kk < 2u; ++kk)
-                {
-                    const uint32_t k    = kBase + kk * 4u;
-                    const uint32_t addr = ldsBase + offset(k, seg) + inSeg;
-                    s16x4          v;
-                    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v) : "v"(addr) : "memory");
-                    reinterpret_cast<s16x4*>(regs)[kk] = v;
-                }
+                // (the second four K rows: kBase has bit 2 clear and swz does not look at it, so they are a constant away)
+                const uint32_t addr = ldsBase + offset(kBase, seg) + inSeg;
+                s16x4          v0, v1;
+                asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(v0) : "v"(addr) : "memory");
+                asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(v1) : "v"(addr), "n"(4u * rowBytes) : "memory");
+                reinterpret_cast<s16x4*>(regs)[0] = v0;
+                reinterpret_cast<s16x4*>(regs)[1] = v1;
             }
         };
 
@@ -421,6 +418,20 @@ namespace rocwmma
                 out[0] = v[0];
                 out[1] = v[1];
             }
+            // Two of them: the lane's group reads K rows k0 .. k0 + 15 (k0 a multiple of 16) of the 16 elements that
+            // start at dim16 (a multiple of 16); the lane receives element dim16 + lane % 16.  (swz does not look at bit 3 of
+            // the K row: the second read is a constant away.)
+            ROCWMMA_DEVICE static ROCWMMA_INLINE void read16(uint32_t* out, uint32_t ldsBase, uint32_t k0, uint32_t dim16, uint32_t lane)
+            {
+                typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+                const uint32_t s    = lane & 15u;
+                const uint32_t addr = ldsBase + offset(k0 + (s >> 1), dim16 >> 4) + ((s & 1u) << 3);
+                u32x2_t        v0, v1;
+                asm volatile("ds_read_b64_tr_b8 %0, %1" : "=v"(v0) : "v"(addr) : "memory");
+                asm volatile("ds_read_b64_tr_b8 %0, %1 offset:%2" : "=v"(v1) : "v"(addr), "n"(8u * rowBytes) : "memory");
+                reinterpret_cast<u32x2_t*>(out)[0] = v0;
+                reinterpret_cast<u32x2_t*>(out)[1] = v1;
+            }
 
             // Operand of one 16-wide MFMA block with 16 K values per lane (v_mfma_i32_16x16x64_i8):
             // lane l ends up with dim = dim0 + l % 16 and k = 64 ks + (l / 16) * 16 + 0..15.
@@ -431,10 +442,7 @@ namespace rocwmma
             {
                 static_assert(KPackBytes == 16u, "16-wide blocks of 8-bit types take 16 bytes of K per lane");
                 const uint32_t ldsBase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((LdsPtr)ldsTile));
-                const uint32_t kBase   = ks * 64u + (lane >> 4) * 16u;
-#pragma unroll
-                for(uint32_t kk = 0; kk < 2u; ++kk)
-                    read8(reinterpret_cast<uint32_t(*)[2]>(regs)[kk], ldsBase, kBase + 8u * kk, dim0, lane);
+                read16(reinterpret_cast<uint32_t*>(regs), ldsBase, ks * 64u + (lane >> 4) * 16u, dim0, lane);
             }
 
             // Operand of one 32-wide MFMA block: lane l ends up with dim = dim0 + l % 32 and
