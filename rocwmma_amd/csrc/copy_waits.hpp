@@ -12,11 +12,13 @@
 
 namespace rocwmma_amd
 {
-    // C staged through two LDS buffers: `groups` groups of `copies` copies each, group g + 2 issued when group g has been
-    // read and its results have been stored.  In flight when group `group` must have landed: the next group's copies.
-    constexpr uint32_t stagedCInFlight(uint32_t group, uint32_t groups, uint32_t copies)
+    // C staged through `buffers` LDS buffers: `groups` groups of `copies` copies each, the first `buffers` of them issued at once,
+    // group g + buffers when group g has been read and its results have been stored.  In flight when group `group` must have
+    // landed: the copies of the groups issued behind it.
+    constexpr uint32_t stagedCInFlight(uint32_t group, uint32_t groups, uint32_t copies, uint32_t buffers = 2u)
     {
-        return group + 1u < groups ? copies : 0u;
+        const uint32_t behind = groups - 1u - group;
+        return (behind < buffers - 1u ? behind : buffers - 1u) * copies;
     }
 } // namespace rocwmma_amd
 

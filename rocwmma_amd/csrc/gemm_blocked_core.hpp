@@ -150,6 +150,9 @@ namespace rocwmma_amd
             // from transposing reads) is left as it was: 5 % slower with one issuer.  So are the kernels with
             // block scales: their main loop loads scales into registers, and behind a branch that only some
             // waves take the compiler waits for every copy in flight before it uses them (five times slower).
+            // Wave tiles of 128 rows, one wave per SIMD (the loop is at Cfg::WideWave below): the accumulators take 256 registers, so they
+            // live in the accumulation half of the register file.
+            static constexpr bool     WideWave = WavesPerSimd_ == 1u && BlocksM_ == 8u && BlockEdge_ == 16u && Stages_ == 2u && StagesB == 3u;
             static constexpr uint32_t CopyWaves
                 = (Waves == 8u && WavesPerSimd_ == 2u && (Stages_ == 2u || Stages_ == 3u) && (AKMajor || BKMajor) && !Scaled_) ? 4u : Waves;
             // LDS read instructions per MFMA step: b128 reads per block (K-major) or two transposing b64 reads
@@ -159,12 +162,16 @@ namespace rocwmma_amd
             static constexpr uint32_t ReadsPerStep = ReadsA + ReadsB;
             static constexpr uint32_t MfmasPerStep = BlocksM * BlocksN;
             // beta * C operand staged through LDS in the epilogue, in groups of Block rows by
-            // GroupBlocks blocks (256- or 512-byte rows), two group buffers per wave
+            // GroupBlocks blocks (256- or 512-byte rows)
             static constexpr uint32_t GroupBlocks
                 = (WaveN == 128u && 2u * Block * 128u * sizeof(OutT) * Waves <= LdsBytes) ? 128u / Block : 64u / Block;
             static constexpr bool StagedC = sizeof(OutT) == 4u && WaveN % 64u == 0u
                                             && BlocksM * (BlocksN / GroupBlocks) >= 2u
                                             && 2u * Block * GroupBlocks * Block * sizeof(OutT) * Waves <= LdsBytes;
+
+            // group buffers per wave: four for wide waves, which are half as many (with two, 4096^3 bf16 with C took as long as with eight
+            // waves, 127.2 against 126.7 us; with four 122.1 against 128.1), two else
+            static constexpr uint32_t BuffersC = WideWave && 4u * Block * GroupBlocks * Block * sizeof(OutT) * Waves <= LdsBytes ? 4u : 2u;
 
             // C of the small tiles (at most 32 registers of it) is loaded in front of the main loop: behind it, the loads' latency
             // is a large part of a short problem (per call in a captured graph: 256^3 f16 4.0 -> 3.55 us, 512 x 1024 x 1024 e4m3
@@ -198,8 +205,13 @@ namespace rocwmma_amd
             // on the same K row modulo 16
             // (the 8-bit tile's looks at K row bit 4 as well, the float32 tile's at bit 2 only)
             static constexpr uint32_t SwizzleRows = sizeof(InT) == 4u ? 8u : (sizeof(InT) == 2u ? 16u : 32u);
-            static_assert((AKMajor || (Waves * TileA::rowsPerCopy) % SwizzleRows == 0u)
-                              && (BKMajor || (Waves * TileB::rowsPerCopy) % SwizzleRows == 0u),
+            // lane offsets that the copies of a wave take turns with, where its copies do not all start on the same K row modulo that
+            static constexpr uint32_t turns(bool kMajor, uint32_t rowsPerCopy)
+            {
+                return kMajor || (Waves * rowsPerCopy) % SwizzleRows == 0u ? 1u : SwizzleRows / (Waves * rowsPerCopy);
+            }
+            static constexpr uint32_t TurnsA = turns(AKMajor, TileA::rowsPerCopy), TurnsB = turns(BKMajor, TileB::rowsPerCopy);
+            static_assert(WideWave || (TurnsA == 1u && TurnsB == 1u),
                           "wave pool too small for the dim-major tile");
             // the K-major tile's swizzle looks at row bits 0..3 likewise
             static_assert((!AKMajor || (Waves * TileA::rowsPerCopy) % 16u == 0u)
@@ -800,10 +812,178 @@ namespace rocwmma_amd
                 __builtin_amdgcn_sched_barrier(0);
             }
 
+            // Wide waves: the accumulators while they are summed.  The epilogue takes them a row of blocks at a time (takeRow), so that
+            // only that row is in ordinary registers.
+            typedef CompT Result __attribute__((ext_vector_type(4)));
+            Result        sum[Cfg::WideWave ? Cfg::BlocksM : 1u][Cfg::WideWave ? Cfg::BlocksN : 1u];
+            auto          takeRow = [&](uint32_t bi) {
+                if constexpr(Cfg::WideWave)
+                {
+#pragma unroll
+                    for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+                    {
+                        asm volatile("" : "+a"(sum[bi][bj]));
+#pragma unroll
+                        for(uint32_t e = 0; e < 4u; ++e)
+                            acc[bi][bj].x[e] = sum[bi][bj][e];
+                    }
+                }
+                (void)bi;
+            };
+
             constexpr uint32_t S      = Cfg::Stages;
             // `stages` stages of K from stage0 on: >= S - 1 of them (checked by the host)
 
-            if constexpr(S == 2u && Cfg::KSteps == 1u)
+            if constexpr(Cfg::WideWave)
+            {
+                // Four waves of 128 x 128 (128 x 64 in half tiles), one per SIMD; A ring of two stages of 128 bytes, B ring of three.
+                // Against eight waves of 64 x 128 every LDS byte feeds a third more flops, nothing is issued twice and the copies are
+                // spread over the whole stage: those of B(i + 2) over its first step, those of A(i + 2) over the second, one to eight
+                // matrix instructions, so no wave ever queues behind them.  What bounds it is the power cap: 2290 clocks a stage
+                // without reads and copies, 2420 with (2048 of matrix work), 1.7 GHz on normally distributed data, 2.4 on zeros.
+                // 8192^3: bf16 both row-major 840 -> 780 us, f16 A row-major / B col-major 807 -> 762; 4096^3 112.7 -> 105.7, 109 -> 101.6.
+                // The matrix instructions are written in assembly: with the builtins the compiler moves all accumulators through
+                // ordinary registers once per stage (twice the time).  They go through the blocks in squares of 2 x 2, along and back, so
+                // that each shares an operand with the one before (row by row: 1.0-1.5 % slower under the power cap).
+                static_assert(Part == TilePart::Whole && std::is_same<Emit, Epilogue>::value && !Cfg::PrefetchC && Cfg::KSteps == 2u && Cfg::KPackBytes == 16u && Cfg::BlocksN % 2u == 0u, "wide waves: whole K ranges, two steps a stage");
+                constexpr uint32_t TurnsA = Cfg::TurnsA, TurnsB = Cfg::TurnsB;
+                uint32_t           aOff[TurnsA], bOff[TurnsB];
+#pragma unroll
+                for(uint32_t t = 0; t < TurnsA; ++t)
+                    aOff[t] = TileA::laneSourceOffset(lane, wave + t * Cfg::Waves, ldaB);
+#pragma unroll
+                for(uint32_t t = 0; t < TurnsB; ++t)
+                    bOff[t] = TileB::laneSourceOffset(lane, wave + t * Cfg::Waves, ldbB);
+                auto sourceA = [&] { return Cfg::Edges ? lds::makeSource(aSrc, aEnd) : lds::makeSource(aSrc); };
+                auto sourceB = [&] { return Cfg::Edges ? lds::makeSource(bSrc, bEnd) : lds::makeSource(bSrc); };
+                auto copyA = [&](uint32_t slot, uint32_t i, lds::BufferRsrc const& src) {
+                    const uint32_t copy = i * Cfg::Waves + wave;
+                    lds::asyncCopy16(ldsRaw + slot * Cfg::StrideA + copy * 1024u, src, insideK(Cfg::AKMajor, aOff[i % TurnsA], aLaneK, aLeft),
+                                     TileA::copySourceOffset(copy, ldaB));
+                };
+                auto copyB = [&](uint32_t slot, uint32_t i, lds::BufferRsrc const& src) {
+                    const uint32_t copy = i * Cfg::Waves + wave;
+                    lds::asyncCopy16(ldsRaw + Cfg::FirstB + slot * Cfg::StrideB + copy * 1024u, src, insideK(Cfg::BKMajor, bOff[i % TurnsB], bLaneK, bLeft),
+                                     TileB::copySourceOffset(copy, ldbB));
+                };
+                // (more == false: the last stage is copied again, into a slot nobody reads; edge tiles read nothing there)
+                auto advanceA = [&](bool more) {
+                    aSrc += Cfg::EdgesK || more ? aStep : size_t{0};
+                    if constexpr(Cfg::EdgesK)
+                        aLeft = aLeft > Cfg::MacroK ? aLeft - Cfg::MacroK : 0u;
+                };
+                auto advanceB = [&](bool more) {
+                    bSrc += Cfg::EdgesK || more ? bStep : size_t{0};
+                    if constexpr(Cfg::EdgesK)
+                        bLeft = bLeft > Cfg::MacroK ? bLeft - Cfg::MacroK : 0u;
+                };
+                typedef uint32_t Operand __attribute__((ext_vector_type(4)));
+                Operand          fa[2][Cfg::BlocksM], fb[2][Cfg::BlocksN];
+#pragma unroll
+                for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
+#pragma unroll
+                    for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+                        sum[bi][bj] = Result{0, 0, 0, 0};
+                constexpr uint32_t Reads = Cfg::BlocksM + Cfg::BlocksN, Mfmas = Cfg::BlocksM * Cfg::BlocksN;
+                // operand q of a step: the blocks of A, then those of B
+                auto readOperand = [&](uint32_t set, uint32_t slotA, uint32_t slotB, uint32_t ks, uint32_t q) {
+                    if(q < Cfg::BlocksM)
+                        TileA::template readBlock16<16u>(&fa[set][q], ldsRaw + slotA * Cfg::StrideA, waveM * Cfg::WaveM + q * 16u, ks, lane);
+                    else
+                        TileB::template readBlock16<16u>(&fb[set][q - Cfg::BlocksM], ldsRaw + Cfg::FirstB + slotB * Cfg::StrideB,
+                                                         waveN * Cfg::WaveN + (q - Cfg::BlocksM) * 16u, ks, lane);
+                };
+                auto pinSet = [&](uint32_t set) {
+#pragma unroll
+                    for(uint32_t q = 0; q < Cfg::BlocksM; ++q)
+                        lds::pinRegisters(fa[set][q]);
+#pragma unroll
+                    for(uint32_t q = 0; q < Cfg::BlocksN; ++q)
+                        lds::pinRegisters(fb[set][q]);
+                };
+                // (the accumulators are kept transposed: the instruction's first multiplicand is B)
+                auto multiplyBlock = [&](uint32_t set, uint32_t bi, uint32_t bj) {
+#if ROCWMMA_ARCH_GFX950
+                    if constexpr(std::is_same<InT, float16_t>::value)
+                        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(sum[bi][bj]) : "v"(fb[set][bj]), "v"(fa[set][bi]));
+                    else if constexpr(sizeof(InT) == 2u)
+                        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(sum[bi][bj]) : "v"(fb[set][bj]), "v"(fa[set][bi]));
+                    else
+                        asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+a"(sum[bi][bj]) : "v"(fb[set][bj]), "v"(fa[set][bi]));
+#else
+                    (void)set, (void)bi, (void)bj;
+#endif
+                };
+                // One step on fragment set `set`: its matrix instructions, the next step's reads among the first three quarters of them and
+                // `Copies` copies spread over all.
+                auto step = [&](auto setC, auto&& read, auto copiesC, auto&& copy) {
+                    constexpr uint32_t set = decltype(setC)::value, Copies = decltype(copiesC)::value;
+                    constexpr uint32_t PerRead = Mfmas * 3u / 4u / Reads, PerCopy = Mfmas / Copies, Squares = Cfg::BlocksN / 2u;
+#pragma unroll
+                    for(uint32_t x = 0; x < Mfmas; ++x)
+                    {
+                        const uint32_t square = x / 4u, inside = x % 4u, si = square / Squares;
+                        const uint32_t sj     = si % 2u == 0u ? square % Squares : Squares - 1u - square % Squares;
+                        multiplyBlock(set, 2u * si + inside / 2u, 2u * sj + ((inside / 2u) ^ (inside % 2u)));
+                        const bool readNow = x % PerRead == 0u && x / PerRead < Reads, copyNow = x % PerCopy == PerCopy / 2u && x / PerCopy < Copies;
+                        if(readNow)
+                            read(x / PerRead);
+                        if(copyNow)
+                            copy(x / PerCopy);
+                        if(readNow || copyNow)
+                            __builtin_amdgcn_sched_barrier(0);
+                    }
+                };
+#pragma unroll
+                for(uint32_t st = 0; st < 2u; ++st)
+                {
+                    const lds::BufferRsrc srcA = sourceA(), srcB = sourceB();
+#pragma unroll
+                    for(uint32_t c = 0; c < Cfg::CopiesA; ++c)
+                        copyA(st, c, srcA);
+#pragma unroll
+                    for(uint32_t c = 0; c < Cfg::CopiesB; ++c)
+                        copyB(st, c, srcB);
+                    advanceA(st + 1u < stages);
+                    advanceB(st + 1u < stages);
+                }
+                lds::waitCopiesAndReads<Cfg::Copies>(); // stage 0 has landed
+                lds::barrier();
+#pragma unroll
+                for(uint32_t q = 0; q < Reads; ++q)
+                    readOperand(0u, 0u, 0u, 0u, q);
+                lds::waitReads();
+                pinSet(0u);
+                uint32_t slotB = 0u;
+                for(uint32_t i = 0; i < stages; ++i)
+                {
+                    const uint32_t slotA = i % 2u, nextB = slotB == 2u ? 0u : slotB + 1u, freeB = nextB == 2u ? 0u : nextB + 1u;
+                    __builtin_amdgcn_sched_barrier(0);
+                    // (the slot of B that stage i - 1 has left)
+                    const lds::BufferRsrc srcB = sourceB();
+                    step(std::integral_constant<uint32_t, 0u>{}, [&](uint32_t q) { readOperand(1u, slotA, slotB, 1u, q); },
+                         std::integral_constant<uint32_t, Cfg::CopiesB>{}, [&](uint32_t c) { copyB(freeB, c, srcB); });
+                    advanceB(i + 3u < stages);
+                    __builtin_amdgcn_sched_barrier(0);
+                    lds::waitCopiesAndReads<Cfg::CopiesB>(); // stage i + 1 has landed (B of stage i + 2 may be in flight), stage i is in registers
+                    pinSet(1u);
+                    lds::barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                    const lds::BufferRsrc srcA = sourceA();
+                    step(std::integral_constant<uint32_t, 1u>{}, [&](uint32_t q) { readOperand(0u, slotA ^ 1u, nextB, 0u, q); },
+                         std::integral_constant<uint32_t, Cfg::CopiesA>{}, [&](uint32_t c) { copyA(slotA, c, srcA); });
+                    advanceA(i + 3u < stages);
+                    slotB = nextB;
+                    __builtin_amdgcn_sched_barrier(0);
+                    lds::waitReads();
+                    pinSet(0u);
+                }
+                lds::waitCopiesAndReads<0u>(); // the surplus copies still target this workgroup's LDS
+                lds::barrier();
+                // (the compiler does not know the last matrix instructions: their results are written 16 clocks or so behind them)
+                asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+            }
+            else if constexpr(S == 2u && Cfg::KSteps == 1u)
             {
                 // Ring of two stages, one MFMA step per stage whose fragments would not fit the register
                 // file twice (fp8 16x16x128: 8 registers per block and operand).  The A fragments of a
@@ -1487,10 +1667,11 @@ namespace rocwmma_amd
                     constexpr uint32_t CopiesC     = GroupBytes / 1024u;
                     constexpr uint32_t GroupsPerRow = Cfg::BlocksN / GB;
                     constexpr uint32_t NG          = Cfg::BlocksM * GroupsPerRow;
-                    static_assert((RowBytes == 256u || RowBytes == 512u) && 2u * GroupBytes * Cfg::Waves <= Cfg::LdsBytes
-                                      && NG >= 2u,
+                    constexpr uint32_t Buffers     = Cfg::BuffersC;
+                    static_assert((RowBytes == 256u || RowBytes == 512u) && Buffers * GroupBytes * Cfg::Waves <= Cfg::LdsBytes
+                                      && NG >= Buffers,
                                   "C staging geometry");
-                    char*          myLds  = ldsRaw + wave * (2u * GroupBytes);
+                    char*          myLds  = ldsRaw + wave * (Buffers * GroupBytes);
                     const char*    cWave  = reinterpret_cast<const char*>(c + static_cast<size_t>(wRow) * ldc + wCol);
                     const size_t   ldcB   = static_cast<size_t>(ldc) * sizeof(OutT);
                     const uint32_t cpRow  = lane / RowChunks; // row inside a copy
@@ -1512,23 +1693,32 @@ namespace rocwmma_amd
                                 src = reinterpret_cast<const char*>(c) + static_cast<size_t>(row < m ? row : m - 1u) * ldcB
                                       + (colB < n * static_cast<uint32_t>(sizeof(OutT)) ? colB : 0u);
                             }
-                            lds::asyncCopy16Streaming(myLds + (gi % 2u) * GroupBytes + i * 1024u, src);
+                            lds::asyncCopy16Streaming(myLds + (gi % Buffers) * GroupBytes + i * 1024u, src);
                         }
                     };
                     const uint32_t rdRow  = accRow;
                     const uint32_t rdBase = rdRow * RowBytes;
-                    copyGroup(0u);
-                    copyGroup(1u);
+#pragma unroll
+                    for(uint32_t gi = 0; gi < Buffers; ++gi)
+                        copyGroup(gi);
 #pragma unroll
                     for(uint32_t gi = 0; gi < NG; ++gi)
                     {
                         const uint32_t bi = gi / GroupsPerRow, bj0 = (gi % GroupsPerRow) * GB;
                         // (the stores of D do not count, see copy_waits.hpp)
-                        if(stagedCInFlight(gi, NG, CopiesC) != 0u)
+                        const uint32_t inFlight = stagedCInFlight(gi, NG, CopiesC, Buffers); // (a constant: the loop is unrolled)
+                        constexpr uint32_t Three = Buffers == 4u ? 3u * CopiesC : 0u, Two = Buffers == 4u ? 2u * CopiesC : 0u;
+                        if(Buffers == 4u && inFlight == Three)
+                            lds::waitCopiesAndReads<Three>();
+                        else if(Buffers == 4u && inFlight == Two)
+                            lds::waitCopiesAndReads<Two>();
+                        else if(inFlight != 0u)
                             lds::waitCopiesAndReads<CopiesC>();
                         else
                             lds::waitCopiesAndReads<0u>();
                         asm volatile("" ::: "memory");
+                        if(gi % GroupsPerRow == 0u)
+                            takeRow(bi);
                         typename Cfg::FragC io[GB];
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
@@ -1538,7 +1728,7 @@ namespace rocwmma_amd
                                 // logical chunk of this run: block bj holds Block / 4 chunks per row
                                 const uint32_t g = bj * (Cfg::Block / 4u) + 2u * r + accGroup;
                                 detail::copyBytes<16u>(io[bj].x + 4u * r,
-                                                       myLds + (gi % 2u) * GroupBytes + rdBase + ((g ^ (rdRow & 15u)) << 4));
+                                                       myLds + (gi % Buffers) * GroupBytes + rdBase + ((g ^ (rdRow & 15u)) << 4));
                             }
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
@@ -1555,11 +1745,11 @@ namespace rocwmma_amd
                             storeBlock(bi, bj0 + bj, acc[bi][bj0 + bj]);
                         __builtin_amdgcn_sched_barrier(0);
                         // behind the stores: the next wait then leaves these copies in flight and not the stores
-                        if(gi + 2u < NG)
+                        if(gi + Buffers < NG)
                         {
                             lds::waitReads(); // the buffer is overwritten next
                             asm volatile("" ::: "memory");
-                            copyGroup(gi + 2u);
+                            copyGroup(gi + Buffers);
                         }
                     }
                 }
@@ -1606,6 +1796,7 @@ namespace rocwmma_amd
 #pragma unroll
                 for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                 {
+                    takeRow(bi);
 #pragma unroll
                     for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
                     {
@@ -1638,6 +1829,7 @@ namespace rocwmma_amd
 #pragma unroll
                 for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                 {
+                    takeRow(bi);
                     if constexpr(std::is_same<OutT, CompT>::value)
                     {
                         // results replace the accumulators, so no two stores share data registers

@@ -42,6 +42,15 @@ namespace rocwmma_amd
             {
                 return edges ? (BK || !AK) : (AK && BK);
             }
+            // Big on whole tiles: four waves of 128 x 128, one per SIMD, where the time of a tile is matrix work (8192^3 and 4096^3 in the
+            // pairs A row / B col, A row / B row, A col / B col, A col / B row, eight waves of 64 x 128 and these: f16 834 -> 797, bf16 835 ->
+            // 786, f16 870 -> 842, f16 880 -> 885 us; int8 425 -> 406, 443 -> 424, 437 -> 421, 484 -> 431).  16-bit operands that are both
+            // dim-major keep the eight waves (24 LDS reads of a step are transposing ones and hold up the only wave of a SIMD), and so do
+            // edge tiles (3984 x 4000 x 4080: -5 to +3 %; int8 spills) and fp8, whose fragments leave no room for a second set.
+            static constexpr bool WideWaves(bool edges)
+            {
+                return !edges && !Fp8 && (AK || BK || sizeof(InT) == 1u);
+            }
             template <uint32_t WavesM, uint32_t WavesN, uint32_t M, uint32_t N, uint32_t Stages, uint32_t PerSimd, uint32_t Edge, bool Edges, uint32_t StageKB = 0u,
                       bool Extra = false>
             using Config = BlockedConfig<InT, OutT, CompT, AK, BK, WavesM, WavesN, M, N, Stages, PerSimd, Edge, Edges, false, Fused, StageKB, Extra>;
@@ -49,7 +58,9 @@ namespace rocwmma_amd
             template <Rung R, bool Edges>
             static constexpr auto select()
             {
-                if constexpr(R == Rung::Big)
+                if constexpr(R == Rung::Big && WideWaves(Edges))
+                    return Config<2, 2, 8, 8, 2, 1, 16, false, 0, true>{};
+                else if constexpr(R == Rung::Big)
                     return Config<4, 2, 4 / D2, 8 / D2, 2, 2, E2, Edges, 0, ExtraB(Edges)>{};
                 else if constexpr(R == Rung::Wide)
                     return Config<4, 2, 4 / D3, 4 / D3, 3, 2, E3, Edges>{};
@@ -74,6 +85,9 @@ namespace rocwmma_amd
             }
             template <Rung R, bool Edges>
             using Of = decltype(select<R, Edges>());
+            // Big's rows and pipeline with half the columns, for the tiles of a last round that would be at most half full
+            using HalfOfBig = std::conditional_t<WideWaves(false), Config<2, 2, 8, 4, 2, 1, 16, false, 0, true>,
+                                                 Config<4, 2, 4 / D2, 4 / D2, 2, 2, E2, false, 0, ExtraB(false)>>;
         };
 
         // Whether one block per wave may be chosen over the rungs: it steps along K in 32 bits, 256 leading dimensions at most, and
@@ -119,9 +133,7 @@ namespace rocwmma_amd
                         return;
                     if constexpr(rung == Rung::Big)
                     {
-                        // same rows and pipeline with half the columns, for the tiles of a last round that would be at most half full
-                        using Half = BlockedConfig<InT, OutT, CompT, AK, BK, 4, 2, 4 / R::D2, 4 / R::D2, 2, 2, R::E2, false, false, Fused, 0, R::ExtraB(false)>;
-                        rc         = launchSplitTail<Aligned, Half>(g, stream, ex);
+                        rc = launchSplitTail<Aligned, typename R::HalfOfBig>(g, stream, ex);
                         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
                             return;
                     }
