@@ -101,22 +101,41 @@ namespace rocwmma_amd
         int          activation = ROCWMMA_AMD_ACT_NONE;
     };
 
-    ROCWMMA_DEVICE ROCWMMA_INLINE float applyActivation(float v, int activation)
+    ROCWMMA_DEVICE ROCWMMA_INLINE float relu(float v)
     {
-        if(activation == ROCWMMA_AMD_ACT_RELU)
-            return v < 0.0f ? 0.0f : v; // (a NaN stays a NaN, as with a maximum that propagates NaNs)
+        return v < 0.0f ? 0.0f : v; // (a NaN stays a NaN, as with a maximum that propagates NaNs)
+    }
+
+    // x * Phi(x) with Phi(x) = erfc(-x / sqrt 2) / 2 and, for z >= 0, erfc(z) = (a1 t + ... + a5 t^5) exp(-z^2), t = 1 / (1 + p z)
+    // (Abramowitz & Stegun 7.1.26, absolute error below 1.5e-7; the constants below are halves of a1 .. a5): one reciprocal, one
+    // exponential and a dozen multiply-adds, a third of the library erff.
+    ROCWMMA_DEVICE ROCWMMA_INLINE float gelu(float v)
+    {
+        const float z    = fabsf(v) * 0.70710678118654752f;
+        const float t    = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * z);
+        const float poly = t * (0.127414796f + t * (-0.142248368f + t * (0.7107068705f + t * (-0.7265760135f + t * 0.5307027145f))));
+        const float half = poly * __builtin_amdgcn_exp2f(-1.4426950408889634f * z * z);
+        return v * (v >= 0.0f ? 1.0f - half : half);
+    }
+
+    // The activation of `Count` values.  One branch for all of them: with one per value the epilogue of a 256 x 128 tile was 1400
+    // branches in 62 KB of code that runs once, and no value's chain of operations overlapped the next one's
+    // (4096 x 14336 x 4096 f16 GELU 391 -> 373 us, 320 x 4656 x 1024 bf16 12.9 -> 11.6, 48 shapes drawn at random 0.96 in the geometric mean).
+    template <uint32_t Count>
+    ROCWMMA_DEVICE ROCWMMA_INLINE void applyActivation(float (&v)[Count], int activation)
+    {
         if(activation == ROCWMMA_AMD_ACT_GELU)
         {
-            // x * Phi(x) with Phi(x) = erfc(-x / sqrt 2) / 2 and, for z >= 0, erfc(z) = (a1 t + ... + a5 t^5)
-            // exp(-z^2), t = 1 / (1 + p z) (Abramowitz & Stegun 7.1.26, absolute error below 1.5e-7): one
-            // reciprocal, one exponential and a dozen multiply-adds, a third of the library erff.
-            const float z    = fabsf(v) * 0.70710678118654752f;
-            const float t    = __builtin_amdgcn_rcpf(1.0f + 0.3275911f * z);
-            const float poly = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-            const float half = 0.5f * poly * __builtin_amdgcn_exp2f(-1.4426950408889634f * z * z);
-            return v * (v >= 0.0f ? 1.0f - half : half);
+#pragma unroll
+            for(uint32_t i = 0; i < Count; ++i)
+                v[i] = gelu(v[i]);
         }
-        return v;
+        else if(activation == ROCWMMA_AMD_ACT_RELU)
+        {
+#pragma unroll
+            for(uint32_t i = 0; i < Count; ++i)
+                v[i] = relu(v[i]);
+        }
     }
 
     // Block scales of a microscaled GEMM: one E8M0 byte per 32 elements along K of every row of A

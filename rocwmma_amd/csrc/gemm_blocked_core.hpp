@@ -1596,7 +1596,7 @@ namespace rocwmma_amd
             };
             // Fused configurations: the bias values of a lane's columns of one block are fetched (four
             // consecutive floats per run, cache hits after the first row of blocks) just before the
-            // block's results go out; finish() is what every result passes through.
+            // block's results go out.
             static_assert(!Cfg::Fused || std::is_same<CompT, float>::value, "fused epilogue: f32 compute");
             struct BiasOfBlock
             {
@@ -1639,15 +1639,36 @@ namespace rocwmma_amd
                 else
                     return loadBias(bj);
             };
-            auto finish = [&](BiasOfBlock const& bv, uint32_t e, CompT v) -> CompT {
+            // What the results of `Count` blocks of a row from block `first` on pass through: at once, but for 32-wide blocks (16 values
+            // per block and lane), which spilled.
+            auto finish = [&](uint32_t bi, uint32_t first, auto countC) {
                 if constexpr(Cfg::Fused)
-                    return applyActivation(v + bv.v[e], ex.fused.activation);
-                else
                 {
-                    (void)bv, (void)e;
-                    return v;
+                    constexpr uint32_t Count = decltype(countC)::value, Per = Cfg::FragAcc::num_elements;
+                    constexpr uint32_t Group = Cfg::Block == 16u ? Count : 1u;
+#pragma unroll
+                    for(uint32_t from = 0; from < Count; from += Group)
+                    {
+                        float v[Group * Per];
+#pragma unroll
+                        for(uint32_t j = 0; j < Group; ++j)
+                        {
+                            const BiasOfBlock bv = biasOf(first + from + j);
+#pragma unroll
+                            for(uint32_t e = 0; e < Per; ++e)
+                                v[j * Per + e] = acc[bi][first + from + j].x[e] + bv.v[e];
+                        }
+                        applyActivation(v, ex.fused.activation);
+#pragma unroll
+                        for(uint32_t j = 0; j < Group; ++j)
+#pragma unroll
+                            for(uint32_t e = 0; e < Per; ++e)
+                                acc[bi][first + from + j].x[e] = v[j * Per + e];
+                    }
                 }
+                (void)bi, (void)first, (void)countC;
             };
+            constexpr std::integral_constant<uint32_t, Cfg::BlocksN> wholeRow{};
             if(beta != static_cast<CompT>(0))
             {
                 if constexpr(Cfg::StagedC)
@@ -1732,13 +1753,10 @@ namespace rocwmma_amd
                             }
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
-                        {
-                            const BiasOfBlock bv = biasOf(bj0 + bj);
 #pragma unroll
                             for(uint32_t e = 0; e < io[bj].num_elements; ++e)
-                                acc[bi][bj0 + bj].x[e]
-                                    = finish(bv, e, alpha * acc[bi][bj0 + bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]));
-                        }
+                                acc[bi][bj0 + bj].x[e] = alpha * acc[bi][bj0 + bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]);
+                        finish(bi, bj0, std::integral_constant<uint32_t, GB>{});
                         // (results replace the accumulators: every store has registers of its own)
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
@@ -1760,12 +1778,17 @@ namespace rocwmma_amd
                     {
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                            for(uint32_t e = 0; e < early[bi][bj].num_elements; ++e)
+                                acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(early[bi][bj].x[e]);
+                        finish(bi, 0u, wholeRow);
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
                         {
-                            auto&             io = early[bi][bj];
-                            const BiasOfBlock bv = biasOf(bj);
+                            auto& io = early[bi][bj];
 #pragma unroll
                             for(uint32_t e = 0; e < io.num_elements; ++e)
-                                io.x[e] = narrowed<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
+                                io.x[e] = narrowed<OutT>(acc[bi][bj].x[e]);
                             if constexpr(!PairIO)
                                 storeBlock(bi, bj, io);
                             else if(bj % 2u == 1u)
@@ -1799,13 +1822,15 @@ namespace rocwmma_amd
                     takeRow(bi);
 #pragma unroll
                     for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                    {
-                        auto& io = fc[bi % 2u][bj];
-                        const BiasOfBlock bv = biasOf(bj);
 #pragma unroll
-                        for(uint32_t e = 0; e < io.num_elements; ++e)
-                            io.x[e] = narrowed<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io.x[e])));
-                    }
+                        for(uint32_t e = 0; e < Cfg::FragC::num_elements; ++e)
+                            acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(fc[bi % 2u][bj].x[e]);
+                    finish(bi, 0u, wholeRow);
+#pragma unroll
+                    for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                        for(uint32_t e = 0; e < Cfg::FragC::num_elements; ++e)
+                            fc[bi % 2u][bj].x[e] = narrowed<OutT>(acc[bi][bj].x[e]);
                     if constexpr(PairIO)
                     {
 #pragma unroll
@@ -1839,12 +1864,10 @@ namespace rocwmma_amd
                         {
 #pragma unroll
                             for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                            {
-                                const BiasOfBlock bv = biasOf(bj);
 #pragma unroll
                                 for(uint32_t e = 0; e < acc[bi][bj].num_elements; ++e)
-                                    acc[bi][bj].x[e] = finish(bv, e, alpha * acc[bi][bj].x[e]);
-                            }
+                                    acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e];
+                            finish(bi, 0u, wholeRow);
                         }
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
@@ -1855,12 +1878,15 @@ namespace rocwmma_amd
                         typename Cfg::FragC fd[Cfg::BlocksN];
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                        {
-                            const BiasOfBlock bv = biasOf(bj);
 #pragma unroll
                             for(uint32_t e = 0; e < fd[bj].num_elements; ++e)
-                                fd[bj].x[e] = narrowed<OutT>(finish(bv, e, alpha * acc[bi][bj].x[e]));
-                        }
+                                acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e];
+                        finish(bi, 0u, wholeRow);
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                            for(uint32_t e = 0; e < fd[bj].num_elements; ++e)
+                                fd[bj].x[e] = narrowed<OutT>(acc[bi][bj].x[e]);
                         if constexpr(PairIO)
                         {
 #pragma unroll

@@ -74,18 +74,19 @@ namespace rocwmma_amd
             // fused epilogue: the bias of each element's column is added and the activation applied
             // before the result is narrowed
             using MapAcc = typename detail::FragConfig<accumulator, BM, BN, BK, CompT>::Map;
-            auto finish  = [&](uint32_t e, CompT v) -> CompT {
+            constexpr uint32_t Count = FragC::num_elements;
+            auto               finish = [&](CompT(&v)[Count]) {
                 if constexpr(std::is_same<CompT, float32_t>::value)
                 {
                     if(bias)
-                        v += bias[cCol + MapAcc::colOf(e, threadIdx.x % Constants::AMDGCN_WAVE_SIZE)];
-                    return applyActivation(v, activation);
+                    {
+#pragma unroll
+                        for(uint32_t e = 0; e < Count; ++e)
+                            v[e] += bias[cCol + MapAcc::colOf(e, threadIdx.x % Constants::AMDGCN_WAVE_SIZE)];
+                    }
+                    applyActivation(v, activation);
                 }
-                else
-                {
-                    (void)e;
-                    return v;
-                }
+                (void)v;
             };
 
             FragC          fc;
@@ -93,19 +94,21 @@ namespace rocwmma_amd
                                                            : static_cast<size_t>(cCol) * ldc + cRow;
             const size_t   dOff = layoutC == mem_row_major ? static_cast<size_t>(cRow) * ldd + cCol
                                                            : static_cast<size_t>(cCol) * ldd + cRow;
+            CompT v[Count];
+#pragma unroll
+            for(uint32_t i = 0; i < Count; ++i)
+                v[i] = alpha * acc.x[i];
             if(beta != static_cast<CompT>(0))
             {
                 load_matrix_sync(fc, c + cOff, ldc, layoutC);
 #pragma unroll
-                for(uint32_t i = 0; i < fc.num_elements; ++i)
-                    fc.x[i] = narrowed<OutT>(finish(i, alpha * acc.x[i] + beta * static_cast<CompT>(fc.x[i])));
+                for(uint32_t i = 0; i < Count; ++i)
+                    v[i] += beta * static_cast<CompT>(fc.x[i]);
             }
-            else
-            {
+            finish(v);
 #pragma unroll
-                for(uint32_t i = 0; i < fc.num_elements; ++i)
-                    fc.x[i] = narrowed<OutT>(finish(i, alpha * acc.x[i]));
-            }
+            for(uint32_t i = 0; i < Count; ++i)
+                fc.x[i] = narrowed<OutT>(v[i]);
             store_matrix_sync(d + dOff, fc, ldd, layoutC);
         }
 
