@@ -152,7 +152,7 @@ namespace rocwmma_amd
             // waves take the compiler waits for every copy in flight before it uses them (five times slower).
             // Wave tiles of 128 rows, one wave per SIMD (the loop is at Cfg::WideWave below): the accumulators take 256 registers, so they
             // live in the accumulation half of the register file.
-            static constexpr bool     WideWave = WavesPerSimd_ == 1u && BlocksM_ == 8u && BlockEdge_ == 16u && Stages_ == 2u && StagesB == 3u;
+            static constexpr bool     WideWave = WavesPerSimd_ == 1u && BlocksM_ == 8u && BlockEdge_ == 16u && ExtraB_;
             static constexpr uint32_t CopyWaves
                 = (Waves == 8u && WavesPerSimd_ == 2u && (Stages_ == 2u || Stages_ == 3u) && (AKMajor || BKMajor) && !Scaled_) ? 4u : Waves;
             // LDS read instructions per MFMA step: b128 reads per block (K-major) or two transposing b64 reads
@@ -836,9 +836,10 @@ namespace rocwmma_amd
 
             if constexpr(Cfg::WideWave)
             {
-                // Four waves of 128 x 128 (128 x 64 in half tiles), one per SIMD; A ring of two stages of 128 bytes, B ring of three.
+                // Four waves of 128 x 128 (128 x 64 in half tiles), one per SIMD; A ring of two stages of 128 bytes, B ring of three (256 x 128
+                // tiles: three and four).
                 // Against eight waves of 64 x 128 every LDS byte feeds a third more flops, nothing is issued twice and the copies are
-                // spread over the whole stage: those of B(i + 2) over its first step, those of A(i + 2) over the second, one to eight
+                // spread over the whole stage: those of B(i + S) over its first step, those of A(i + S) over the second, one to eight
                 // matrix instructions, so no wave ever queues behind them.  What bounds it is the power cap: 2290 clocks a stage
                 // without reads and copies, 2420 with (2048 of matrix work), 1.7 GHz on normally distributed data, 2.4 on zeros.
                 // 8192^3: bf16 both row-major 840 -> 780 us, f16 A row-major / B col-major 807 -> 762; 4096^3 112.7 -> 105.7, 109 -> 101.6.
@@ -935,7 +936,7 @@ namespace rocwmma_amd
                     }
                 };
 #pragma unroll
-                for(uint32_t st = 0; st < 2u; ++st)
+                for(uint32_t st = 0; st < S; ++st)
                 {
                     const lds::BufferRsrc srcA = sourceA(), srcB = sourceB();
 #pragma unroll
@@ -947,32 +948,35 @@ namespace rocwmma_amd
                     advanceA(st + 1u < stages);
                     advanceB(st + 1u < stages);
                 }
-                lds::waitCopiesAndReads<Cfg::Copies>(); // stage 0 has landed
+                lds::waitCopiesAndReads<(S - 1u) * Cfg::Copies>(); // stage 0 has landed
                 lds::barrier();
 #pragma unroll
                 for(uint32_t q = 0; q < Reads; ++q)
                     readOperand(0u, 0u, 0u, 0u, q);
                 lds::waitReads();
                 pinSet(0u);
-                uint32_t slotB = 0u;
+                // (slots of stage i; the slot of B that stage i - 1 has left is the one that is in front of stage i's)
+                uint32_t slotA = 0u, slotB = 0u, freeB = S;
                 for(uint32_t i = 0; i < stages; ++i)
                 {
-                    const uint32_t slotA = i % 2u, nextB = slotB == 2u ? 0u : slotB + 1u, freeB = nextB == 2u ? 0u : nextB + 1u;
+                    const uint32_t nextA = slotA == S - 1u ? 0u : slotA + 1u, nextB = slotB == S ? 0u : slotB + 1u;
                     __builtin_amdgcn_sched_barrier(0);
-                    // (the slot of B that stage i - 1 has left)
                     const lds::BufferRsrc srcB = sourceB();
                     step(std::integral_constant<uint32_t, 0u>{}, [&](uint32_t q) { readOperand(1u, slotA, slotB, 1u, q); },
                          std::integral_constant<uint32_t, Cfg::CopiesB>{}, [&](uint32_t c) { copyB(freeB, c, srcB); });
-                    advanceB(i + 3u < stages);
+                    advanceB(i + S + 1u < stages);
                     __builtin_amdgcn_sched_barrier(0);
-                    lds::waitCopiesAndReads<Cfg::CopiesB>(); // stage i + 1 has landed (B of stage i + 2 may be in flight), stage i is in registers
+                    // stage i + 1 has landed (the stages behind it and B of stage i + S may be in flight), stage i is in registers
+                    lds::waitCopiesAndReads<(S - 2u) * Cfg::Copies + Cfg::CopiesB>();
                     pinSet(1u);
                     lds::barrier();
                     __builtin_amdgcn_sched_barrier(0);
                     const lds::BufferRsrc srcA = sourceA();
-                    step(std::integral_constant<uint32_t, 1u>{}, [&](uint32_t q) { readOperand(0u, slotA ^ 1u, nextB, 0u, q); },
+                    step(std::integral_constant<uint32_t, 1u>{}, [&](uint32_t q) { readOperand(0u, nextA, nextB, 0u, q); },
                          std::integral_constant<uint32_t, Cfg::CopiesA>{}, [&](uint32_t c) { copyA(slotA, c, srcA); });
-                    advanceA(i + 3u < stages);
+                    advanceA(i + S + 1u < stages);
+                    freeB = slotB;
+                    slotA = nextA;
                     slotB = nextB;
                     __builtin_amdgcn_sched_barrier(0);
                     lds::waitReads();

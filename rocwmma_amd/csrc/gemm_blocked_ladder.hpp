@@ -51,6 +51,12 @@ namespace rocwmma_amd
             {
                 return !edges && !Fp8 && (AK || BK || sizeof(InT) == 1u);
             }
+            // Wide (256 x 128) likewise on four waves of 128 x 64, with the ring one stage deeper (all of the LDS): three quarters of the LDS
+            // reads, copies spread over the stage.  Where A is K-contiguous, partly filled tiles too; eight waves of 64 x 64 and these:
+            // 512 x 14336 x 4096 f16 with GELU 69.0 -> 65.1 us, 768 x 5504 x 4096 f16 46.6 -> 44.8, A row / B row 51.9 -> 48.5, 2000 x 3056 x
+            // 1360 bf16 23.8 -> 23.1, 24.4 -> 22.6, int8 768 x 5504 x 8192 46.8 -> 44.7, 53.2 -> 48.9.  With a dim-major A it loses
+            // as much as it gains (0.96 to 1.05, with C read in 16 bits 1.27): transposing reads hold up the only wave of a SIMD.
+            static constexpr bool WideHalves = AK && !Fp8;
             template <uint32_t WavesM, uint32_t WavesN, uint32_t M, uint32_t N, uint32_t Stages, uint32_t PerSimd, uint32_t Edge, bool Edges, uint32_t StageKB = 0u,
                       bool Extra = false>
             using Config = BlockedConfig<InT, OutT, CompT, AK, BK, WavesM, WavesN, M, N, Stages, PerSimd, Edge, Edges, false, Fused, StageKB, Extra>;
@@ -62,6 +68,8 @@ namespace rocwmma_amd
                     return Config<2, 2, 8, 8, 2, 1, 16, false, 0, true>{};
                 else if constexpr(R == Rung::Big)
                     return Config<4, 2, 4 / D2, 8 / D2, 2, 2, E2, Edges, 0, ExtraB(Edges)>{};
+                else if constexpr(R == Rung::Wide && WideHalves)
+                    return Config<2, 2, 8, 4, 3, 1, 16, Edges, 0, true>{};
                 else if constexpr(R == Rung::Wide)
                     return Config<4, 2, 4 / D3, 4 / D3, 3, 2, E3, Edges>{};
                 else if constexpr(R == Rung::Mid)
@@ -137,7 +145,7 @@ namespace rocwmma_amd
                         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE)
                             return;
                     }
-                    if constexpr(!Fused || rung == Rung::Big)
+                    if constexpr(!Fused || rung == Rung::Big || rung == Rung::Wide)
                     {
                         rc = launchCfg<typename R::template Of<rung, false>>(g, stream, ex);
                         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE) // (no whole tiles)

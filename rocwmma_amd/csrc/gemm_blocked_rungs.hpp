@@ -10,7 +10,7 @@ namespace rocwmma_amd
     // The rungs, largest tile first.  What differs is how many bytes a flop costs, how many stages of K are in flight while a
     // tile waits for memory, and how long a tile takes to start:
     //   Big         256 x 256, 8 waves (whole tiles of most pairs: 4), A ring of two stages, B ring of two or three
-    //   Wide        256 x 128, 8 waves, ring of three
+    //   Wide        256 x 128, ring of three, 4 waves (A K-contiguous, 16-bit and int8) or 8
     //   Mid         128 x 128, 4 waves, two workgroups per unit, A ring of two, B ring of three
     //   MidLines    128 x 128, 4 waves, one workgroup per unit, ring of four
     //   Ring2       128 x 128, 4 waves, two workgroups per unit, ring of two, 32-wide blocks
