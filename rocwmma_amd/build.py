@@ -16,7 +16,7 @@ LIB_PATH = os.path.join(HERE, "librocwmma_amd.so")
 AUX_LIB_PATH = os.path.join(HERE, "librocwmma_amd_aux.so")
 
 SOURCES = ["api.hip", "gemm_wave_tile.hip", "gemm_blocked.hip", "gemm_blocked_f16.hip", "gemm_blocked_bf16.hip", "gemm_blocked_fp8.hip",
-           "gemm_blocked_i8.hip", "gemm_blocked_f32.hip", "gemm_fused_f16.hip", "gemm_fused_bf16.hip", "gemm_fused_fp8.hip", "gemm_streamk.hip", "gemm_skinny.hip", "gemm_mx.hip", "gemv.hip", "dlrm.hip", "dlrm_sample.hip", "dlrm_general.hip", "dlrm_general_fwd.hip"]
+           "gemm_blocked_i8.hip", "gemm_blocked_f32.hip", "gemm_fused_f16.hip", "gemm_fused_bf16.hip", "gemm_fused_fp8.hip", "gemm_streamk.hip", "gemm_skinny.hip", "gemm_few_rows.hip", "gemm_mx.hip", "gemv.hip", "dlrm.hip", "dlrm_sample.hip", "dlrm_general.hip", "dlrm_general_fwd.hip"]
 # test and benchmark support: fragment-API self-test kernels and measurement probes
 AUX_SOURCES = ["aux_api.hip", "selftest.hip", "mfma_ceiling.hip", "mfma_streams.hip", "stream_ceiling.hip"]
 

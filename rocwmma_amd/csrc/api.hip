@@ -216,9 +216,12 @@ int rocwmma_amd_gemm_ex(int         algo,
     GemmArgs args{m, n, k, a, b, c, d, lda, ldb, c ? ldc : ldd, ldd, alpha, beta, layout_c};
     if(algo == ROCWMMA_AMD_GEMM_AUTO && m <= 128u)
     {
-        // few token rows against a wide 8-bit weight matrix: the weight-streaming kernels (<= 32 rows;
-        // 48 rows with the K slices spread over workgroups)
+        // few token rows against a weight matrix: the weight-streaming kernels (<= 32 rows of a wide one; 48 rows with the K slices
+        // spread over workgroups), then the kernel whose waves share K
         rc = launchGemmSkinny(dtype_in, dtype_out, layout_a, layout_b, args, asStream(stream));
+        if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)
+            return rc;
+        rc = launchGemmFewRows(dtype_in, dtype_out, layout_a, layout_b, args, asStream(stream));
         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)
             return rc;
     }
@@ -359,6 +362,9 @@ int rocwmma_amd_gemm_bias_act(int          dtype_in,
     if(!isGfx950Current())
         return ROCWMMA_AMD_NO_DEVICE;
     GemmArgs args{m, n, k, a, b, c, d, lda, ldb, c ? ldc : ldd, ldd, alpha, beta, layout_c, bias, activation};
+    rc = launchGemmFewRows(dtype_in, dtype_out, layout_a, layout_b, args, asStream(stream));
+    if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)
+        return rc;
     rc = launchGemmBlockedFused(dtype_in, dtype_out, layout_a, layout_b, args, asStream(stream));
     if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)
         return rc;

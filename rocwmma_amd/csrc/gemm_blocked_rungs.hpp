@@ -157,9 +157,9 @@ namespace rocwmma_amd
         return c.start + c.steps * kKB + waves * (c.fetch * kKB + c.store * outBytes);
     }
 
-    // The rung with the least estimated time.  waveTile: one block per wave may be chosen.
+    // The rung with the least estimated time (which goes to *estimate).  waveTile: one block per wave may be chosen.
     constexpr Rung cheapestRung(OperandKind kind, uint32_t pair, uint32_t m, uint32_t n, uint64_t kBytes, uint32_t outBytes, uint32_t units,
-                                bool waveTile)
+                                bool waveTile, float* estimate = nullptr)
     {
         RungTable const& table = kRungTables[static_cast<uint32_t>(kind)][pair];
         const float      kKB = static_cast<float>(kBytes) * 1e-3f, out = static_cast<float>(outBytes);
@@ -175,8 +175,14 @@ namespace rocwmma_amd
                 time = t;
             }
         }
-        if(waveTile && kBytes <= kWaveTileMaxBytes && waveTileTime(table, m, n, kKB, out) < time)
+        const float wave = waveTile && kBytes <= kWaveTileMaxBytes ? waveTileTime(table, m, n, kKB, out) : time;
+        if(wave < time)
+        {
             best = Rung::WaveTile;
+            time = wave;
+        }
+        if(estimate)
+            *estimate = time;
         return best;
     }
 } // namespace rocwmma_amd

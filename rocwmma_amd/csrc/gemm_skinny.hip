@@ -551,6 +551,11 @@ namespace rocwmma_amd
             // whole 1 KiB copies per row of A, whole fragment steps per K slice, A resident in LDS
             if(g.m % 16u != 0u || g.n % 16u != 0u || (g.k * E) % 1024u != 0u)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+            // Up to 32 columns per compute unit the kernel for few rows is faster (gemm_few_rows.hpp; int8, 16 rows, n = 2048, 4096, 8192, K =
+            // 4096: 10.3 -> 4.9, 10.4 -> 6.5, 12.2 -> 8.7 us; 32 rows 11.6 -> 5.3, 11.7 -> 6.9, 14.0 -> 8.6), beyond them within 10 % of
+            // this one on either side (14336 x 4096 13.6 / 13.1 and 15.6 / 14.4, x 1024 4.9 / 5.3 and 5.6 / 6.2, 28672 x 1024 7.0 / 9.3).
+            if(g.n <= 32u * computeUnits())
+                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
             // K steps of a wave's slice fetched together: as many as divide the slice, up to 8
             const uint32_t steps = g.k * E / (kSkinnySlices * kSkinnyKBytes);
             if(g.m == 16u)

@@ -1,0 +1,24 @@
+"""Which problems the kernel for few rows takes, and on which tile (plain g++, no GPU)."""
+import os
+import subprocess
+
+from few_rows import CASES
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def few_of(tmp_path, problems):
+    exe = tmp_path / "few_of"
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-o", str(exe), os.path.join(ROOT, "tests", "host", "few_of.cpp")])
+    asked = "".join("%d %d %d %d %d\n" % p for p in problems)
+    return [int(x) for x in subprocess.run([str(exe)], input=asked, stdout=subprocess.PIPE, text=True, check=True).stdout.split()]
+
+
+def test_cases_run_on_the_tiles_they_name(tmp_path):
+    got = few_of(tmp_path, [(kind, m, n, k, out) for kind, _, m, n, k, out in CASES])
+    wrong = [(case, nb) for case, nb in zip(CASES, got) if case[1] != nb]
+    assert not wrong, wrong
+
+
+def test_wide_weights_and_short_k_stay_with_the_blocked_kernel(tmp_path):
+    assert few_of(tmp_path, [(0, 128, 14336, 8192, 2), (0, 64, 14336, 8192, 4), (1, 128, 14336, 4096, 4), (2, 96, 8192, 1024, 4), (0, 16, 256, 64, 4)]) == [0] * 5
