@@ -104,6 +104,26 @@ def library():
     return _lib
 
 
+_native = None
+
+
+def _calls():
+    """The library's functions by way of _calls.so (csrc/python_calls.c): the same arguments and status, device pointers as
+    tensors, without ctypes' cost per argument."""
+    global _native
+    if _native is None:
+        L = library()
+        try:
+            from . import _calls as native
+        except ImportError as e:
+            raise RuntimeError(f"rocwmma_amd/_calls.so cannot be loaded: build it with `python rocwmma_amd/build.py` ({e})") from e
+        for name in ("gemm_ex", "gemm_bias_act", "gemm_mx", "gemv", "dlrm_fwd_ex", "dlrm_bwd_ex"):
+            function = getattr(L, "rocwmma_amd_" + name)
+            native.bind(name, ctypes.cast(function, ctypes.c_void_p).value, function)
+        _native = native
+    return _native
+
+
 def aux_library_path():
     return os.path.join(HERE, _AUX_LIB_NAME)
 
@@ -169,7 +189,8 @@ def _stream():
         fast = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         if fast is not None:
             # (no Stream object per call: a launch from Python costs a few microseconds, and this is one of them)
-            _raw_stream = lambda: fast(torch.cuda.current_device())
+            device = torch.cuda.current_device
+            _raw_stream = lambda: fast(device())
         else:
             _raw_stream = lambda: torch.cuda.current_stream().cuda_stream
     return _raw_stream()
@@ -202,8 +223,10 @@ def gemm(dtype_in, dtype_out, layout_a, layout_b, layout_c, m, n, k, a, b, c, d,
     nat = n if layout_c == ROW_MAJOR else m
     ldc = ldc if ldc is not None else nat
     ldd = ldd if ldd is not None else nat
-    gemm_raw(dtype_in, dtype_out, layout_a, layout_b, layout_c, m, n, k, _ptr(a), lda, _ptr(b), ldb,
-             _ptr(c), ldc, _ptr(d), ldd, alpha, beta, algo)
+    rc = (_native or _calls()).gemm_ex(algo, dtype_in, dtype_out, layout_a, layout_b, layout_c, m, n, k, a, lda, b, ldb, c, ldc, d, ldd,
+                                       alpha, beta, (_raw_stream or _stream)())
+    if rc != 0:
+        raise RocwmmaError(rc, "gemm")
     return d
 
 
@@ -260,9 +283,8 @@ def gemm_bias_act(dtype_in, dtype_out, layout_a, layout_b, layout_c, m, n, k, a,
     nat = n if layout_c == ROW_MAJOR else m
     ldc = ldc if ldc is not None else nat
     ldd = ldd if ldd is not None else nat
-    rc = library().rocwmma_amd_gemm_bias_act(dtype_in, dtype_out, layout_a, layout_b, layout_c, m, n, k, _ptr(a), lda,
-                                             _ptr(b), ldb, _ptr(c), ldc, _ptr(d), ldd, alpha, beta, _ptr(bias), activation,
-                                             _stream())
+    rc = _calls().gemm_bias_act(dtype_in, dtype_out, layout_a, layout_b, layout_c, m, n, k, a, lda, b, ldb, c, ldc, d, ldd, alpha, beta,
+                                bias, activation, _stream())
     _check(rc, "gemm_bias_act")
     return d
 
@@ -284,10 +306,8 @@ def gemm_mx(dtype_in, layout_a, layout_b, layout_c, m, n, k, a, scale_a, b, scal
     ldd = ldd if ldd is not None else nat
     ld_scale_a = ld_scale_a if ld_scale_a is not None else k // 32
     ld_scale_b = ld_scale_b if ld_scale_b is not None else k // 32
-    rc = library().rocwmma_amd_gemm_mx(dtype_in, layout_a, layout_b, layout_c, m, n, k, _ptr(a), lda, _ptr(scale_a),
-                                       ld_scale_a, _ptr(b), ldb, _ptr(scale_b), ld_scale_b, _ptr(c), ldc, _ptr(d), ldd,
-                                       alpha, beta, _ptr(workspace),
-                                       0 if workspace is None else workspace.numel() * workspace.element_size(), _stream())
+    rc = _calls().gemm_mx(dtype_in, layout_a, layout_b, layout_c, m, n, k, a, lda, scale_a, ld_scale_a, b, ldb, scale_b, ld_scale_b, c, ldc,
+                          d, ldd, alpha, beta, workspace, 0 if workspace is None else workspace.numel() * workspace.element_size(), _stream())
     _check(rc, "gemm_mx")
     return d
 
@@ -321,8 +341,7 @@ def gemm_mx_packed(dtype_in, layout_a, layout_b, layout_c, m, n, k, a, b, c, d, 
 def gemv(m, k, ncols, a, x, y, alpha=1.0, beta=0.0, lda=None, ldx=None, ldy=None):
     """Y = alpha*A*X + beta*Y in place; A f16 row-major m x k, X f16 k x ncols column-major,
     Y f32 m x ncols column-major."""
-    rc = library().rocwmma_amd_gemv(m, k, ncols, _ptr(a), lda or k, _ptr(x), ldx or k, _ptr(y), ldy or m,
-                                    alpha, beta, _stream())
+    rc = _calls().gemv(m, k, ncols, a, lda or k, x, ldx or k, y, ldy or m, alpha, beta, _stream())
     _check(rc, "gemv")
     return y
 
@@ -332,7 +351,7 @@ def dlrm_fwd(inp, out, m, k, batch, dtype=None):
     if dtype is None:
         _check(library().rocwmma_amd_dlrm_fwd(_ptr(inp), _ptr(out), m, k, batch, _stream()), "dlrm_fwd")
     else:
-        _check(library().rocwmma_amd_dlrm_fwd_ex(dtype, _ptr(inp), _ptr(out), m, k, batch, _stream()), "dlrm_fwd_ex")
+        _check(_calls().dlrm_fwd_ex(dtype, inp, out, m, k, batch, _stream()), "dlrm_fwd_ex")
     return out
 
 
@@ -342,8 +361,7 @@ def dlrm_bwd(inp, upstream, grad, mlp_grad, m, k, batch, dtype=None):
         _check(library().rocwmma_amd_dlrm_bwd(_ptr(inp), _ptr(upstream), _ptr(grad), _ptr(mlp_grad), m, k, batch,
                                               _stream()), "dlrm_bwd")
     else:
-        _check(library().rocwmma_amd_dlrm_bwd_ex(dtype, _ptr(inp), _ptr(upstream), _ptr(grad), _ptr(mlp_grad), m, k, batch,
-                                                 _stream()), "dlrm_bwd_ex")
+        _check(_calls().dlrm_bwd_ex(dtype, inp, upstream, grad, mlp_grad, m, k, batch, _stream()), "dlrm_bwd_ex")
     return grad, mlp_grad
 
 

@@ -1,5 +1,6 @@
 """Builds rocwmma_amd/librocwmma_amd.so, the product library, and rocwmma_amd/librocwmma_amd_aux.so,
-the test and benchmark support library (gfx950 only) from rocwmma_amd/csrc/*.hip with hipcc.
+the test and benchmark support library (gfx950 only) from rocwmma_amd/csrc/*.hip with hipcc, and
+rocwmma_amd/_calls.so, the CPython entry to the product library, from csrc/python_calls.c with the host compiler.
 
 The libraries are built in-tree; tests, the smoke check and the benchmark load what is there and
 only build when nothing is."""
@@ -7,6 +8,7 @@ import concurrent.futures
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -14,6 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "librocwmma_amd.so")
 AUX_LIB_PATH = os.path.join(HERE, "librocwmma_amd_aux.so")
+CALLS_PATH = os.path.join(HERE, "_calls.so")
 
 SOURCES = ["api.hip", "gemm_wave_tile.hip", "gemm_blocked.hip", "gemm_blocked_f16.hip", "gemm_blocked_bf16.hip", "gemm_blocked_fp8.hip",
            "gemm_blocked_i8.hip", "gemm_blocked_f32.hip", "gemm_fused_f16.hip", "gemm_fused_bf16.hip", "gemm_fused_fp8.hip", "gemm_streamk.hip", "gemm_skinny.hip", "gemm_few_rows.hip", "gemm_mx.hip", "gemv.hip", "dlrm.hip", "dlrm_sample.hip", "dlrm_general.hip", "dlrm_general_fwd.hip"]
@@ -52,10 +55,18 @@ def _link(path, objs):
         raise RuntimeError(f"link failed:\n{res.stdout[-4000:]}")
 
 
+def _build_calls():
+    cmd = [os.environ.get("CC", "cc"), "-O2", "-Wall", "-Wextra", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
+           os.path.join(CSRC, "python_calls.c"), "-o", CALLS_PATH]
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host compiler failed for python_calls.c:\n{res.stdout[-4000:]}")
+
+
 def build_library(force=True, jobs=None, only=None):
-    """Compile every translation unit and link both shared libraries.  Returns the product
+    """Compile every translation unit and link the shared libraries.  Returns the product
     library's path.  `only`: a list of source names to recompile (the other objects are reused)."""
-    if not force and os.path.exists(LIB_PATH) and os.path.exists(AUX_LIB_PATH):
+    if not force and os.path.exists(LIB_PATH) and os.path.exists(AUX_LIB_PATH) and os.path.exists(CALLS_PATH):
         return LIB_PATH
     os.makedirs(OBJ_DIR, exist_ok=True)
     todo = [s for s in SOURCES + AUX_SOURCES if only is None or s in only]
@@ -65,6 +76,7 @@ def build_library(force=True, jobs=None, only=None):
     obj = lambda s: os.path.join(OBJ_DIR, os.path.splitext(s)[0] + ".o")
     _link(LIB_PATH, [obj(s) for s in SOURCES])
     _link(AUX_LIB_PATH, [obj(s) for s in AUX_SOURCES])
+    _build_calls()
     return LIB_PATH
 
 
