@@ -217,10 +217,13 @@ int rocwmma_amd_gemm_ex(int         algo,
     if(algo == ROCWMMA_AMD_GEMM_AUTO && m <= 128u)
     {
         // few token rows against a weight matrix: the weight-streaming kernels (<= 32 rows of a wide one; 48 rows with the K slices
-        // spread over workgroups), then the kernel whose waves share K
+        // spread over workgroups)
         rc = launchGemmSkinny(dtype_in, dtype_out, layout_a, layout_b, args, asStream(stream));
         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)
             return rc;
+    }
+    if(algo == ROCWMMA_AMD_GEMM_AUTO)
+    {
         rc = launchGemmFewRows(dtype_in, dtype_out, layout_a, layout_b, args, asStream(stream));
         if(rc != ROCWMMA_AMD_UNSUPPORTED_SHAPE && rc != ROCWMMA_AMD_UNSUPPORTED_TYPE)
             return rc;

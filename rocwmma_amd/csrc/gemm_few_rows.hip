@@ -8,7 +8,7 @@ namespace rocwmma_amd
 {
     int launchGemmFewRows(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream)
     {
-        if(layoutA != ROCWMMA_AMD_ROW_MAJOR || layoutB != ROCWMMA_AMD_COL_MAJOR || g.layoutC != ROCWMMA_AMD_ROW_MAJOR || g.m > kFewMaxRows
+        if(layoutA != ROCWMMA_AMD_ROW_MAJOR || layoutB != ROCWMMA_AMD_COL_MAJOR || g.layoutC != ROCWMMA_AMD_ROW_MAJOR
            || g.m % 16u != 0u || g.n % 16u != 0u)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         const bool        half   = dtypeIn == ROCWMMA_AMD_F16 || dtypeIn == ROCWMMA_AMD_BF16;
@@ -17,25 +17,27 @@ namespace rocwmma_amd
         const uint32_t    outBytes = dtypeOut == ROCWMMA_AMD_F32 || dtypeOut == ROCWMMA_AMD_I32 ? 4u : (dtypeOut == ROCWMMA_AMD_I8 ? 1u : 2u);
         const FewChoice   few      = cheapestFew(g.m, g.n, kBytes, computeUnits());
         float             blocked  = 0.0f;
+        if(few.mb == 0u)
+            return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         cheapestRung(kind, layoutPair(true, true), g.m, g.n, kBytes, outBytes, computeUnits(), true, &blocked);
         if(few.time * kFewMargin > blocked)
             return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
         if(dtypeIn == ROCWMMA_AMD_F16 && dtypeOut == ROCWMMA_AMD_F32)
-            return launchFewRows<float16_t, float32_t, float32_t>(g, stream, few.nb);
+            return launchFewRows<float16_t, float32_t, float32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_F16 && dtypeOut == ROCWMMA_AMD_F16)
-            return launchFewRows<float16_t, float16_t, float32_t>(g, stream, few.nb);
+            return launchFewRows<float16_t, float16_t, float32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_BF16 && dtypeOut == ROCWMMA_AMD_F32)
-            return launchFewRows<bfloat16_t, float32_t, float32_t>(g, stream, few.nb);
+            return launchFewRows<bfloat16_t, float32_t, float32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_BF16 && dtypeOut == ROCWMMA_AMD_BF16)
-            return launchFewRows<bfloat16_t, bfloat16_t, float32_t>(g, stream, few.nb);
+            return launchFewRows<bfloat16_t, bfloat16_t, float32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_E4M3 && dtypeOut == ROCWMMA_AMD_F32)
-            return launchFewRows<float8_t, float32_t, float32_t>(g, stream, few.nb);
+            return launchFewRows<float8_t, float32_t, float32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_E5M2 && dtypeOut == ROCWMMA_AMD_F32)
-            return launchFewRows<bfloat8_t, float32_t, float32_t>(g, stream, few.nb);
+            return launchFewRows<bfloat8_t, float32_t, float32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_I8 && dtypeOut == ROCWMMA_AMD_I32)
-            return launchFewRows<int8_t, int32_t, int32_t>(g, stream, few.nb);
+            return launchFewRows<int8_t, int32_t, int32_t>(g, stream, few);
         if(dtypeIn == ROCWMMA_AMD_I8 && dtypeOut == ROCWMMA_AMD_I8)
-            return launchFewRows<int8_t, int8_t, int32_t>(g, stream, few.nb);
+            return launchFewRows<int8_t, int8_t, int32_t>(g, stream, few);
         return ROCWMMA_AMD_UNSUPPORTED_TYPE;
     }
 

@@ -1,21 +1,23 @@
-// GEMM for few token rows: D = act(alpha * A * B + beta * C + bias) for M <= 128 rows against an N x K weight matrix
-// (A row-major, B col-major, C / D row-major), any K.  Included by the translation units that instantiate it.
+// GEMM with few results for its K (few token rows against a weight matrix above all): D = act(alpha * A * B + beta * C + bias), A
+// row-major, B col-major, C / D row-major, any K.  Included by the translation units that instantiate it.
 //
 // The reference's GEMM kernels (samples/perf_hgemm.cpp:518-714) and the blocked kernel here give a workgroup a tile of D and all
-// of K: with so few rows there are few tiles, each walks K alone, and most of the chip idles.  Here the waves of a workgroup
-// share K instead: NB blocks of 16 weight rows and all of A's rows per workgroup, and every wave multiplies a quarter or an
+// of K: with few rows and columns there are few tiles, each walks K alone, and most of the chip idles.  Here the waves of a workgroup
+// share K instead: MB blocks of 16 rows of A and NB of 16 weight rows per workgroup, and every wave multiplies a quarter or an
 // eighth of K of all of them.  Its operands come through a ring of 128-byte steps in LDS that is the wave's own, so the main loop
 // has no barrier.  (Fragments loaded straight into registers were two to three times slower: the 16 lanes that a load serves
 // together are 16 rows, i.e. 16 lines for 256 bytes, 30 GB/s per compute unit; a copy into LDS takes whole lines.)  The
 // partial sums meet in LDS and are added in the order of the waves: results do not depend on timing.  What bounds it is a
 // compute unit's copies: (MB + NB) * 16 rows of K for NB * 16 columns of results, about 100 GB/s of them by one unit and 12 TB/s by
 // all.  Before (blocked or weight-streaming kernel) and now, us: 16 x 3056 x 7168 bf16 with GELU 39.2 -> 11.8, 16 x 1776 x 5824 f16
-// 28.5 -> 7.2, 64 x 1024 x 8192 f16 30.3 -> 14.9, 32 x 2848 x 6656 int8 16.7 -> 6.5, 96 x 2496 x 3840 f16 19.2 -> 14.4.
+// 28.5 -> 7.2, 64 x 1024 x 8192 f16 30.3 -> 14.9, 32 x 2848 x 6656 int8 16.7 -> 6.5, 416 x 480 x 5280 f16 25.3 -> 15.4,
+// 112 x 320 x 5632 f16 23.5 -> 6.7, 240 x 592 x 2240 bf16 12.2 -> 6.4.
 #ifndef ROCWMMA_AMD_CSRC_GEMM_FEW_ROWS_HPP
 #define ROCWMMA_AMD_CSRC_GEMM_FEW_ROWS_HPP
 
 #include "common.hpp"
 #include "gemm_few_rows_rule.hpp"
+#include <utility>
 #include <rocwmma/rocwmma_lds.hpp>
 
 using namespace rocwmma;
@@ -24,6 +26,7 @@ namespace rocwmma_amd
 {
     namespace
     {
+        constexpr uint32_t kFewXcds    = 8u; // dies, one L2 each
         constexpr uint32_t kFewNowhere = 0x80000000u; // lane offset beyond every buffer: the load returns zeros
 
         template <uint32_t MB_, uint32_t NB_>
@@ -51,7 +54,11 @@ namespace rocwmma_amd
 
             const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
             const uint32_t row = lane & 15u, group = lane >> 4; // of a lane's results in a block: its row, its four columns
-            const uint32_t n0 = blockIdx.x * NB * 16u;
+            // Workgroups of the same weights on one XCD (ids congruent mod 8), whose L2 then fetches them once.
+            const uint32_t groupsM = ceilDiv(g.m, MB * 16u), id = blockIdx.x / kFewXcds;
+            const uint32_t m0 = id % groupsM * MB * 16u, n0 = (id / groupsM * kFewXcds + blockIdx.x % kFewXcds) * NB * 16u;
+            if(n0 >= g.n) // (the whole workgroup)
+                return;
             const uint32_t ldaB = g.lda * E, ldbB = g.ldb * E, kBytes = g.k * E;
             const uint32_t steps = ceilDiv(kBytes, kFewStep), begin = steps * wave / Waves, end = steps * (wave + 1u) / Waves;
             const uint32_t kEnd = min(kBytes, end * kFewStep); // this wave's part of K ends here
@@ -66,7 +73,7 @@ namespace rocwmma_amd
                 aOff[half]  = Rows::laneSourceOffset(lane, half, ldaB);
                 bOff[half]  = Rows::laneSourceOffset(lane, half, ldbB);
             }
-            const lds::BufferRsrc srcA = lds::makeSource(g.a);
+            const lds::BufferRsrc srcA = lds::makeSource(static_cast<const char*>(g.a) + static_cast<size_t>(m0) * ldaB);
             const lds::BufferRsrc srcB = lds::makeSource(static_cast<const char*>(g.b) + static_cast<size_t>(n0) * ldbB);
             char* const           ring = ldsRaw + wave * (Ring * Tile::StepBytes);
             auto                  issue = [&](uint32_t slot, uint32_t step) {
@@ -85,7 +92,7 @@ namespace rocwmma_amd
                     lds::asyncCopy16(to + (2u * MB + c) * 1024u, srcB, n0 + c / 2u * 16u < g.n ? b[c % 2u] : kFewNowhere, c * 8u * ldbB + at);
 #pragma unroll
                 for(uint32_t c = 0; c < 2u * MB; ++c)
-                    lds::asyncCopy16(to + c * 1024u, srcA, c / 2u * 16u < g.m ? a[c % 2u] : kFewNowhere, c * 8u * ldaB + at);
+                    lds::asyncCopy16(to + c * 1024u, srcA, m0 + c / 2u * 16u < g.m ? a[c % 2u] : kFewNowhere, c * 8u * ldaB + at);
             };
 
             FragAcc acc[MB][NB];
@@ -140,7 +147,7 @@ namespace rocwmma_amd
             __syncthreads();
             for(uint32_t block = wave; block < MB * NB; block += Waves)
             {
-                const uint32_t r = block / NB * 16u + row, col = n0 + block % NB * 16u + group * 4u;
+                const uint32_t r = m0 + block / NB * 16u + row, col = n0 + block % NB * 16u + group * 4u;
                 Quad           sum = partial[block * 64u + lane];
 #pragma unroll
                 for(uint32_t w = 1; w < Waves; ++w)
@@ -181,6 +188,13 @@ namespace rocwmma_amd
             }
         }
 
+        // f(integral_constant 0), f(1), ...
+        template <typename F, uint32_t... I>
+        void forTiles(F& f, std::integer_sequence<uint32_t, I...>)
+        {
+            (f(std::integral_constant<uint32_t, I>{}), ...);
+        }
+
         template <typename InT, typename OutT, typename CompT, uint32_t MB, uint32_t NB>
         int launchFewTile(GemmArgs const& g, hipStream_t stream)
         {
@@ -190,44 +204,25 @@ namespace rocwmma_amd
                && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(Tile::LdsBytes))
                       != hipSuccess)
                 return ROCWMMA_AMD_LAUNCH_FAILED;
-            hipLaunchKernelGGL(kernel, dim3(ceilDiv(g.n, NB * 16u)), dim3(64u * Tile::Waves), Tile::LdsBytes, stream, g);
+            hipLaunchKernelGGL(kernel, dim3(ceilDiv(g.m, MB * 16u) * ceilDiv(g.n, NB * 16u * kFewXcds) * kFewXcds), dim3(64u * Tile::Waves), Tile::LdsBytes, stream, g);
             return launchStatus();
         }
 
-        template <typename InT, typename OutT, typename CompT, uint32_t NB>
-        int launchFewBlocks(GemmArgs const& g, hipStream_t stream)
-        {
-            int  rc      = ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            auto attempt = [&](auto blocks) {
-                constexpr uint32_t MB = decltype(blocks)::value;
-                if constexpr(fewHasTile(MB, NB))
-                    if(fewRowBlocks(g.m) == MB)
-                        rc = launchFewTile<InT, OutT, CompT, MB, NB>(g, stream);
-            };
-            attempt(std::integral_constant<uint32_t, 1u>{});
-            attempt(std::integral_constant<uint32_t, 2u>{});
-            attempt(std::integral_constant<uint32_t, 3u>{});
-            attempt(std::integral_constant<uint32_t, 4u>{});
-            attempt(std::integral_constant<uint32_t, 6u>{});
-            attempt(std::integral_constant<uint32_t, 8u>{});
-            return rc;
-        }
-
         template <typename InT, typename OutT, typename CompT>
-        int launchFewRows(GemmArgs const& g, hipStream_t stream, uint32_t nb)
+        int launchFewRows(GemmArgs const& g, hipStream_t stream, FewChoice const& choice)
         {
-            // (copies address the rows of A, and of a workgroup's weights, inside a 2 GiB window)
-            if(static_cast<uint64_t>(g.lda) * sizeof(InT) * g.m >= 0x7FFF0000ull || static_cast<uint64_t>(g.ldb) * sizeof(InT) * 16u * nb >= 0x7FFF0000ull)
+            // (copies address a workgroup's rows of A, and its weights, inside a 2 GiB window)
+            if(static_cast<uint64_t>(g.lda) * sizeof(InT) * 16u * choice.mb >= 0x7FFF0000ull
+               || static_cast<uint64_t>(g.ldb) * sizeof(InT) * 16u * choice.nb >= 0x7FFF0000ull)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            switch(nb)
-            {
-            case 1u:
-                return launchFewBlocks<InT, OutT, CompT, 1>(g, stream);
-            case 2u:
-                return launchFewBlocks<InT, OutT, CompT, 2>(g, stream);
-            default:
-                return launchFewBlocks<InT, OutT, CompT, 4>(g, stream);
-            }
+            int  rc      = ROCWMMA_AMD_UNSUPPORTED_SHAPE;
+            auto attempt = [&](auto index) {
+                constexpr FewCost tile = kFewCosts[decltype(index)::value];
+                if(tile.mb == choice.mb && tile.nb == choice.nb)
+                    rc = launchFewTile<InT, OutT, CompT, tile.mb, tile.nb>(g, stream);
+            };
+            forTiles(attempt, std::make_integer_sequence<uint32_t, kFewTiles>{});
+            return rc;
         }
     } // namespace
 } // namespace rocwmma_amd

@@ -1,4 +1,4 @@
-"""The kernel for few rows (tests/few_rows.py) against one block per wave (GEMM_WAVE_TILE, itself compared with the oracle in
+"""The kernel whose waves share K (tests/few_rows.py) against one block per wave (GEMM_WAVE_TILE, itself compared with the oracle in
 tests/test_gpu_gemm.py).  The operands are small whole numbers: products and sums are exact in whatever order, so results must be
 equal bit for bit; the operands lie in frames of NaN (int8: 99), D in a guard."""
 import pytest
@@ -12,8 +12,8 @@ from util import CM, RM
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("kind,nb,m,n,k_bytes,out", CASES)
-def test_few_rows_equal_one_block_per_wave(kind, nb, m, n, k_bytes, out):
+@pytest.mark.parametrize("kind,mb,nb,m,n,k_bytes,out", CASES)
+def test_few_rows_equal_one_block_per_wave(kind, mb, nb, m, n, k_bytes, out):
     import torch
 
     gen = torch.Generator(device="cuda").manual_seed(m + n + k_bytes)

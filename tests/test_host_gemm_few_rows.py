@@ -1,4 +1,4 @@
-"""Which problems the kernel for few rows takes, and on which tile (plain g++, no GPU)."""
+"""Which problems the kernel whose waves share K takes, and on which tile (plain g++, no GPU)."""
 import os
 import subprocess
 
@@ -11,14 +11,15 @@ def few_of(tmp_path, problems):
     exe = tmp_path / "few_of"
     subprocess.check_call(["g++", "-std=c++17", "-O1", "-Wall", "-o", str(exe), os.path.join(ROOT, "tests", "host", "few_of.cpp")])
     asked = "".join("%d %d %d %d %d\n" % p for p in problems)
-    return [int(x) for x in subprocess.run([str(exe)], input=asked, stdout=subprocess.PIPE, text=True, check=True).stdout.split()]
+    out = subprocess.run([str(exe)], input=asked, stdout=subprocess.PIPE, text=True, check=True).stdout
+    return [tuple(int(x) for x in line.split()) for line in out.splitlines()]
 
 
 def test_cases_run_on_the_tiles_they_name(tmp_path):
-    got = few_of(tmp_path, [(kind, m, n, k, out) for kind, _, m, n, k, out in CASES])
-    wrong = [(case, nb) for case, nb in zip(CASES, got) if case[1] != nb]
+    got = few_of(tmp_path, [(kind, m, n, k, out) for kind, _, _, m, n, k, out in CASES])
+    wrong = [(case, tile) for case, tile in zip(CASES, got) if case[1:3] != tile]
     assert not wrong, wrong
 
 
 def test_wide_weights_and_short_k_stay_with_the_blocked_kernel(tmp_path):
-    assert few_of(tmp_path, [(0, 128, 14336, 8192, 2), (0, 64, 14336, 8192, 4), (1, 128, 14336, 4096, 4), (2, 96, 8192, 1024, 4), (0, 16, 256, 64, 4)]) == [0] * 5
+    assert few_of(tmp_path, [(0, 128, 14336, 8192, 2), (0, 64, 14336, 8192, 4), (1, 128, 14336, 4096, 4), (2, 96, 8192, 1024, 4), (0, 16, 256, 64, 4)]) == [(0, 0)] * 5
