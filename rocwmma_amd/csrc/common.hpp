@@ -170,7 +170,7 @@ namespace rocwmma_amd
     int launchGemmFusedBf16(int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
     int launchGemmFusedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
     int launchGemmSkinny(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream);
-    // Few token rows (A row-major, B col-major, C / D row-major), bias and activation included: ROCWMMA_AMD_UNSUPPORTED_SHAPE where the
+    // Few results for their K (A row-major, B col-major, C / D row-major), bias and activation included: ROCWMMA_AMD_UNSUPPORTED_SHAPE where the
     // blocked kernel is estimated to be faster.
     int launchGemmFewRows(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream);
     // Stream-K: the 256 x 256 tiling with the tile count balanced over persistent workgroups.  The
