@@ -1800,6 +1800,68 @@ namespace rocwmma_amd
                         }
                     }
                 }
+                else if constexpr(Cfg::WideWave)
+                {
+                    // 16- and 8-bit C: all of the wave's C is requested at once, 16 to 64 loads that the only wave of its SIMD has in flight (two rows
+                    // of blocks ahead, as below, was half as much per compute unit as with eight waves).  Edge tiles: rows and columns past the
+                    // problem's fetch some element of C, used by nobody; a branch around every load cost more than the loads.  1040 x 6000 x 256, C
+                    // and D f16: eight waves of 64 x 64 11.8 us, two rows ahead 14.8, at once 10.9; C and D int8, K = 512, 14.9, 19.1, 13.2; on whole
+                    // tiles, 4096^3 f16, 110.6, 102.8, 101.6.
+                    constexpr uint32_t Pieces = PairIO ? Cfg::BlocksN / 2u : Cfg::BlocksN; // of a row of blocks
+                    typedef uint32_t   Words __attribute__((ext_vector_type(PairIO ? 4u : sizeof(OutT))));
+                    Words              raw[Cfg::BlocksM][Pieces];
+#pragma unroll
+                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
+                    {
+                        const uint32_t row = wRow + bi * Cfg::Block + accRow;
+                        const OutT*    src = c + static_cast<size_t>(Cfg::Edges && row >= m ? m - 1u : row) * ldc;
+#pragma unroll
+                        for(uint32_t p = 0; p < Pieces; ++p)
+                        {
+                            const uint32_t col = wCol + (PairIO ? 2u * p * Cfg::Block + pairCol : p * Cfg::Block + 4u * accGroup);
+                            raw[bi][p]         = *reinterpret_cast<const Words*>(src + (Cfg::Edges && col >= n ? 0u : col));
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
+                    {
+                        takeRow(bi);
+                        typename Cfg::FragC io[Cfg::BlocksN];
+#pragma unroll
+                        for(uint32_t p = 0; p < Pieces; ++p)
+                        {
+                            if constexpr(PairIO)
+                            {
+                                __builtin_memcpy(io[2u * p].x, &raw[bi][p], 8);
+                                __builtin_memcpy(io[2u * p + 1u].x, reinterpret_cast<const char*>(&raw[bi][p]) + 8, 8);
+                                swapPair(io[2u * p], io[2u * p + 1u]);
+                            }
+                            else
+                                __builtin_memcpy(io[p].x, &raw[bi][p], sizeof(Words));
+                        }
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                            for(uint32_t e = 0; e < Cfg::FragC::num_elements; ++e)
+                                acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]);
+                        finish(bi, 0u, wholeRow);
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                            for(uint32_t e = 0; e < Cfg::FragC::num_elements; ++e)
+                                io[bj].x[e] = narrowed<OutT>(acc[bi][bj].x[e]);
+#pragma unroll
+                        for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+                        {
+                            if constexpr(!PairIO)
+                                storeBlock(bi, bj, io[bj]);
+                            else if(bj % 2u == 1u)
+                                storePair(bi, bj - 1u, io[bj - 1u], io[bj]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
                 else
                 {
                 typename Cfg::FragC fc[2][Cfg::BlocksN];
@@ -1823,7 +1885,6 @@ namespace rocwmma_amd
 #pragma unroll
                 for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                 {
-                    takeRow(bi);
 #pragma unroll
                     for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
