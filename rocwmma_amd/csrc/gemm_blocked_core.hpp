@@ -812,6 +812,23 @@ namespace rocwmma_amd
                 __builtin_amdgcn_sched_barrier(0);
             }
 
+            // Where a wave's rows begin in the tile, and the row of its block bi behind that.  Wide waves: 128 rows, or, where rows of a 32-bit D are
+            // a multiple of 32 KiB apart, two runs of 64, in turn with the other waves' runs.  The waves write the same block of theirs at about
+            // the same time, and with 128 rows between them that is 4 MiB, which the memory channels do not tell apart; nor do they 1 MiB, which
+            // is why runs of 64 rows are not taken for rows of 16 KiB.  bf16, eight waves of 64 x 128, runs of 128, of 64: with C 4096 x 8192 x 256
+            // 61.4, 75.0, 62.0 us, x 1024 92.3, 102.1, 91.2; 8192 x 4096 x 256 69.0, 61.0, 70.1, x 1024 99.4, 90.2, 98.1; without C 8192 x 8192 x 256
+            // 72.0, 77.9, 69.7.  (16-bit D, 4096 x 16384 x 1024 with C 156.8, 140.6, 145.9.)
+            constexpr bool RunsOfD  = Cfg::WideWave && sizeof(OutT) == 4u;
+            const bool     twoRuns  = RunsOfD && static_cast<uint32_t>(ldd * sizeof(OutT)) % 32768u == 0u;
+            const uint32_t waveRow  = waveM * (twoRuns ? Cfg::WaveM / 2u : Cfg::WaveM);
+            const uint32_t upperRow = twoRuns ? Cfg::MacroM / 2u : Cfg::WaveM / 2u;
+            auto           blockRow = [&](uint32_t bi) {
+                if constexpr(RunsOfD)
+                    return bi < Cfg::BlocksM / 2u ? bi * Cfg::Block : upperRow + (bi - Cfg::BlocksM / 2u) * Cfg::Block;
+                else
+                    return bi * Cfg::Block;
+            };
+
             // Wide waves: the accumulators while they are summed.  The epilogue takes them a row of blocks at a time (takeRow), so that
             // only that row is in ordinary registers.
             typedef CompT Result __attribute__((ext_vector_type(4)));
@@ -889,7 +906,7 @@ namespace rocwmma_amd
                 // operand q of a step: the blocks of A, then those of B
                 auto readOperand = [&](uint32_t set, uint32_t slotA, uint32_t slotB, uint32_t ks, uint32_t q) {
                     if(q < Cfg::BlocksM)
-                        TileA::template readBlock16<16u>(&fa[set][q], ldsRaw + slotA * Cfg::StrideA, waveM * Cfg::WaveM + q * 16u, ks, lane);
+                        TileA::template readBlock16<16u>(&fa[set][q], ldsRaw + slotA * Cfg::StrideA, waveRow + blockRow(q), ks, lane);
                     else
                         TileB::template readBlock16<16u>(&fb[set][q - Cfg::BlocksM], ldsRaw + Cfg::FirstB + slotB * Cfg::StrideB,
                                                          waveN * Cfg::WaveN + (q - Cfg::BlocksM) * 16u, ks, lane);
@@ -1506,7 +1523,7 @@ namespace rocwmma_amd
             // the stores of a group issue back to back (a store whose data registers are about
             // to be overwritten holds up the instruction stream until it has read them), and
             // the C blocks of the next two groups are in flight while a group is finished.
-            const uint32_t wRow        = row0 + waveM * Cfg::WaveM;
+            const uint32_t wRow        = row0 + waveRow;
             const uint32_t wCol        = col0 + waveN * Cfg::WaveN;
             // Plain stores: the 32-byte pieces a store instruction writes per row are merged into
             // full lines in the L2.  Non-temporal stores bypass that merge and were 3-5x slower
@@ -1519,11 +1536,11 @@ namespace rocwmma_amd
             // (edge tiles: a lane's run of four columns of one row is inside the problem or outside it
             // as a whole, N being a multiple of 16)
             auto inside = [&](uint32_t bi, uint32_t bj, uint32_t r) {
-                return wRow + bi * Cfg::Block + accRow < m && wCol + bj * Cfg::Block + 8u * r + 4u * accGroup < n;
+                return wRow + blockRow(bi) + accRow < m && wCol + bj * Cfg::Block + 8u * r + 4u * accGroup < n;
             };
             auto storeBlock = [&](uint32_t bi, uint32_t bj, auto const& f) {
                 typedef uint32_t Words __attribute__((ext_vector_type(sizeof(OutT))));
-                OutT* dst = d + static_cast<size_t>(wRow + bi * Cfg::Block) * ldd + wCol + bj * Cfg::Block;
+                OutT* dst = d + static_cast<size_t>(wRow + blockRow(bi)) * ldd + wCol + bj * Cfg::Block;
 #pragma unroll
                 for(uint32_t r = 0; r < Runs; ++r)
                 {
@@ -1534,7 +1551,7 @@ namespace rocwmma_amd
                 }
             };
             auto loadBlockC = [&](uint32_t bi, uint32_t bj, auto& f) {
-                const OutT* src = c + static_cast<size_t>(wRow + bi * Cfg::Block) * ldc + wCol + bj * Cfg::Block;
+                const OutT* src = c + static_cast<size_t>(wRow + blockRow(bi)) * ldc + wCol + bj * Cfg::Block;
                 if constexpr(!Cfg::Edges)
                     load_matrix_sync(f, src, ldc);
                 else
@@ -1560,7 +1577,7 @@ namespace rocwmma_amd
             constexpr bool PairIO = Cfg::Block == 16u && sizeof(OutT) == 2u && Cfg::BlocksN % 2u == 0u;
             const uint32_t pairCol = (accGroup & 1u) * 16u + 4u * (accGroup & 2u);
             auto           blockOffset = [&](uint32_t bi, uint32_t bj, uint32_t ld) {
-                return static_cast<size_t>(wRow + bi * Cfg::Block) * ld + wCol + bj * Cfg::Block;
+                return static_cast<size_t>(wRow + blockRow(bi)) * ld + wCol + bj * Cfg::Block;
             };
             auto swapPair = [](auto& fx, auto& fy) {
                 uint32_t x[2], y[2];
@@ -1578,7 +1595,7 @@ namespace rocwmma_amd
             };
             // (edge tiles: a lane's eight columns of one row are inside the problem or outside it as a whole)
             auto insidePair = [&](uint32_t bi, uint32_t bj) {
-                return !Cfg::Edges || (wRow + bi * Cfg::Block + accRow < m && wCol + bj * Cfg::Block + pairCol < n);
+                return !Cfg::Edges || (wRow + blockRow(bi) + accRow < m && wCol + bj * Cfg::Block + pairCol < n);
             };
             auto storePair = [&](uint32_t bi, uint32_t bj, auto& fx, auto& fy) {
                 swapPair(fx, fy);
@@ -1709,11 +1726,11 @@ namespace rocwmma_amd
                             const uint32_t r = RowsPerCopy * i + cpRow;
                             const char*    src;
                             if constexpr(!Cfg::Edges)
-                                src = cWave + (bi * Cfg::Block + r) * ldcB + bj0 * Cfg::Block * sizeof(OutT) + ((chunk ^ (r & 15u)) << 4);
+                                src = cWave + (blockRow(bi) + r) * ldcB + bj0 * Cfg::Block * sizeof(OutT) + ((chunk ^ (r & 15u)) << 4);
                             else
                             {
                                 // (rows and columns past the problem's fetch some element of C, used by nobody)
-                                const uint32_t row  = wRow + bi * Cfg::Block + r;
+                                const uint32_t row  = wRow + blockRow(bi) + r;
                                 const uint32_t colB = (wCol + bj0 * Cfg::Block) * static_cast<uint32_t>(sizeof(OutT)) + ((chunk ^ (r & 15u)) << 4);
                                 src = reinterpret_cast<const char*>(c) + static_cast<size_t>(row < m ? row : m - 1u) * ldcB
                                       + (colB < n * static_cast<uint32_t>(sizeof(OutT)) ? colB : 0u);
@@ -1813,7 +1830,7 @@ namespace rocwmma_amd
 #pragma unroll
                     for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                     {
-                        const uint32_t row = wRow + bi * Cfg::Block + accRow;
+                        const uint32_t row = wRow + blockRow(bi) + accRow;
                         const OutT*    src = c + static_cast<size_t>(Cfg::Edges && row >= m ? m - 1u : row) * ldc;
 #pragma unroll
                         for(uint32_t p = 0; p < Pieces; ++p)

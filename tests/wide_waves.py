@@ -7,3 +7,9 @@ NARROW_C = [(0, 0, "Wide", 1040, 6000, 416, 2), (0, 0, "Wide", 528, 7184, 4128, 
             (0, 1, "Wide", 2560, 2560, 768, 2), (1, 0, "Wide", 1536, 3584, 1024, 1), (0, 0, "Big", 2048, 7168, 3072, 2),
             (0, 1, "Big", 2048, 7168, 3072, 2), (0, 2, "Big", 2048, 7168, 3072, 2), (1, 0, "Big", 2048, 7168, 3072, 1),
             (1, 1, "Big", 2048, 7168, 3072, 1), (1, 2, "Big", 2048, 7168, 3072, 1), (1, 3, "Big", 2048, 7168, 3072, 1)]
+
+# rows of a 32-bit D 32 KiB apart: waves of two runs of rows, in whole tiles, in half tiles of a last round, and in partly filled ones
+RUNS_OF_ROWS = [(0, 0, "Wide", 768, 8192, 4096, 4), (0, 1, "Wide", 784, 8192, 2080, 4), (0, 0, "Wide", 784, 8192, 1312, 4),
+                (1, 0, "Wide", 784, 8192, 1312, 4), (1, 1, "Wide", 784, 8192, 4128, 4), (0, 0, "Big", 2560, 8192, 3072, 4),
+                (0, 1, "Big", 4096, 8192, 3072, 4), (0, 2, "Big", 5120, 8192, 3072, 4), (1, 0, "Big", 4096, 8192, 3072, 4),
+                (1, 1, "Big", 2560, 8192, 3072, 4), (1, 2, "Big", 4096, 8192, 3072, 4), (1, 3, "Big", 5120, 8192, 3072, 4)]
