@@ -105,21 +105,45 @@ def library():
 
 
 _native = None
+_FREQUENT = ("gemm_ex", "gemm_bias_act", "gemm_mx", "gemv", "dlrm_fwd_ex", "dlrm_bwd_ex")
+
+
+class _ByCtypes:
+    """The library's functions as the CPython entry has them, for an interpreter that it is not built for: ctypes converts the
+    arguments (a GEMM call then takes about 4 us more of host time)."""
+
+    def __init__(self, L):
+        for name in _FREQUENT:
+            setattr(self, name, self._entry(getattr(L, "rocwmma_amd_" + name)))
+
+    @staticmethod
+    def _entry(function):
+        pointers = [at for at, t in enumerate(function.argtypes) if t is ctypes.c_void_p]
+
+        def call(*args):
+            args = list(args)
+            for at in pointers:
+                if at < len(args) and hasattr(args[at], "data_ptr"):
+                    args[at] = args[at].data_ptr()
+            return function(*args)
+
+        return call
 
 
 def _calls():
-    """The library's functions by way of _calls.so (csrc/python_calls.c): the same arguments and status, device pointers as
-    tensors, without ctypes' cost per argument."""
+    """The library's functions by way of the CPython entry (csrc/python_calls.c): the same arguments and status, device pointers as
+    tensors, without ctypes' cost per argument.  It is built for one interpreter; another one goes through ctypes."""
     global _native
     if _native is None:
         L = library()
         try:
             from . import _calls as native
-        except ImportError as e:
-            raise RuntimeError(f"rocwmma_amd/_calls.so cannot be loaded: build it with `python rocwmma_amd/build.py` ({e})") from e
-        for name in ("gemm_ex", "gemm_bias_act", "gemm_mx", "gemv", "dlrm_fwd_ex", "dlrm_bwd_ex"):
-            function = getattr(L, "rocwmma_amd_" + name)
-            native.bind(name, ctypes.cast(function, ctypes.c_void_p).value, function)
+        except ImportError:
+            native = _ByCtypes(L)
+        else:
+            for name in _FREQUENT:
+                function = getattr(L, "rocwmma_amd_" + name)
+                native.bind(name, ctypes.cast(function, ctypes.c_void_p).value, function)
         _native = native
     return _native
 

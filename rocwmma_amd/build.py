@@ -1,6 +1,7 @@
 """Builds rocwmma_amd/librocwmma_amd.so, the product library, and rocwmma_amd/librocwmma_amd_aux.so,
-the test and benchmark support library (gfx950 only) from rocwmma_amd/csrc/*.hip with hipcc, and
-rocwmma_amd/_calls.so, the CPython entry to the product library, from csrc/python_calls.c with the host compiler.
+the test and benchmark support library (gfx950 only) from rocwmma_amd/csrc/*.hip with hipcc, and rocwmma_amd/_calls.<tag>.so, the
+CPython entry to the product library for the interpreter that builds it, from csrc/python_calls.c with the host compiler (where there
+is none, or no header of the interpreter, the calls go through ctypes instead).
 
 The libraries are built in-tree; tests, the smoke check and the benchmark load what is there and
 only build when nothing is."""
@@ -16,7 +17,8 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 LIB_PATH = os.path.join(HERE, "librocwmma_amd.so")
 AUX_LIB_PATH = os.path.join(HERE, "librocwmma_amd_aux.so")
-CALLS_PATH = os.path.join(HERE, "_calls.so")
+# (the interpreter's tag in the name: another one does not load it)
+CALLS_PATH = os.path.join(HERE, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 SOURCES = ["api.hip", "gemm_wave_tile.hip", "gemm_blocked.hip", "gemm_blocked_f16.hip", "gemm_blocked_bf16.hip", "gemm_blocked_fp8.hip",
            "gemm_blocked_i8.hip", "gemm_blocked_f32.hip", "gemm_fused_f16.hip", "gemm_fused_bf16.hip", "gemm_fused_fp8.hip", "gemm_streamk.hip", "gemm_skinny.hip", "gemm_few_rows.hip", "gemm_mx.hip", "gemv.hip", "dlrm.hip", "dlrm_sample.hip", "dlrm_general.hip", "dlrm_general_fwd.hip"]
@@ -56,17 +58,27 @@ def _link(path, objs):
 
 
 def _build_calls():
+    """Whether the CPython entry could be built: rocwmma_amd.api does without it."""
     cmd = [os.environ.get("CC", "cc"), "-O2", "-Wall", "-Wextra", "-shared", "-fPIC", "-I" + sysconfig.get_paths()["include"],
            os.path.join(CSRC, "python_calls.c"), "-o", CALLS_PATH]
-    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"host compiler failed for python_calls.c:\n{res.stdout[-4000:]}")
+    try:
+        res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+        trouble = res.stdout if res.returncode != 0 else None
+    except OSError as e:
+        trouble = str(e)
+    if trouble is not None:
+        if os.path.exists(CALLS_PATH):
+            os.remove(CALLS_PATH)  # (of older sources)
+        print(f"python_calls.c not built, calls go through ctypes:\n{trouble[-4000:]}", file=sys.stderr)
+    return trouble is None
 
 
 def build_library(force=True, jobs=None, only=None):
     """Compile every translation unit and link the shared libraries.  Returns the product
     library's path.  `only`: a list of source names to recompile (the other objects are reused)."""
-    if not force and os.path.exists(LIB_PATH) and os.path.exists(AUX_LIB_PATH) and os.path.exists(CALLS_PATH):
+    if not force and os.path.exists(LIB_PATH) and os.path.exists(AUX_LIB_PATH):
+        if not os.path.exists(CALLS_PATH):
+            _build_calls()
         return LIB_PATH
     os.makedirs(OBJ_DIR, exist_ok=True)
     todo = [s for s in SOURCES + AUX_SOURCES if only is None or s in only]

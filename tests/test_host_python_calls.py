@@ -73,3 +73,45 @@ def test_same_as_ctypes(calls, name):
             assert outcome(lib, getattr(module, name), args) == outcome(lib, getattr(lib, name), by_ctypes), (at, value)
     for args in (base[:-1], []):
         assert outcome(lib, getattr(module, name), args) == outcome(lib, getattr(lib, name), args)
+
+
+@pytest.mark.parametrize("name", list(FORMS))
+def test_without_the_entry_the_same_calls_go_through_ctypes(calls, name):
+    lib, module = calls
+
+    class Library:
+        def __getattr__(self, attribute):
+            return getattr(lib, attribute[len("rocwmma_amd_"):])
+
+    by_ctypes = getattr(api._ByCtypes(Library()), name)
+    plain = {I: 3, U: 70000, P: Tensor(0x7F0012345670), F: 2.5, Z: 1 << 40}
+    base = [plain[t] for t in FORMS[name]]
+    none = [None if t is P else v for t, v in zip(FORMS[name], base)]
+    for args in (base, none, base[:-1], ["3"] + base[1:]):
+        assert outcome(lib, by_ctypes, args) == outcome(lib, getattr(module, name), args)
+
+
+def test_another_interpreter_goes_through_ctypes(monkeypatch):
+    import sys
+
+    if not os.path.exists(build.LIB_PATH):
+        pytest.skip("not built")
+    monkeypatch.setitem(sys.modules, "rocwmma_amd._calls", None)  # (its import raises ImportError)
+    monkeypatch.delattr("rocwmma_amd._calls", raising=False)
+    monkeypatch.setattr(api, "_native", None)
+    assert isinstance(api._calls(), api._ByCtypes)
+    # (no GPU in it: the library refuses a matrix without rows)
+    assert api._calls().gemv(0, 0, 0, None, 0, None, 0, None, 0, 1.0, 0.0, None) == api.library().rocwmma_amd_gemv(0, 0, 0, None, 0, None, 0, None, 0, 1.0, 0.0, None) != 0
+
+
+def test_the_entry_is_for_one_interpreter_and_the_build_does_without_it(monkeypatch, tmp_path, capsys):
+    import sysconfig
+
+    assert build.CALLS_PATH.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+    for path in (build.LIB_PATH, build.AUX_LIB_PATH):
+        if not os.path.exists(path):
+            pytest.skip("not built")
+    monkeypatch.setattr(build, "CALLS_PATH", str(tmp_path / "_calls.so"))
+    monkeypatch.setenv("CC", str(tmp_path / "no-such-compiler"))
+    assert build.build_library(force=False) == build.LIB_PATH
+    assert "ctypes" in capsys.readouterr().err
