@@ -99,7 +99,16 @@ namespace rocwmma_amd
         // fused epilogue (rocwmma_amd_gemm_bias_act): D = act(alpha * A * B + beta * C + bias[column])
         const float* bias       = nullptr; // one value per column of D, or nullptr
         int          activation = ROCWMMA_AMD_ACT_NONE;
+        // the blocked kernel's rung (a Rung, gemm_blocked_rungs.hpp) where it has been chosen for this problem already; 0: not yet
+        uint8_t rung = 0;
     };
+
+    // Whether one block per wave may be chosen over the blocked kernel's rungs: it steps along K in 32 bits, 256 leading dimensions at
+    // most, and launches four threads per row.  (All sizes alike, as the choice is made on the transposed problem for a col-major D.)
+    inline bool waveTileTakes(GemmArgs const& g)
+    {
+        return (g.m | g.n | g.lda | g.ldb | g.ldc | g.ldd) < (1u << 24);
+    }
 
     ROCWMMA_DEVICE ROCWMMA_INLINE float relu(float v)
     {
@@ -171,8 +180,8 @@ namespace rocwmma_amd
     int launchGemmFusedFp8(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& g, hipStream_t stream);
     int launchGemmSkinny(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream);
     // Few results for their K (A row-major, B col-major, C / D row-major), bias and activation included: ROCWMMA_AMD_UNSUPPORTED_SHAPE where the
-    // blocked kernel is estimated to be faster.
-    int launchGemmFewRows(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs const& args, hipStream_t stream);
+    // blocked kernel is estimated to be faster, which then finds the rung of that estimate in args.rung.
+    int launchGemmFewRows(int dtypeIn, int dtypeOut, int layoutA, int layoutB, GemmArgs& args, hipStream_t stream);
     // Stream-K: the 256 x 256 tiling with the tile count balanced over persistent workgroups.  The
     // workspace holds one slot of raw accumulators per workgroup plus flags (streamKWorkspaceBytes).
     constexpr uint32_t kStreamKSlotBytes = 256u * 256u * 4u;

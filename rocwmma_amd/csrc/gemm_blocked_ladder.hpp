@@ -98,12 +98,6 @@ namespace rocwmma_amd
                                                  Config<4, 2, 4 / D2, 4 / D2, 2, 2, E2, false, 0, ExtraB(false)>>;
         };
 
-        // Whether one block per wave may be chosen over the rungs: it steps along K in 32 bits, 256 leading dimensions at most, and
-        // launches four threads per row.  (All sizes alike, as the choice is made on the transposed problem for a col-major D.)
-        inline bool waveTileTakes(GemmArgs const& g)
-        {
-            return (g.m | g.n | g.lda | g.ldb | g.ldc | g.ldd) < (1u << 24);
-        }
         template <typename InT>
         constexpr OperandKind operandKind()
         {
@@ -122,8 +116,10 @@ namespace rocwmma_amd
             using Aligned               = typename R::template Of<Rung::Big, false>;
             if(use == TileUse::Large)
                 return launchCfg<Aligned>(g, stream, ex);
-            const Rung best = cheapestRung(kind, pair, g.m, g.n, static_cast<uint64_t>(g.k) * sizeof(InT), sizeof(OutT), computeUnits(),
-                                           use == TileUse::Any && waveTileTakes(g));
+            const uint64_t kBytes = static_cast<uint64_t>(g.k) * sizeof(InT);
+            const Rung     best   = use == TileUse::Any && g.rung != 0u
+                                        ? static_cast<Rung>(g.rung)
+                                        : cheapestRung(kind, pair, g.m, g.n, kBytes, sizeof(OutT), computeUnits(), use == TileUse::Any && waveTileTakes(g));
             if(best == Rung::WaveTile)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
             // A rung refuses a problem whose operand rows span more than a copy's window (ROCWMMA_AMD_UNSUPPORTED_SHAPE): the smaller

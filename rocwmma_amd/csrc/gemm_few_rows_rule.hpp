@@ -45,7 +45,8 @@ namespace rocwmma_amd
     {
         const uint32_t rows = m / 16u, cols = n / 16u; // blocks
         FewChoice      best = {0u, 0u, 1e30f};
-        if(static_cast<uint64_t>(rows) * cols > 12u * units) // (more than any tile here is good for)
+        // (more than any tile here is good for; K of one step, which no two waves share: the blocked kernel was estimated faster for every m and n)
+        if(static_cast<uint64_t>(rows) * cols > 12u * units || kBytes <= kFewStep)
             return best;
         const uint32_t by[4] = {rows, (rows + 1u) / 2u, (rows + 2u) / 3u, (rows + 3u) / 4u};
         const float    kKB = static_cast<float>(kBytes) * 1e-3f, perUnit = 1.0f / static_cast<float>(units);

@@ -23,3 +23,8 @@ def test_cases_run_on_the_tiles_they_name(tmp_path):
 
 def test_wide_weights_and_short_k_stay_with_the_blocked_kernel(tmp_path):
     assert few_of(tmp_path, [(0, 128, 14336, 8192, 2), (0, 64, 14336, 8192, 4), (1, 128, 14336, 4096, 4), (2, 96, 8192, 1024, 4), (0, 16, 256, 64, 4)]) == [(0, 0)] * 5
+
+
+def test_one_step_of_k_stays_with_the_blocked_kernel(tmp_path):
+    problems = [(kind, m, n, k_bytes, out) for kind in range(3) for out in (1, 2, 4) for m in (16, 32, 160, 1024) for n in (16, 128, 2048) for k_bytes in (32, 64, 128)]
+    assert few_of(tmp_path, problems) == [(0, 0)] * len(problems)
