@@ -16,6 +16,7 @@
 //   * the four K-slice partial accumulators of a block meet in LDS; the sum is formed in a
 //     fixed order, so the result is deterministic (and bit-exact for int8).
 #include "common.hpp"
+#include "gemm_skinny_rule.hpp"
 #include <rocwmma/rocwmma_lds.hpp>
 
 using namespace rocwmma;
@@ -24,11 +25,8 @@ namespace rocwmma_amd
 {
     namespace
     {
-        constexpr uint32_t kSkinnySlices = 4;   // K slices per block of weight rows
         constexpr uint32_t kSkinnyBlocks = 4;   // blocks of 16 weight rows per workgroup
         constexpr uint32_t kSkinnyWaves  = kSkinnySlices * kSkinnyBlocks;
-        constexpr uint32_t kSkinnyKBytes = 128; // bytes of K per fragment step (128 8-bit or 64 16-bit elements)
-        constexpr uint32_t kSkinnyMaxA   = 131072; // bytes of LDS the token matrix may take
 
         // Scaled: fp8 operands with one E8M0 scale per 32 elements of K (block-scaled / MX); a fragment step
         // is then one v_mfma_scale_f32_16x16x128_f8f6f4, whose scale operand of lane l belongs to row
@@ -297,11 +295,7 @@ namespace rocwmma_amd
         // The atomic adds set the pace (about 3 ns per output element and slice over the whole
         // chip: 64 x 14336 x 4096 takes 24 us, 128 rows would take 36 us against 25 us on the
         // blocked kernel, which therefore keeps the multiples of 128).
-        constexpr uint32_t kSlicedWaves = 8;
-        constexpr uint32_t kSlicedNB    = 2; // blocks of 16 weight rows per wave
-        constexpr uint32_t kSlicedCols  = kSlicedWaves * kSlicedNB * 16u; // output columns per workgroup
         constexpr uint32_t kSlicedAhead = 4;
-        constexpr uint32_t kSlicedMaxM  = 128;
 
         template <typename OutT, typename CompT>
         __global__ void __launch_bounds__(256)
@@ -493,84 +487,25 @@ namespace rocwmma_amd
         }
 
         template <typename InT, typename OutT, typename CompT>
-        int pickSliced(GemmArgs const& g, hipStream_t stream)
-        {
-            constexpr uint32_t E = sizeof(InT);
-            // (n: the kernel that initialises D counts 4-element groups in 32 bits)
-            if(g.m % 16u != 0u || g.m >= kSlicedMaxM || g.n % 16u != 0u || g.n > (1u << 24) || (g.k * E) % 1024u != 0u)
-                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            // From 64 rows on the blocked kernel is as fast or faster, in one launch and without atomic adds.  Below, K is what decides,
-            // alike for 8- and 16-bit types: the blocked kernel has one workgroup walk all of K (about 2.4 us per KiB of it), here
-            // the second launch and the atomic adds of every slice (more with more columns) come on top of the weights.  48 rows,
-            // n columns, int8, blocked / here in us:
-            //     K bytes     n = 256      4096         7168         8192         14336        28672
-            //        4096   11.7 / 13.6  11.9 / 14.8  15.0 / 17.5  15.4 / 18.0  17.4 / 22.6  29.7 / 32.6
-            //        6144   16.2 / 14.0  19.5 / 16.7  20.9 / 19.8  21.1 / 20.9  23.1 / 32.1  39.0 / 55.6
-            //        8192   20.5 / 13.6  25.3 / 18.1  26.5 / 22.5  27.0 / 24.7  31.2 / 32.0  51.8 / 59.6
-            //       28672   64.2 / 14.2  81.1 / 32.2  85.6 / 57.4  87.7 / 60.7
-            // (float16 with 6144 bytes and n = 7168, 8192: 48 rows 20.8 / 21.1, 21.2 / 22.4; 32 rows, fewer adds, 20.4 / 18.2, 20.6 / 19.3.)
-            const uint64_t kBytes    = static_cast<uint64_t>(g.k) * E;
-            const uint64_t perUnit   = kBytes / (g.m > 32u ? 256u : 192u); // columns
-            const bool     fewerAdds = g.n <= computeUnits() * (perUnit < 32u ? perUnit : 32u);
-            if(g.m >= 64u || kBytes <= 4096u || !fewerAdds)
-                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            // K slices: whole 1 KiB copies per row and whole batches of fragment steps per slice, the
-            // A slice within 128 KiB of LDS; as few slices as fill the compute units
-            const uint32_t groups = (g.n + kSlicedCols - 1u) / kSlicedCols;
-            const uint32_t units  = g.k * E / 1024u;
-            uint32_t       slices = 0;
-            for(uint32_t s = 1; s <= units; ++s)
-            {
-                if(units % s != 0u || g.m * (g.k / s) * E > kSkinnyMaxA)
-                    continue;
-                slices = s;
-                if(groups * s >= computeUnits() * 3u / 4u)
-                    break;
-            }
-            if(slices == 0u)
-                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            switch(g.m / 16u)
-            {
-            case 1: // (16 and 32 rows come here only when all of A does not fit the LDS)
-                return launchSliced<InT, OutT, CompT, 1>(g, stream, slices);
-            case 2:
-                return launchSliced<InT, OutT, CompT, 2>(g, stream, slices);
-            case 3:
-                return launchSliced<InT, OutT, CompT, 3>(g, stream, slices);
-            default:
-                return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            }
-        }
-
-        template <typename InT, typename OutT, typename CompT>
         int pickShape(GemmArgs const& g, hipStream_t stream)
         {
-            constexpr uint32_t E = sizeof(InT);
-            if(g.m > 32u || g.m * g.k * E > kSkinnyMaxA)
-                return pickSliced<InT, OutT, CompT>(g, stream);
-            // whole 1 KiB copies per row of A, whole fragment steps per K slice, A resident in LDS
-            if(g.m % 16u != 0u || g.n % 16u != 0u || (g.k * E) % 1024u != 0u)
+            const uint64_t kBytes = static_cast<uint64_t>(g.k) * sizeof(InT);
+            if(g.m >= 64u || kBytes % 1024u != 0u) // (as the rules have it, without the call that asks for the units)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            // Up to 32 columns per compute unit the kernel for few rows is faster (gemm_few_rows.hpp; int8, 16 rows, n = 2048, 4096, 8192, K =
-            // 4096: 10.3 -> 4.9, 10.4 -> 6.5, 12.2 -> 8.7 us; 32 rows 11.6 -> 5.3, 11.7 -> 6.9, 14.0 -> 8.6), beyond them within 10 % of
-            // this one on either side (14336 x 4096 13.6 / 13.1 and 15.6 / 14.4, x 1024 4.9 / 5.3 and 5.6 / 6.2, 28672 x 1024 7.0 / 9.3).
-            if(g.n <= 32u * computeUnits())
+            const uint32_t units = computeUnits(), steps = skinnySteps(g.m, g.n, kBytes, units), slices = kSlicesOf(g.m, g.n, kBytes, units);
+            if(slices != 0u)
+                return g.m == 16u   ? launchSliced<InT, OutT, CompT, 1>(g, stream, slices)
+                       : g.m == 32u ? launchSliced<InT, OutT, CompT, 2>(g, stream, slices)
+                                    : launchSliced<InT, OutT, CompT, 3>(g, stream, slices);
+            if(steps == 0u)
                 return ROCWMMA_AMD_UNSUPPORTED_SHAPE;
-            // K steps of a wave's slice fetched together: as many as divide the slice, up to 8
-            const uint32_t steps = g.k * E / (kSkinnySlices * kSkinnyKBytes);
             if(g.m == 16u)
-            {
-                if(steps % 8u == 0u)
-                    return launchOne<InT, OutT, CompT, 1, 8>(g, stream);
-                if(steps % 4u == 0u)
-                    return launchOne<InT, OutT, CompT, 1, 4>(g, stream);
-                return launchOne<InT, OutT, CompT, 1, 2>(g, stream);
-            }
-            if(steps % 8u == 0u)
-                return launchOne<InT, OutT, CompT, 2, 8>(g, stream);
-            if(steps % 4u == 0u)
-                return launchOne<InT, OutT, CompT, 2, 4>(g, stream);
-            return launchOne<InT, OutT, CompT, 2, 2>(g, stream);
+                return steps == 8u   ? launchOne<InT, OutT, CompT, 1, 8>(g, stream)
+                       : steps == 4u ? launchOne<InT, OutT, CompT, 1, 4>(g, stream)
+                                     : launchOne<InT, OutT, CompT, 1, 2>(g, stream);
+            return steps == 8u   ? launchOne<InT, OutT, CompT, 2, 8>(g, stream)
+                   : steps == 4u ? launchOne<InT, OutT, CompT, 2, 4>(g, stream)
+                                 : launchOne<InT, OutT, CompT, 2, 2>(g, stream);
         }
     } // namespace
 
