@@ -11,3 +11,10 @@ def test_cases_run_on_the_rungs_they_name(rung_of, name):  # noqa: F811
     asked = "".join("%d %d %d %d %d %d\n" % (kind, pair, m, n, k_bytes, out) for kind, pair, _, m, n, k_bytes, out in cases)
     wrong = [(case, rung) for case, rung in zip(cases, rung_of(text=asked)) if case[2] != rung]
     assert not wrong, wrong
+
+
+def test_half_tiles_have_a_last_round_of_at_most_half_the_units():
+    for kind, pair, rung, m, n, k_bytes, out in wide_waves.HALF_TILES:
+        assert m % 256 == 0 and n % 256 == 0 and k_bytes % 128 == 0
+        tiles = (m // 256) * (n // 256)
+        assert tiles > 256 and 0 < tiles % 256 <= 128
