@@ -173,6 +173,15 @@ namespace rocwmma_amd
             // waves, 127.2 against 126.7 us; with four 122.1 against 128.1), two else
             static constexpr uint32_t BuffersC = WideWave && 4u * Block * GroupBlocks * Block * sizeof(OutT) * Waves <= LdsBytes ? 4u : 2u;
 
+            // Fused epilogue of 256 x 256 tiles on wide waves, and of their half tiles: a loop over the rows of blocks that is not unrolled (with
+            // a C of 16 bits it is).  256 results per lane through bias and GELU one after the other are 37 KB of code, and what a first call, or
+            // one behind other kernels, waits for is that code, with one wave per SIMD and nobody to cover it.  f16, GELU, K = 512 to 4096, operands
+            // not used before, eight waves, four unrolled, four with the loop, us: 1536 x 14336 x 512 51.2, 54.9, 50.3; 2048 x 14336 x 1024 79.6, 81.3,
+            // 77.4; 2048 x 7168 x 2048 70.3, 68.2, 62.1; 4096^3 117.9, 111.2, 107.7; with a C of 32 bits 2560 x 7168 x 1024 78.5, 83.9, 78.9.
+            // The same operands again: 40.7, 41.9, 40.8; 72.3, 70.7, 69.8; 57.9, 55.6, 55.4; 109.7, 104.5, 103.6; 68.5, 67.2, 69.5.  128 results
+            // per lane (256 x 128 tiles) gain nothing: 512 x 14336 x 4096 79.6, 80.6 unrolled, 81.4 with the loop, again 65.6, 58.3, 61.1.
+            static constexpr bool RolledRows = Fused_ && WideWave && Stages_ == 2u;
+
             // C of the small tiles (at most 32 registers of it) is loaded in front of the main loop: behind it, the loads' latency
             // is a large part of a short problem (per call in a captured graph: 256^3 f16 4.0 -> 3.55 us, 512 x 1024 x 1024 e4m3
             // 5.4 -> 4.8, 640 x 1200 x 1360 bf16 10.0 -> 9.5).
@@ -830,11 +839,35 @@ namespace rocwmma_amd
             };
 
             // Wide waves: the accumulators while they are summed.  The epilogue takes them a row of blocks at a time (takeRow), so that
-            // only that row is in ordinary registers.
+            // only that row is in ordinary registers: row bi of blocks to acc[at].
             typedef CompT Result __attribute__((ext_vector_type(4)));
             Result        sum[Cfg::WideWave ? Cfg::BlocksM : 1u][Cfg::WideWave ? Cfg::BlocksN : 1u];
-            auto          takeRow = [&](uint32_t bi) {
-                if constexpr(Cfg::WideWave)
+            auto          takeRow = [&](uint32_t bi, uint32_t at) {
+                if constexpr(Cfg::RolledRows)
+                {
+                    // (which row is known when the kernel runs: a branch per row around the moves out of the accumulation registers, which are
+                    // written in assembly because the compiler makes them in front of the loop else, for all rows, and spills)
+#pragma unroll
+                    for(uint32_t r = 0; r < Cfg::BlocksM; ++r)
+                        if(bi == r)
+                        {
+#pragma unroll
+                            for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
+#pragma unroll
+                                for(uint32_t e = 0; e < 4u; ++e)
+                                {
+                                    const CompT from = sum[r][bj][e];
+                                    CompT       to;
+#if ROCWMMA_ARCH_GFX950
+                                    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(to) : "a"(from));
+#else
+                                    to = from;
+#endif
+                                    acc[at][bj].x[e] = to;
+                                }
+                        }
+                }
+                else if constexpr(Cfg::WideWave)
                 {
 #pragma unroll
                     for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
@@ -842,10 +875,10 @@ namespace rocwmma_amd
                         asm volatile("" : "+a"(sum[bi][bj]));
 #pragma unroll
                         for(uint32_t e = 0; e < 4u; ++e)
-                            acc[bi][bj].x[e] = sum[bi][bj][e];
+                            acc[at][bj].x[e] = sum[bi][bj][e];
                     }
                 }
-                (void)bi;
+                (void)bi, (void)at;
             };
 
             constexpr uint32_t S      = Cfg::Stages;
@@ -1725,7 +1758,9 @@ namespace rocwmma_amd
                         {
                             const uint32_t r = RowsPerCopy * i + cpRow;
                             const char*    src;
-                            if constexpr(!Cfg::Edges)
+                            if constexpr(Cfg::RolledRows) // (what does not depend on bi stays in front of the loop)
+                                src = cWave + blockRow(bi) * ldcB + (r * ldcB + ((chunk ^ (r & 15u)) << 4));
+                            else if constexpr(!Cfg::Edges)
                                 src = cWave + (blockRow(bi) + r) * ldcB + bj0 * Cfg::Block * sizeof(OutT) + ((chunk ^ (r & 15u)) << 4);
                             else
                             {
@@ -1743,12 +1778,13 @@ namespace rocwmma_amd
 #pragma unroll
                     for(uint32_t gi = 0; gi < Buffers; ++gi)
                         copyGroup(gi);
-#pragma unroll
+                    static_assert(!Cfg::RolledRows || (GroupsPerRow == 1u && !Cfg::Edges), "a row of blocks is one group of C");
+#pragma unroll Cfg::RolledRows ? 1u : NG
                     for(uint32_t gi = 0; gi < NG; ++gi)
                     {
-                        const uint32_t bi = gi / GroupsPerRow, bj0 = (gi % GroupsPerRow) * GB;
+                        const uint32_t bi = gi / GroupsPerRow, bj0 = (gi % GroupsPerRow) * GB, at = Cfg::RolledRows ? 0u : bi;
                         // (the stores of D do not count, see copy_waits.hpp)
-                        const uint32_t inFlight = stagedCInFlight(gi, NG, CopiesC, Buffers); // (a constant: the loop is unrolled)
+                        const uint32_t inFlight = stagedCInFlight(gi, NG, CopiesC, Buffers); // (a constant where the loop is unrolled)
                         constexpr uint32_t Three = Buffers == 4u ? 3u * CopiesC : 0u, Two = Buffers == 4u ? 2u * CopiesC : 0u;
                         if(Buffers == 4u && inFlight == Three)
                             lds::waitCopiesAndReads<Three>();
@@ -1759,8 +1795,8 @@ namespace rocwmma_amd
                         else
                             lds::waitCopiesAndReads<0u>();
                         asm volatile("" ::: "memory");
-                        if(gi % GroupsPerRow == 0u)
-                            takeRow(bi);
+                        if(!Cfg::RolledRows && gi % GroupsPerRow == 0u)
+                            takeRow(bi, at);
                         typename Cfg::FragC io[GB];
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
@@ -1772,16 +1808,18 @@ namespace rocwmma_amd
                                 detail::copyBytes<16u>(io[bj].x + 4u * r,
                                                        myLds + (gi % Buffers) * GroupBytes + rdBase + ((g ^ (rdRow & 15u)) << 4));
                             }
+                        if constexpr(Cfg::RolledRows)
+                            takeRow(bi, at); // (behind the reads: its branches pass while they are under way)
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
 #pragma unroll
                             for(uint32_t e = 0; e < io[bj].num_elements; ++e)
-                                acc[bi][bj0 + bj].x[e] = alpha * acc[bi][bj0 + bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]);
-                        finish(bi, bj0, std::integral_constant<uint32_t, GB>{});
+                                acc[at][bj0 + bj].x[e] = alpha * acc[at][bj0 + bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]);
+                        finish(at, bj0, std::integral_constant<uint32_t, GB>{});
                         // (results replace the accumulators: every store has registers of its own)
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
-                            storeBlock(bi, bj0 + bj, acc[bi][bj0 + bj]);
+                            storeBlock(bi, bj0 + bj, acc[at][bj0 + bj]);
                         __builtin_amdgcn_sched_barrier(0);
                         // behind the stores: the next wait then leaves these copies in flight and not the stores
                         if(gi + Buffers < NG)
@@ -1826,36 +1864,45 @@ namespace rocwmma_amd
                     // tiles, 4096^3 f16, 110.6, 102.8, 101.6.
                     constexpr uint32_t Pieces = PairIO ? Cfg::BlocksN / 2u : Cfg::BlocksN; // of a row of blocks
                     typedef uint32_t   Words __attribute__((ext_vector_type(PairIO ? 4u : sizeof(OutT))));
-                    Words              raw[Cfg::BlocksM][Pieces];
-#pragma unroll
-                    for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
-                    {
+                    // (with the fused epilogue at most 64 registers of it, the rows behind them as soon as theirs are free: all of them spill)
+                    constexpr uint32_t PerRow = Pieces * sizeof(Words) / 4u, Ahead = Cfg::Fused && PerRow > 8u ? Cfg::BlocksM / 2u : Cfg::BlocksM;
+                    Words              raw[Ahead][Pieces];
+                    auto               loadRow = [&](uint32_t bi) {
                         const uint32_t row = wRow + blockRow(bi) + accRow;
                         const OutT*    src = c + static_cast<size_t>(Cfg::Edges && row >= m ? m - 1u : row) * ldc;
 #pragma unroll
                         for(uint32_t p = 0; p < Pieces; ++p)
                         {
                             const uint32_t col = wCol + (PairIO ? 2u * p * Cfg::Block + pairCol : p * Cfg::Block + 4u * accGroup);
-                            raw[bi][p]         = *reinterpret_cast<const Words*>(src + (Cfg::Edges && col >= n ? 0u : col));
+                            raw[bi % Ahead][p] = *reinterpret_cast<const Words*>(src + (Cfg::Edges && col >= n ? 0u : col));
                         }
-                    }
+                    };
+#pragma unroll
+                    for(uint32_t bi = 0; bi < Ahead; ++bi)
+                        loadRow(bi);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                     {
-                        takeRow(bi);
+                        takeRow(bi, bi);
+                        Words row[Pieces];
+#pragma unroll
+                        for(uint32_t p = 0; p < Pieces; ++p)
+                            row[p] = raw[bi % Ahead][p];
+                        if(bi + Ahead < Cfg::BlocksM)
+                            loadRow(bi + Ahead);
                         typename Cfg::FragC io[Cfg::BlocksN];
 #pragma unroll
                         for(uint32_t p = 0; p < Pieces; ++p)
                         {
                             if constexpr(PairIO)
                             {
-                                __builtin_memcpy(io[2u * p].x, &raw[bi][p], 8);
-                                __builtin_memcpy(io[2u * p + 1u].x, reinterpret_cast<const char*>(&raw[bi][p]) + 8, 8);
+                                __builtin_memcpy(io[2u * p].x, &row[p], 8);
+                                __builtin_memcpy(io[2u * p + 1u].x, reinterpret_cast<const char*>(&row[p]) + 8, 8);
                                 swapPair(io[2u * p], io[2u * p + 1u]);
                             }
                             else
-                                __builtin_memcpy(io[p].x, &raw[bi][p], sizeof(Words));
+                                __builtin_memcpy(io[p].x, &row[p], sizeof(Words));
                         }
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
@@ -1933,10 +1980,11 @@ namespace rocwmma_amd
             }
             else
             {
-#pragma unroll
+#pragma unroll Cfg::RolledRows ? 1u : Cfg::BlocksM
                 for(uint32_t bi = 0; bi < Cfg::BlocksM; ++bi)
                 {
-                    takeRow(bi);
+                    const uint32_t at = Cfg::RolledRows ? 0u : bi;
+                    takeRow(bi, at);
                     if constexpr(std::is_same<OutT, CompT>::value)
                     {
                         // results replace the accumulators, so no two stores share data registers
@@ -1947,13 +1995,13 @@ namespace rocwmma_amd
 #pragma unroll
                             for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
-                                for(uint32_t e = 0; e < acc[bi][bj].num_elements; ++e)
-                                    acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e];
-                            finish(bi, 0u, wholeRow);
+                                for(uint32_t e = 0; e < acc[at][bj].num_elements; ++e)
+                                    acc[at][bj].x[e] = alpha * acc[at][bj].x[e];
+                            finish(at, 0u, wholeRow);
                         }
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
-                            storeBlock(bi, bj, acc[bi][bj]);
+                            storeBlock(bi, bj, acc[at][bj]);
                     }
                     else
                     {
@@ -1962,13 +2010,13 @@ namespace rocwmma_amd
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
                             for(uint32_t e = 0; e < fd[bj].num_elements; ++e)
-                                acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e];
-                        finish(bi, 0u, wholeRow);
+                                acc[at][bj].x[e] = alpha * acc[at][bj].x[e];
+                        finish(at, 0u, wholeRow);
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
                             for(uint32_t e = 0; e < fd[bj].num_elements; ++e)
-                                fd[bj].x[e] = narrowed<OutT>(acc[bi][bj].x[e]);
+                                fd[bj].x[e] = narrowed<OutT>(acc[at][bj].x[e]);
                         if constexpr(PairIO)
                         {
 #pragma unroll
