@@ -1694,8 +1694,11 @@ namespace rocwmma_amd
                     return loadBias(bj);
             };
             // What the results of `Count` blocks of a row from block `first` on pass through: at once, but for 32-wide blocks (16 values
-            // per block and lane), which spilled.
-            auto finish = [&](uint32_t bi, uint32_t first, auto countC) {
+            // per block and lane), which spilled.  Those keep a branch on the activation per value where there is a C: e4m3 with bias,
+            // a branch per value and one per block, us: 1280 x 4608 x 256 A col / B row 15.0, 17.3; 912 x 6432 x 256 14.6, 16.4; with GELU 16.8, 15.3;
+            // 1024 x 7040 x 768 both row-major 21.1, 22.0, with GELU 21.6, 24.2.  Without C one branch is the faster one: 11.9, 11.5; 12.1, 11.4;
+            // 16.7, 15.7.
+            auto finish = [&](uint32_t bi, uint32_t first, auto countC, auto withC) {
                 if constexpr(Cfg::Fused)
                 {
                     constexpr uint32_t Count = decltype(countC)::value, Per = Cfg::FragAcc::num_elements;
@@ -1712,7 +1715,18 @@ namespace rocwmma_amd
                             for(uint32_t e = 0; e < Per; ++e)
                                 v[j * Per + e] = acc[bi][first + from + j].x[e] + bv.v[e];
                         }
-                        applyActivation(v, ex.fused.activation);
+                        if constexpr(Cfg::Block == 32u && decltype(withC)::value)
+                        {
+#pragma unroll
+                            for(uint32_t i = 0; i < Group * Per; ++i)
+                            {
+                                float one[1] = {v[i]};
+                                applyActivation(one, ex.fused.activation);
+                                v[i] = one[0];
+                            }
+                        }
+                        else
+                            applyActivation(v, ex.fused.activation);
 #pragma unroll
                         for(uint32_t j = 0; j < Group; ++j)
 #pragma unroll
@@ -1720,8 +1734,10 @@ namespace rocwmma_amd
                                 acc[bi][first + from + j].x[e] = v[j * Per + e];
                     }
                 }
-                (void)bi, (void)first, (void)countC;
+                (void)bi, (void)first, (void)countC, (void)withC;
             };
+            constexpr std::true_type  withC{};
+            constexpr std::false_type withoutC{};
             constexpr std::integral_constant<uint32_t, Cfg::BlocksN> wholeRow{};
             if(beta != static_cast<CompT>(0))
             {
@@ -1815,7 +1831,7 @@ namespace rocwmma_amd
 #pragma unroll
                             for(uint32_t e = 0; e < io[bj].num_elements; ++e)
                                 acc[at][bj0 + bj].x[e] = alpha * acc[at][bj0 + bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]);
-                        finish(at, bj0, std::integral_constant<uint32_t, GB>{});
+                        finish(at, bj0, std::integral_constant<uint32_t, GB>{}, withC);
                         // (results replace the accumulators: every store has registers of its own)
 #pragma unroll
                         for(uint32_t bj = 0; bj < GB; ++bj)
@@ -1840,7 +1856,7 @@ namespace rocwmma_amd
 #pragma unroll
                             for(uint32_t e = 0; e < early[bi][bj].num_elements; ++e)
                                 acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(early[bi][bj].x[e]);
-                        finish(bi, 0u, wholeRow);
+                        finish(bi, 0u, wholeRow, withC);
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
                         {
@@ -1909,7 +1925,7 @@ namespace rocwmma_amd
 #pragma unroll
                             for(uint32_t e = 0; e < Cfg::FragC::num_elements; ++e)
                                 acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(io[bj].x[e]);
-                        finish(bi, 0u, wholeRow);
+                        finish(bi, 0u, wholeRow, withC);
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
@@ -1954,7 +1970,7 @@ namespace rocwmma_amd
 #pragma unroll
                         for(uint32_t e = 0; e < Cfg::FragC::num_elements; ++e)
                             acc[bi][bj].x[e] = alpha * acc[bi][bj].x[e] + beta * static_cast<CompT>(fc[bi % 2u][bj].x[e]);
-                    finish(bi, 0u, wholeRow);
+                    finish(bi, 0u, wholeRow, withC);
 #pragma unroll
                     for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
@@ -1997,7 +2013,7 @@ namespace rocwmma_amd
 #pragma unroll
                                 for(uint32_t e = 0; e < acc[at][bj].num_elements; ++e)
                                     acc[at][bj].x[e] = alpha * acc[at][bj].x[e];
-                            finish(at, 0u, wholeRow);
+                            finish(at, 0u, wholeRow, withoutC);
                         }
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
@@ -2011,7 +2027,7 @@ namespace rocwmma_amd
 #pragma unroll
                             for(uint32_t e = 0; e < fd[bj].num_elements; ++e)
                                 acc[at][bj].x[e] = alpha * acc[at][bj].x[e];
-                        finish(at, 0u, wholeRow);
+                        finish(at, 0u, wholeRow, withoutC);
 #pragma unroll
                         for(uint32_t bj = 0; bj < Cfg::BlocksN; ++bj)
 #pragma unroll
