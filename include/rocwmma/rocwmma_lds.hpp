@@ -65,6 +65,20 @@ namespace rocwmma
             return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, bytes, 0x00020000);
         }
 
+        // The same with a descriptor that is in scalar registers for certain.  (The scalar ALU compares no 64-bit numbers by size, and a compiler that
+        // then leaves the descriptor in vector registers makes every copy a loop over the lanes' descriptors.)
+        ROCWMMA_DEVICE ROCWMMA_INLINE BufferRsrc makeScalarSource(const void* base, const void* end)
+        {
+            const ptrdiff_t left  = static_cast<const char*>(end) - static_cast<const char*>(base);
+            const int       bytes = left <= 0 ? 0 : (left > 0x7FFFFFFF ? 0x7FFFFFFF : static_cast<int>(left));
+            const uintptr_t at    = reinterpret_cast<uintptr_t>(base);
+            // (the builtin returns a signed int: halves of 32 bits without a sign before they are put together)
+            const uint32_t low  = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at)));
+            const uint32_t high = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at >> 32)));
+            return __builtin_amdgcn_make_buffer_rsrc(
+                reinterpret_cast<void*>(static_cast<uintptr_t>(high) << 32 | low), 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+        }
+
         ROCWMMA_DEVICE ROCWMMA_INLINE void asyncCopy16(void* ldsBase, BufferRsrc src, uint32_t laneOffset, uint32_t waveOffset)
         {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(

@@ -173,6 +173,11 @@ namespace rocwmma_amd
             // waves, 127.2 against 126.7 us; with four 122.1 against 128.1), two else
             static constexpr uint32_t BuffersC = WideWave && 4u * Block * GroupBlocks * Block * sizeof(OutT) * Waves <= LdsBytes ? 4u : 2u;
 
+            // Partly filled 256 x 256 tiles of fp8, both operands row-major, with the fused epilogue: the compiler left the descriptors of the
+            // copies in vector registers, and every copy was a loop over the lanes' descriptors (3456 x 2944 x 2816 with GELU 54.9 us, 48.5 with
+            // scalar ones).
+            static constexpr bool ScalarSources = Edges_ && Fused_ && BlockEdge_ == 32u && AKMajor && !BKMajor && MacroN == 256u;
+
             // Fused epilogue of 256 x 256 tiles on wide waves, and of their half tiles: a loop over the rows of blocks that is not unrolled (with
             // a C of 16 bits it is).  256 results per lane through bias and GELU one after the other are 37 KB of code, and what a first call, or
             // one behind other kernels, waits for is that code, with one wave per SIMD and nobody to cover it.  f16, GELU, K = 512 to 4096, operands
@@ -640,7 +645,7 @@ namespace rocwmma_amd
             // stage instead of running past the end of the operand; edge tiles read nothing there)
             auto issueA = [&](uint32_t slot, bool advance = true) {
                 char*                 ldsA = ldsRaw + slot * Cfg::StrideA;
-                const lds::BufferRsrc src  = Cfg::Edges ? lds::makeSource(aSrc, aEnd) : lds::makeSource(aSrc);
+                const lds::BufferRsrc src  = Cfg::ScalarSources ? lds::makeScalarSource(aSrc, aEnd) : Cfg::Edges ? lds::makeSource(aSrc, aEnd) : lds::makeSource(aSrc);
                 if constexpr(CopyWaves < Cfg::Waves)
                 {
                     if(wave < CopyWaves)
@@ -675,7 +680,7 @@ namespace rocwmma_amd
             };
             auto issueB = [&](uint32_t slot, bool advance = true) {
                 char*                 ldsB = ldsRaw + Cfg::FirstB + slot * Cfg::StrideB;
-                const lds::BufferRsrc src  = Cfg::Edges ? lds::makeSource(bSrc, bEnd) : lds::makeSource(bSrc);
+                const lds::BufferRsrc src  = Cfg::ScalarSources ? lds::makeScalarSource(bSrc, bEnd) : Cfg::Edges ? lds::makeSource(bSrc, bEnd) : lds::makeSource(bSrc);
                 if constexpr(CopyWaves < Cfg::Waves)
                 {
                     if(wave < CopyWaves)

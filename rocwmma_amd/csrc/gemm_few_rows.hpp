@@ -78,7 +78,8 @@ namespace rocwmma_amd
             char* const           ring = ldsRaw + wave * (Ring * Tile::StepBytes);
             auto                  issue = [&](uint32_t slot, uint32_t step) {
                 char* const    to = ring + slot * Tile::StepBytes;
-                const uint32_t at = step * kFewStep;
+                // (readfirstlane: the 64 x 32 tile had the copies' offsets in vector registers, and every copy was a loop over the lanes')
+                const uint32_t at = __builtin_amdgcn_readfirstlane(step * kFewStep);
                 uint32_t       a[2], b[2];
 #pragma unroll
                 for(uint32_t half = 0; half < 2u; ++half)
