@@ -57,7 +57,8 @@ def test_bias_and_activation_on_edge_tiles(dtype_in, dtype_out, tol, la, lb, act
 @pytest.mark.parametrize("la,lb", [(RM, CM), (CM, RM)])
 @pytest.mark.parametrize("dtype_in,dtype_out,tol", TRIPLES)
 def test_bias_and_activation_on_the_large_tile(dtype_in, dtype_out, tol, la, lb, act):
-    """2048 x 4352 x 256: whole tiles of every size, 136 of 256 x 256 on 256 compute units."""
+    """2048 x 4352 x 256: 136 tiles of 256 x 256 on 256 compute units, i.e. the large tile with the
+    last (only) round cut into half tiles on a 256-unit device."""
     m, n, k = 2048, 4352, 256
     a, b, c, bias = case(200, dtype_in, dtype_out, m, n, k)
     rows = np.arange(0, m, 37, dtype=np.uint32)

@@ -6,12 +6,8 @@ import oracle as orc
 import rocwmma_amd as rw
 from test_gpu_gemm_rungs import PAIRS, framed, guarded
 from util import CM, RM
-from wide_waves import RING_STARTS
 
 pytestmark = pytest.mark.gpu
-
-RESULTS = {(0, 4): [(orc.F16, orc.F32), (orc.BF16, orc.F32)], (0, 2): [(orc.F16, orc.F16), (orc.BF16, orc.BF16)], (1, 4): [(orc.I8, orc.I32)],
-           (1, 1): [(orc.I8, orc.I8)]}
 
 
 @pytest.mark.parametrize("stages", [1, 2, 3, 4, 5, 6, 13])
@@ -32,21 +28,20 @@ def test_every_stage_count(dtype_in, dtype_out, stages):
             assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)), (la, lb, beta)
 
 
-@pytest.mark.parametrize("kind,pair,rung,m,n,k_bytes,out", RING_STARTS)
-def test_256_x_128_tiles_over_their_first_stages(kind, pair, rung, m, n, k_bytes, out):
-    """256 x 128 tiles, whole and partly filled, where their ring (three stages of A, four of B) begins and wraps
-    (tests/test_host_gemm_wide_waves.py says that these problems run on them)."""
+@pytest.mark.parametrize("m,n", [(1536, 3584), (528, 7184), (1040, 6000)])
+@pytest.mark.parametrize("k_bytes", [256, 384, 512, 640, 768, 1312, 2080])
+def test_halves_over_their_first_stages(k_bytes, m, n):
+    """256 x 128 tiles, whole and partly filled, where their ring (three stages of A, four of B) begins and wraps."""
     import torch
 
     gen = torch.Generator(device="cuda").manual_seed(k_bytes)
-    la, lb = PAIRS[pair]
-    for dtype_in, dtype_out in RESULTS[kind, out]:
+    for dtype_in, dtype_out in [(orc.F16, orc.F16), (orc.BF16, orc.F32), (orc.I8, orc.I32)]:
         k = k_bytes // (1 if dtype_in == orc.I8 else 2)
-        a, lda = framed(gen, dtype_in, m, k, -2, 2)
-        b, ldb = framed(gen, dtype_in, *((n, k) if lb == CM else (k, n)), -2, 2)
-        c, ldc = framed(gen, dtype_out, m, n, -4, 4)
-        for alpha, beta in [(1.0, 0.0), (1.0, 1.0)]:
+        for lb in (CM, RM):
+            a, lda = framed(gen, dtype_in, m, k, -2, 2)
+            b, ldb = framed(gen, dtype_in, *((n, k) if lb == CM else (k, n)), -2, 2)
+            c, ldc = framed(gen, dtype_out, m, n, -4, 4)
             got, want = guarded(dtype_out, m, n), guarded(dtype_out, m, n)
-            for d, algo in ((got, rw.GEMM_AUTO), (want, rw.GEMM_WAVE_TILE)):
-                rw.gemm(dtype_in, dtype_out, la, lb, RM, m, n, k, a, b, c, d[1024:], alpha, beta, lda=lda, ldb=ldb, ldc=ldc, algo=algo)
-            assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)), (dtype_in, dtype_out, beta)
+            for out, algo in ((got, rw.GEMM_AUTO), (want, rw.GEMM_WAVE_TILE)):
+                rw.gemm(dtype_in, dtype_out, RM, lb, RM, m, n, k, a, b, c, out[1024:], 1.0, 1.0, lda=lda, ldb=ldb, ldc=ldc, algo=algo)
+            assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)), (dtype_in, lb)

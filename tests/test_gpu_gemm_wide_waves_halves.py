@@ -5,7 +5,7 @@ import pytest
 import oracle as orc
 import rocwmma_amd as rw
 from test_gpu_gemm_rungs import PAIRS, framed, guarded, torch_type
-from test_gpu_gemm_wide_waves import RESULTS
+from test_gpu_gemm_wide_waves_ring import RESULTS
 from util import CM, RM
 from wide_waves import HALF_TILES
 

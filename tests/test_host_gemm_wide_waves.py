@@ -2,14 +2,14 @@
 import pytest
 
 import wide_waves
-from test_host_gemm_rungs import rung_of  # noqa: F401  (the fixture)
+from test_host_gemm_small_tiles import route_of  # noqa: F401  (the fixture)
 
 
 @pytest.mark.parametrize("name", [name for name in dir(wide_waves) if name.isupper()])
-def test_cases_run_on_the_rungs_they_name(rung_of, name):  # noqa: F811
+def test_cases_run_on_the_rungs_they_name(route_of, name):  # noqa: F811
     cases = getattr(wide_waves, name)
     asked = "".join("%d %d %d %d %d %d\n" % (kind, pair, m, n, k_bytes, out) for kind, pair, _, m, n, k_bytes, out in cases)
-    wrong = [(case, rung) for case, rung in zip(cases, rung_of(text=asked)) if case[2] != rung]
+    wrong = [(case, rung) for case, rung in zip(cases, route_of(asked)) if case[2] != rung]
     assert not wrong, wrong
 
 
