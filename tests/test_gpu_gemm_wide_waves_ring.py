@@ -5,7 +5,7 @@ import pytest
 import oracle as orc
 import rocwmma_amd as rw
 from test_gpu_gemm_rungs import PAIRS, framed, guarded
-from util import RM
+from util import CM, RM
 from wide_waves import RING_STARTS
 
 pytestmark = pytest.mark.gpu
